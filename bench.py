@@ -142,13 +142,14 @@ def main():
             g = grids[native.grid_index[m.stmt.grid]]
             per_iter += g.class_info(m.stmt.klass)["count"] * 8 * (len([r for r in m.refs if r[1] >= 0]) + 1)
         trip = 50                                   # the pressure loop's iterations per call
-        launches_per_trip = -(-trip // L.tmax)
+        launches_per_trip = round(trip * loop["launches"] / loop["iterations"])
         avg_ms = native.time_loop(0, trip, reps=20)
         bytes_per_launch = per_iter * trip / launches_per_trip
+        tile = "wave tiles" if L.waves else f"{L.core[0]}x{L.core[1]} tiles, halo {L.halo}"
         kernel_name = (f"{L.kernel} (pressure loop blocked: {trip} iterations of Jacobi sweep + 4 boundary "
-                       f"statements in {launches_per_trip} launches of <= {L.tmax}, {L.core[0]}x{L.core[1]} "
-                       f"tiles, halo {L.halo})")
-        kernel_id = f"{L.kernel}:{L.core[0]}x{L.core[1]}:h{L.halo}:t{L.tmax}:w{L.threads}:n{n}"
+                       f"statements in {launches_per_trip} launches, {tile})")
+        kernel_id = (f"{L.kernel}:wave:l{launches_per_trip}:n{n}" if L.waves else
+                     f"{L.kernel}:{L.core[0]}x{L.core[1]}:h{L.halo}:t{L.tmax}:w{L.threads}:n{n}")
 
     name = ctypes_name(lib)
     out = {

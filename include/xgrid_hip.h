@@ -80,6 +80,16 @@ typedef struct xg_group_desc {
  * a halo of `halo` cells kept in LDS (reference: the same statements as
  * separate nests, xgrid/lang/generator.py:369-374 around :289-361). */
 #define XG_LOOP_MAX_STMTS 8
+/* A wave tile of a blocked loop: a workgroup of up to `threads` work-items, each
+ * wave holding `rows` rows of the region in registers. */
+#define XG_LOOP_MAX_WAVE 2
+typedef struct xg_wave_tile {
+  void* fn;
+  void* fn_b;                                /* batched variant */
+  int32_t rows, threads;
+  int32_t lds;                               /* LDS bytes per wave */
+  int32_t waves_per_simd;                    /* waves its registers leave room for */
+} xg_wave_tile;
 typedef struct xg_loop_desc {
   int32_t nstmts;
   int32_t sids[XG_LOOP_MAX_STMTS];
@@ -93,8 +103,14 @@ typedef struct xg_loop_desc {
   int32_t alt;                               /* plain calls on a grid of at most alt_max_cells cells run
                                                 loop plan `alt` (another tile shape of the same loop)
                                                 instead; -1: none */
-  int32_t alt_pad;
+  int32_t nwave;                             /* wave tiles of this loop: when there are any, they run it
+                                                and fn .. fn_check_b are null */
   int64_t alt_max_cells;
+  xg_wave_tile wave[XG_LOOP_MAX_WAVE];
+  void* fn_wcheck;                           /* proves a wave-tile geometry exact on the grid's mask */
+  void* fn_wcheck_b;
+  int32_t wave_cols;                         /* columns of a wave tile's region */
+  int32_t wave_elem;                         /* element bytes of the loop's grid */
 } xg_loop_desc;
 
 /* Function table handed to generated host stubs (the stub runs the kernel's

@@ -47,11 +47,18 @@ class GroupDesc(Structure):
 XG_LOOP_MAX = 8
 
 
+class WaveTile(Structure):
+    _fields_ = [("fn", c_void_p), ("fn_b", c_void_p), ("rows", c_int32), ("threads", c_int32),
+                ("lds", c_int32), ("waves_per_simd", c_int32)]
+
+
 class LoopDesc(Structure):
     _fields_ = [("nstmts", c_int32), ("sids", c_int32 * XG_LOOP_MAX), ("grid_arg", c_int32),
                 ("core0", c_int32), ("core1", c_int32), ("halo", c_int32), ("tmax", c_int32),
                 ("threads", c_int32), ("fn", c_void_p), ("fn_check", c_void_p), ("fn_b", c_void_p),
-                ("fn_check_b", c_void_p), ("alt", c_int32), ("alt_pad", c_int32), ("alt_max_cells", c_int64)]
+                ("fn_check_b", c_void_p), ("alt", c_int32), ("nwave", c_int32), ("alt_max_cells", c_int64),
+                ("wave", WaveTile * 2), ("fn_wcheck", c_void_p), ("fn_wcheck_b", c_void_p),
+                ("wave_cols", c_int32), ("wave_elem", c_int32)]
 
 
 class Api(Structure):

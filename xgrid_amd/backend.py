@@ -20,7 +20,7 @@ from .compilers import compile_device, compile_host, load_host
 from .config import get_config
 from .emit import Emitter, Lowered
 from .grid import Grid
-from .types import Boolean, Floating, GridType, Integer, Pointer, Structure, Void
+from .types import Boolean, Floating, GridType, Integer, Pointer, Structure, Void, element_nbytes
 
 _MODE = {"inplace": _lib.MODE_INPLACE, "pingpong": _lib.MODE_PINGPONG, "twophase": _lib.MODE_TWOPHASE}
 
@@ -154,8 +154,18 @@ class HipKernel:
             ld.halo = L.halo
             ld.tmax = L.tmax
             ld.threads = L.threads
-            ld.fn = fn(L.kernel)
-            ld.fn_check = fn(L.kernel + "_chk")
+            if L.waves:
+                ld.nwave = len(L.waves)
+                ld.wave_cols = L.waves[0].cols
+                ld.wave_elem = element_nbytes(L.stmts[0].stmt.gtype.element)
+                for t, w in enumerate(L.waves):
+                    ld.wave[t].fn = fn(w.kernel)
+                    ld.wave[t].rows, ld.wave[t].threads = w.rows, w.threads
+                    ld.wave[t].lds, ld.wave[t].waves_per_simd = w.lds, w.waves_per_simd
+                ld.fn_wcheck = fn(L.wave_check)
+            else:
+                ld.fn = fn(L.kernel)
+                ld.fn_check = fn(L.kernel + "_chk")
             ld.alt = -1
             if i < len(low.loops) and L.alt is not None:
                 ld.alt = len(low.loops) + nalt
@@ -215,6 +225,11 @@ class HipKernel:
         for i, g in enumerate(low.groups):
             self._groups[i].fn_b = fn(g.kernel + "_b")
         for i, L in enumerate(list(low.loops) + [L.alt for L in low.loops if L.alt is not None]):
+            if L.waves:
+                for t, w in enumerate(L.waves):
+                    self._loops[i].wave[t].fn_b = fn(w.kernel + "_b")
+                self._loops[i].fn_wcheck_b = fn(L.wave_check + "b")
+                continue
             self._loops[i].fn_b = fn(L.kernel + "_b") if L.batched else None
             self._loops[i].fn_check_b = fn(L.kernel + "_chkb") if L.batched else None
 

@@ -68,15 +68,27 @@ typedef struct xg_launch_hdr {
 /* Temporally blocked loop: several iterations of a loop body of stencil
  * statements on one grid, per workgroup tile, in LDS. */
 #define XG_TB_MAX_STMTS 8
+/* Wave tiles: the most iterations a launch of several tiles runs, and the widest halo of its
+ * regions; the region of a workgroup that checks a mask. */
+#define XG_WAVE_MAX_ITERS 16
+#define XG_WAVE_MAX_HALO 24
+#define XG_WAVE_CHECK_ROWS 96
+#define XG_WAVE_CHECK_COLS 128
 typedef struct xg_tb_hdr {
   xg_gview src;                    /* the grid's level 0 before the launch */
   xg_gview dst;                    /* receives every cell after `iters` iterations */
   const int32_t* mask;             /* boundary mask (null: every cell is class 0) */
-  int32_t* fail;                   /* validation launch: set when a core cell is not exact */
+  int32_t* fail;                   /* validation launch: set when a core cell is not exact (wave tiles:
+                                      per iteration, how far away a cell's value comes from) */
   int32_t klass[XG_TB_MAX_STMTS];  /* class of each statement */
   int32_t iters;                   /* iterations in this launch (<= the compiled maximum) */
   int32_t uniform;                 /* every loaded view has the grid's shape */
-} xg_tb_hdr;                       /* 24 + 24 + 8 + 8 + 32 + 8 = 104 bytes */
+  /* Wave tiles (see wave_axis in xgrid_device.h): tiles along each axis (in a check its own),
+   * halo, and the box that class 0 fills exactly (empty: none), whose cells need no mask. */
+  int32_t nt0, nt1, halo;
+  int32_t blo[2], bhi[2];
+  int32_t pad;
+} xg_tb_hdr;                       /* 24 + 24 + 8 + 8 + 32 + 8 + 16 + 16 = 136 bytes */
 
 /* Batched launches: one launch runs one statement (or blocked loop, or chain
  * of boundary statements) for many independent instances of one kernel.  A
@@ -96,6 +108,6 @@ typedef struct xg_btent {
   const void* params[XG_TB_MAX_STMTS];
   int64_t tile0;
   int64_t ntiles;
-} xg_btent;                              /* 104 + 64 + 64 + 16 = 248 bytes */
+} xg_btent;                              /* 136 + 64 + 64 + 16 = 280 bytes */
 
 #endif

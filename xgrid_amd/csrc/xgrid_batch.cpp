@@ -47,6 +47,7 @@ struct PendingLaunch {
   size_t table_off;    // first entry
   int32_t n;           // entries (kTiles) / statements per instance (kGroup)
   int64_t total;       // tiles (kTiles) / instances (kGroup)
+  unsigned lds = 0;    // dynamic LDS bytes of a workgroup
 };
 
 struct BatchGraph {
@@ -126,7 +127,7 @@ int issue(xg_batch* b, void* dev) {
     if (L.kind == kTiles) {
       void* args[3] = {&E, &n, &total};
       e = hipModuleLaunchKernel((hipFunction_t)L.fn, (unsigned)launch_blocks(b, total), 1, 1, (unsigned)L.threads, 1,
-                                1, 0, g_dev.stream, args, nullptr);
+                                1, L.lds, g_dev.stream, args, nullptr);
     } else {
       void* args[2] = {&E, &n};
       e = hipModuleLaunchKernel((hipFunction_t)L.fn, (unsigned)total, 1, 1, (unsigned)L.threads, 1, 1, 0,
@@ -373,13 +374,16 @@ int run_positions(xg_batch* b, const std::vector<Pos>& pos, const std::vector<in
 int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx,
              const std::vector<std::vector<const void*>>& par) {
   std::vector<int> blocked, check, plain;            // positions in idx
+  const xg_loop_desc& ld = b->inst[(size_t)idx[0]].k->loops[(size_t)lid].d;
   for (size_t t = 0; t < idx.size(); ++t) {
     xg_kernel* k = b->inst[(size_t)idx[t]].k;
     LoopPlan& L = k->loops[(size_t)lid];
-    const bool can = k->blocked && trip > 0 && L.d.fn_b && L.d.fn_check_b && loop_blockable(k, L) && L.state >= 0;
+    const bool built = L.d.nwave ? L.d.wave[0].fn_b && L.d.fn_wcheck_b : L.d.fn_b && L.d.fn_check_b;
+    const bool can = k->blocked && trip > 0 && built && loop_blockable(k, L) && L.state >= 0;
     // a launch of more iterations than the plan's checks ran needs a check of its own
+    // (wave tiles: one check per mask says what every number of iterations needs)
+    const bool unproven = can && (L.state == 0 || (!L.d.nwave && std::min<int64_t>(L.d.tmax, trip) > L.validated));
     // (a check needs a synchronisation, so none is captured)
-    const bool unproven = can && (L.state == 0 || std::min<int64_t>(L.d.tmax, trip) > L.validated);
     if (!can || (unproven && b->mode == kCapture))
       plain.push_back((int)t);
     else if (unproven)
@@ -388,6 +392,7 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
       blocked.push_back((int)t);
   }
   std::vector<int64_t> remaining(idx.size(), trip);
+  auto longest = [](const LoopPlan& L) -> int64_t { return L.d.nwave ? L.cut.iters : L.d.tmax; };
   auto tb_launch = [&](const std::vector<int>& set, bool chk) -> int {
     if (set.empty()) return XG_OK;
     xg_kernel* k0 = b->inst[(size_t)idx[(size_t)set[0]]].k;
@@ -399,12 +404,16 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
       xg_kernel* k = b->inst[(size_t)idx[(size_t)t]].k;
       LoopPlan& L = k->loops[(size_t)lid];
       xg_grid* G = k->grids[(size_t)L.d.grid_arg];
-      const int T = (int)std::min<int64_t>(L.d.tmax, remaining[(size_t)t]);
       xg_btent e;
       std::memset(&e, 0, sizeof e);
-      fill_tb_hdr(k, L, e.th, T, k->d_fail);
       e.tile0 = total;
-      e.ntiles = ceil_div(G->shape[0], L.d.core0) * ceil_div(G->shape[1], L.d.core1);
+      if (L.d.nwave && chk) {
+        fill_wave_check(k, L, e.th, k->d_fail);
+        e.ntiles = (int64_t)e.th.nt0 * e.th.nt1;
+      } else {
+        fill_tb_hdr(k, L, e.th, (int)std::min<int64_t>(longest(L), remaining[(size_t)t]), k->d_fail);
+        e.ntiles = L.d.nwave ? L.cut.blocks() : ceil_div(G->shape[0], L.d.core0) * ceil_div(G->shape[1], L.d.core1);
+      }
       total += e.ntiles;
       std::vector<size_t> ro, po;
       for (int j = 0; j < L.d.nstmts; ++j) {
@@ -417,7 +426,7 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
       ents.push_back(e);
       roff.push_back(ro);
       poff.push_back(po);
-      L.launches++;
+      if (!(L.d.nwave && chk)) L.launches++;
     }
     if (total > 0x7fffffff) return fail(XG_ERR_ARG, "batched launch has too many tiles");
     const size_t base = put(b, ents.data(), ents.size() * sizeof(xg_btent));
@@ -426,8 +435,15 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
         set_rel(b, base + i * sizeof(xg_btent) + offsetof(xg_btent, refs) + j * sizeof(void*), roff[i][j]);
         set_rel(b, base + i * sizeof(xg_btent) + offsetof(xg_btent, params) + j * sizeof(void*), poff[i][j]);
       }
-    b->launches.push_back(PendingLaunch{chk ? L0.d.fn_check_b : L0.d.fn_b, kTiles, L0.d.threads, base,
-                                        (int32_t)ents.size(), total});
+    void* fn = chk ? L0.d.fn_check_b : L0.d.fn_b;
+    int threads = L0.d.threads;
+    unsigned lds = 0;
+    if (L0.d.nwave) {
+      fn = chk ? L0.d.fn_wcheck_b : L0.d.wave[L0.cut.tile].fn_b;
+      threads = chk ? kWaveCheckThreads : L0.cut.waves * 64;
+      lds = chk ? 0u : (unsigned)(L0.cut.waves * L0.d.wave[L0.cut.tile].lds);
+    }
+    b->launches.push_back(PendingLaunch{fn, kTiles, threads, base, (int32_t)ents.size(), total, lds});
     return XG_OK;
   };
   auto advance = [&](const std::vector<int>& set) {
@@ -435,30 +451,30 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
       xg_kernel* k = b->inst[(size_t)idx[(size_t)t]].k;
       LoopPlan& L = k->loops[(size_t)lid];
       xg_grid* G = k->grids[(size_t)L.d.grid_arg];
-      const int64_t T = std::min<int64_t>(L.d.tmax, remaining[(size_t)t]);
+      const int64_t T = std::min<int64_t>(longest(L), remaining[(size_t)t]);
       std::swap(G->levels[0], G->scratch);
       remaining[(size_t)t] -= T;
       L.iterations += T;
     }
   };
   if (!check.empty()) {
-    // prove the plan on each instance's mask: a checking launch, then read the flags
+    // prove the plan on each instance's mask: a checking launch, then read the answers
     for (int t : check) {
       xg_kernel* k = b->inst[(size_t)idx[(size_t)t]].k;
       if (!k->d_fail) {
         void* p = nullptr;
-        if (int rc = dev_alloc(sizeof(int32_t), true, &p)) return rc;
+        if (int rc = dev_alloc(kCheckBytes, true, &p)) return rc;
         k->d_fail = (int32_t*)p;
       }
-      XG_HIP(hipMemsetAsync(k->d_fail, 0, sizeof(int32_t), g_dev.stream));
+      XG_HIP(hipMemsetAsync(k->d_fail, 0, kCheckBytes, g_dev.stream));
     }
     int rc = tb_launch(check, true);
     if (!rc) rc = flush_direct(b);
     if (rc) return rc;
-    std::vector<int32_t> flags(check.size(), 0);
+    std::vector<std::array<int32_t, XG_WAVE_MAX_ITERS>> answers(check.size());
     for (size_t c = 0; c < check.size(); ++c) {
       xg_kernel* k = b->inst[(size_t)idx[(size_t)check[c]]].k;
-      XG_HIP(hipMemcpyAsync(&flags[c], k->d_fail, sizeof(int32_t), hipMemcpyDeviceToHost, g_dev.stream));
+      XG_HIP(hipMemcpyAsync(answers[c].data(), k->d_fail, kCheckBytes, hipMemcpyDeviceToHost, g_dev.stream));
     }
     XG_HIP(hipStreamSynchronize(g_dev.stream));
     b->n_validations++;
@@ -466,7 +482,10 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
     for (size_t c = 0; c < check.size(); ++c) {
       xg_kernel* k = b->inst[(size_t)idx[(size_t)check[c]]].k;
       LoopPlan& L = k->loops[(size_t)lid];
-      if (flags[c]) {
+      if (L.d.nwave) {
+        wave_answer(L, answers[c].data());
+        blocked.push_back(check[c]);
+      } else if (answers[c][0]) {
         L.state = -1;                 // its scratch is discarded; it runs the loop unblocked
         plain.push_back(check[c]);
       } else {
@@ -475,8 +494,31 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
         passed.push_back(check[c]);
       }
     }
-    advance(passed);
+    advance(passed);                  // the checking variant also ran these iterations
     blocked.insert(blocked.end(), passed.begin(), passed.end());
+  }
+  if (ld.nwave) {
+    // the instances of a launch share one tile, workgroup size and iteration count
+    std::vector<int> ok;
+    std::vector<WaveShape> shapes;
+    for (int t : blocked) {
+      xg_kernel* k = b->inst[(size_t)idx[(size_t)t]].k;
+      LoopPlan& L = k->loops[(size_t)lid];
+      if (wave_outrun(L, trip)) {
+        L.state = -1;
+        plain.push_back(t);
+        continue;
+      }
+      ok.push_back(t);
+      shapes.push_back(wave_shape(k->grids[(size_t)ld.grid_arg], L));
+    }
+    const WaveCut cut = ok.empty() ? WaveCut{} : wave_choose(ld, shapes, trip);
+    for (size_t i = 0; i < ok.size(); ++i) {
+      if (cut.waves) b->inst[(size_t)idx[(size_t)ok[i]]].k->loops[(size_t)lid].cut = wave_cut_for(ld, cut, shapes[i]);
+      else plain.push_back(ok[i]);
+    }
+    if (!cut.waves) ok.clear();
+    blocked.swap(ok);
   }
   for (;;) {
     std::vector<int> live;

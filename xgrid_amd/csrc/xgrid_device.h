@@ -65,6 +65,10 @@ __device__ __forceinline__ gptr<T> gp(const void* p) {
  * elements of 16 bytes together, only at addresses that are multiples of 16). */
 template <class T, int K>
 using vecn = T __attribute__((ext_vector_type(K)));
+/* The same at any multiple of the element's size (global memory takes 16-byte
+ * accesses at any multiple of 4 bytes; LDS does not). */
+template <class T, int K>
+using vecu = T __attribute__((ext_vector_type(K), aligned(sizeof(T))));
 /* The views and parameter blocks a batch table points to are written by the
  * host before the launch and only read by kernels: reading them through the
  * constant address space lets uniform reads be scalar loads into SGPRs, as
@@ -717,7 +721,8 @@ __device__ __forceinline__ T tb_ld(const T* lds, const uint8_t* vld, bool& ok, i
  * Lane c of a wave holds column c of a 64-column region; a read at column
  * offset o is the value lane c + o holds, moved across lanes with DPP
  * (wave_shl:1 moves lane c + 1 to lane c, wave_shr:1 lane c - 1 to lane c;
- * lanes whose source lies outside the wave get 0).  Every lane of the wave
+ * lanes whose source lies outside the wave get 0, by bound_ctrl, so no register
+ * is cleared first).  Every lane of the wave
  * must execute the move (it reads other lanes' registers). */
 template <int O>
 __device__ __forceinline__ uint32_t lane_shift_u32(uint32_t x) {
@@ -725,7 +730,7 @@ __device__ __forceinline__ uint32_t lane_shift_u32(uint32_t x) {
   int v = (int)x;
 #pragma unroll
   for (int k = 0; k < (O > 0 ? O : -O); ++k)
-    v = __builtin_amdgcn_update_dpp(0, v, O > 0 ? 0x130 : 0x138, 0xf, 0xf, false);
+    v = __builtin_amdgcn_mov_dpp(v, O > 0 ? 0x130 : 0x138, 0xf, 0xf, true);
   return (uint32_t)v;
 }
 
@@ -750,6 +755,37 @@ __device__ __forceinline__ T lane_shift(T x) {
   } else {
     return (T)lane_shift_u32<O>((uint32_t)x);
   }
+}
+
+/* ---- temporally blocked loops (2-D), wave tiles ---------------------------
+ * One axis of a wave tile's grid: `n` cells cut into `nt` regions of `r` cells
+ * that overlap by 2 h.  The first region starts at the grid's first cell and the
+ * last one ends at its last (no region cell lies outside a grid of at least r
+ * cells, and a region edge on the grid's edge needs no halo): region i starts at
+ * cell `start` and its workgroup writes cells [w0, w1), at least h cells from
+ * every region edge that is not an edge of the grid. */
+struct wave_axis {
+  int start, w0, w1;
+  __device__ __forceinline__ wave_axis(int i, int nt, int n, int r, int h) {
+    const int c = r - 2 * h;
+    start = nt > 1 ? min(i * c, n - r) : 0;
+    w0 = i > 0 ? i * c + h : 0;
+    w1 = i < nt - 1 ? (i + 1) * c + h : n;
+  }
+};
+
+/* Extents (cells to the left, right, above and below, a byte each) of a value that
+ * depends on what `v` says and on the cell (d0, d1) away, whose own extents are `x`;
+ * 255 stays 255. */
+__device__ __forceinline__ uint32_t wave_extent(uint32_t v, uint32_t x, int d0, int d1) {
+  const int d[4] = {-d1, d1, -d0, d0};
+  uint32_t r = 0u;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int e = (int)((x >> (8 * b)) & 255u), o = (int)((v >> (8 * b)) & 255u);
+    r |= (uint32_t)max(o, e == 255 ? 255 : min(max(e + d[b], 0), 254)) << (8 * b);
+  }
+  return r;
 }
 
 /* ---- batched launches ---------------------------------------------------

@@ -4,6 +4,7 @@
 #ifndef XGRID_KERNEL_H
 #define XGRID_KERNEL_H
 
+#include <array>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -15,7 +16,10 @@ namespace xgi {
 constexpr int kThreads = 256;
 constexpr int kGroupThreads = 1024;
 constexpr int64_t kFuseMaxCells = 4096;  // default of g_dev.fuse_max_cells (XGRID_FUSE_MAX_CELLS)
-constexpr int64_t kGraphMinLaunches = 4;    // a call with fewer launches runs them directly (cheaper)
+// A call with fewer launches runs them directly: replaying a graph of one kernel takes 21.8 us
+// of host time against 6.3.  A small cavity is three launches and over 60 us of device time,
+// which hides either.
+constexpr int64_t kGraphMinLaunches = 3;
 // Store grids larger than the 256 MB last-level cache (Infinity Cache) take non-temporal
 // stores in 3-D box tiles: no later launch can find their cells in cache anyway.  The
 // 512^3 heat update moves the same bytes with them and runs 5-6 % faster (the write
@@ -55,12 +59,29 @@ struct EventPair {
   hipEvent_t a, b;
 };
 
-struct LoopPlan {
-  xg_loop_desc d;
-  const void* grid = nullptr;   // the grid the plan was validated on
-  uint64_t mask_version = 0;    // ... and its mask
+// How the launches of a blocked loop on wave tiles cut a grid: which tile, waves per
+// workgroup, halo, tiles per axis, and the iterations of the longest launch.
+struct WaveCut {
+  int32_t tile = 0, waves = 0, halo = 0, nt0 = 1, nt1 = 1, iters = 0;
+  int64_t blocks() const { return (int64_t)nt0 * nt1; }
+};
+
+// What is known about a blocked loop on one mask.  A mask's version is drawn anew each time a
+// grid's mask is set or a grid is made, so it names one grid and one mask for good.
+struct LoopProof {
+  uint64_t mask_version = 0;
   int state = 0;                // 1 exact, 0 unknown, -1 declined
   int validated = 0;            // state 1: launches of at most this many iterations are proven exact
+  uint8_t reach[XG_WAVE_MAX_ITERS] = {};   // wave tiles, state 1: the halo that 1, 2, ... iterations need
+};
+// A program that alternates between grids keeps the proofs of this many masks per loop (a
+// check costs a launch and a synchronisation).
+constexpr size_t kLoopProofs = 32;
+
+struct LoopPlan : LoopProof {
+  xg_loop_desc d;
+  std::vector<LoopProof> others;   // other masks' proofs, most recent first
+  WaveCut cut;                     // wave tiles: the cut of the launches being made
   int64_t launches = 0, iterations = 0;
   std::vector<std::vector<uint8_t>> last_params;
 };
@@ -99,7 +120,7 @@ struct xg_kernel {
   std::vector<xgi::EventPair> events;
   std::vector<xgi::LoopPlan> loops;
   bool blocked = true;
-  int32_t* d_fail = nullptr;        // validation flag of blocked launches
+  int32_t* d_fail = nullptr;        // answer of checking launches (kCheckBytes)
   std::vector<int64_t> exec_count;  // stmt() calls per statement (all modes)
   std::vector<std::vector<uint8_t>> last_params;  // parameters of each statement's last call
   std::vector<uint8_t> key_buf;
@@ -129,6 +150,26 @@ int ensure_scratch(xg_kernel* k);
 // the grid's current mask known?  Resets the plan when the grid or mask changed.
 bool loop_blockable(xg_kernel* k, LoopPlan& L);
 void fill_tb_hdr(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int iters, int32_t* fail_flag);
+// A grid to be cut into wave tiles: its shape, and the halo that 1, 2, ... iterations need.
+struct WaveShape {
+  int32_t n0, n1;
+  const uint8_t* reach;
+};
+inline WaveShape wave_shape(const xg_grid* G, const LoopProof& p) { return {G->shape[0], G->shape[1], p.reach}; }
+// The tile, waves and iterations with which the launches for `trip` iterations run all `shapes`
+// (one batch).  waves = 0: no tile holds the loop.
+WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip);
+// ... with the halo and tile counts of one grid.
+WaveCut wave_cut_for(const xg_loop_desc& d, WaveCut c, const WaveShape& s);
+// Header of a mask's checking launch, and what its answer (XG_WAVE_MAX_ITERS numbers) says.
+void fill_wave_check(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int32_t* answer);
+void wave_answer(LoopPlan& L, const int32_t* answer);
+// Is the loop to be left to plain launches: a launch of trip iterations (at most tmax) would need
+// too wide a halo?
+bool wave_outrun(const LoopPlan& L, int64_t trip);
+constexpr size_t kCheckBytes = XG_WAVE_MAX_ITERS * sizeof(int32_t);   // answer of a checking launch
+constexpr int kWaveCheckThreads = 1024;
+constexpr int64_t kWaveSingleIters = 1024;   // most iterations of a launch when one tile holds a grid
 
 }  // namespace xgi
 

@@ -246,7 +246,7 @@ int64_t blocks_for_dom(int D, const xg_dom& dom, int cols3) {
 // 64 columns per lane-row of a 3-D tile times the columns each lane holds (1, 2 or 4)
 int tile3_cols(const xg_stmt_desc& d) { return d.tile3_cols == 128 || d.tile3_cols == 256 ? d.tile3_cols : 64; }
 
-int do_launch(xg_kernel* k, int32_t sid, void* fn, int64_t blocks, int threads, void** args) {
+int do_launch(xg_kernel* k, int32_t sid, void* fn, int64_t blocks, int threads, void** args, size_t lds = 0) {
   if (blocks <= 0) return XG_OK;
   if (blocks > 0x7fffffff) return fail(XG_ERR_ARG, "launch grid too large");
   const bool timed = (sid >= 0 && sid == k->timed_sid && k->mode == kDirect);
@@ -256,7 +256,7 @@ int do_launch(xg_kernel* k, int32_t sid, void* fn, int64_t blocks, int threads, 
     XG_HIP(hipEventCreate(&ev.b));
     XG_HIP(hipEventRecord(ev.a, g_dev.stream));
   }
-  XG_HIP(hipModuleLaunchKernel((hipFunction_t)fn, (unsigned)blocks, 1, 1, (unsigned)threads, 1, 1, 0,
+  XG_HIP(hipModuleLaunchKernel((hipFunction_t)fn, (unsigned)blocks, 1, 1, (unsigned)threads, 1, 1, (unsigned)lds,
                                g_dev.stream, args, nullptr));
   if (timed) {
     XG_HIP(hipEventRecord(ev.b, g_dev.stream));
@@ -484,13 +484,108 @@ bool loop_blockable(xg_kernel* k, LoopPlan& L) {
     for (int r = 0; r < d.nrefs; ++r)
       if (d.ref_arg[r] != L.d.grid_arg && k->grids[(size_t)d.ref_arg[r]] == G) return false;
   }
-  if (L.grid != (const void*)G || L.mask_version != G->mask_version) {
-    L.state = 0;
-    L.validated = 0;
-    L.grid = G;
-    L.mask_version = G->mask_version;
+  if (L.mask_version != G->mask_version) {
+    LoopProof now;
+    now.mask_version = G->mask_version;
+    for (auto it = L.others.begin(); it != L.others.end(); ++it)
+      if (it->mask_version == G->mask_version) {
+        now = *it;
+        L.others.erase(it);
+        break;
+      }
+    if (L.mask_version && L.state != 0) {
+      if (L.others.size() >= kLoopProofs) L.others.pop_back();
+      L.others.insert(L.others.begin(), L);
+    }
+    static_cast<LoopProof&>(L) = now;
   }
   return true;
+}
+
+// Tiles along an axis of n cells: regions of r cells overlapping by 2 h, the first and
+// last on the grid's edges (xg::wave_axis).
+static int32_t wave_tiles(int32_t n, int32_t r, int32_t h) {
+  return n <= r ? 1 : (int32_t)ceil_div(n - 2 * h, r - 2 * h);
+}
+
+WaveCut wave_cut_for(const xg_loop_desc& d, WaveCut c, const WaveShape& s) {
+  const int32_t r = c.waves * d.wave[c.tile].rows;
+  const bool one = s.n0 <= r && s.n1 <= d.wave_cols;
+  c.halo = one ? 0 : s.reach[std::min(c.iters, XG_WAVE_MAX_ITERS) - 1];
+  c.nt0 = wave_tiles(s.n0, r, c.halo);
+  c.nt1 = wave_tiles(s.n1, d.wave_cols, c.halo);
+  return c;
+}
+
+// Estimated time of one launch of wave tiles, for choosing among cuts: memory traffic, and per
+// round of resident workgroups the iterations, each with the serial chain of one wave's
+// cells, the workgroup's exchange, and the cells of the waves that share a SIMD.  Fitted to
+// cavity sweeps of 65^2 to 2049^2 in both precisions, both tiles and 2 to 16 waves: the
+// cut it picks is within 8 % of the best of about 60 measured ones, mostly the best.
+static double wave_launch_us(const xg_loop_desc& d, const WaveCut& c, int64_t blocks) {
+  const xg_wave_tile& t = d.wave[c.tile];
+  const double cells = (double)t.rows * d.wave_cols / 64;   // of a lane
+  const int64_t cus = std::max(1, g_dev.cus);
+  int64_t per_cu = std::max<int64_t>(1, 4 * t.waves_per_simd / c.waves);
+  if (t.lds > 0) per_cu = std::max<int64_t>(1, std::min<int64_t>(per_cu, 163840 / ((int64_t)c.waves * t.lds)));
+  auto iteration = [&](int64_t n) {   // of n workgroups at once
+    const double per_simd = (double)std::min(per_cu, ceil_div(n, cus)) * c.waves / 4;
+    return 0.064 + 0.0376 * c.waves + 0.0715 * cells + 0.0099 * cells * std::max(1.0, per_simd);
+  };
+  const int64_t full = blocks / (cus * per_cu), rest = blocks % (cus * per_cu);
+  const double its = (double)full * iteration(cus * per_cu) + (rest ? iteration(rest) : 0.0);
+  return 5.0 + 4.42e-5 * (double)blocks * c.waves * cells * d.wave_elem / 4 + c.iters * its;
+}
+
+WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip) {
+  WaveCut best;
+  double best_us = 0.0;
+  for (int32_t t = 0; t < d.nwave; ++t)
+    for (int32_t w = 1; w <= d.wave[t].threads / 64; ++w) {
+      const int32_t r = w * d.wave[t].rows;
+      bool one = true;   // a tile holds every grid: no halo, and every iteration in one launch
+      int32_t widest[XG_WAVE_MAX_ITERS] = {};
+      for (const WaveShape& s : shapes) {
+        if (s.n0 <= r && s.n1 <= d.wave_cols) continue;
+        one = false;
+        for (int i = 0; i < XG_WAVE_MAX_ITERS; ++i) widest[i] = std::max<int32_t>(widest[i], s.reach[i]);
+      }
+      const int64_t most = std::min<int64_t>(trip, one ? kWaveSingleIters : XG_WAVE_MAX_ITERS);
+      for (int64_t T = one ? most : 1; T <= most; ++T) {
+        if (!one && (widest[T - 1] > XG_WAVE_MAX_HALO || r <= 2 * widest[T - 1] || d.wave_cols <= 2 * widest[T - 1])) break;
+        // of the lengths that take as many launches, the shortest
+        if (!one && T > 1 && ceil_div(trip, T - 1) == ceil_div(trip, T)) continue;
+        WaveCut c;
+        c.tile = t;
+        c.waves = w;
+        c.iters = (int32_t)T;
+        int64_t blocks = 0;
+        for (const WaveShape& s : shapes) blocks += wave_cut_for(d, c, s).blocks();
+        const double us = (double)ceil_div(trip, T) * wave_launch_us(d, c, blocks);
+        if (best.waves == 0 || us < best_us) {
+          best = c;
+          best_us = us;
+        }
+      }
+    }
+  return best;
+}
+
+void fill_wave_check(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int32_t* answer) {
+  fill_tb_hdr(k, L, TH, XG_WAVE_MAX_ITERS, answer);
+  const xg_grid* G = k->grids[(size_t)L.d.grid_arg];
+  TH.halo = XG_WAVE_MAX_HALO;
+  TH.nt0 = wave_tiles(G->shape[0], XG_WAVE_CHECK_ROWS, TH.halo);
+  TH.nt1 = wave_tiles(G->shape[1], XG_WAVE_CHECK_COLS, TH.halo);
+}
+
+void wave_answer(LoopPlan& L, const int32_t* answer) {
+  for (int i = 0; i < XG_WAVE_MAX_ITERS; ++i) L.reach[i] = (uint8_t)std::max(answer[i], i + 1);
+  L.state = 1;
+}
+
+bool wave_outrun(const LoopPlan& L, int64_t trip) {
+  return L.reach[std::min<int64_t>({trip, L.d.tmax, XG_WAVE_MAX_ITERS}) - 1] > XG_WAVE_MAX_HALO;
 }
 
 void fill_tb_hdr(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int iters, int32_t* fail_flag) {
@@ -506,6 +601,17 @@ void fill_tb_hdr(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int iters, int32_t* f
     const xg_stmt_desc& d = k->stmts[(size_t)L.d.sids[j]].d;
     TH.klass[j] = d.klass;
     if (!uniform_refs(k, d)) TH.uniform = 0;
+  }
+  const ClassPlan& p = G->plan(0);
+  if (p.kind == XG_DOM_BOX)
+    for (int a = 0; a < 2; ++a) {
+      TH.blo[a] = p.lo[a];
+      TH.bhi[a] = p.hi[a];
+    }
+  if (L.d.nwave) {
+    TH.nt0 = L.cut.nt0;
+    TH.nt1 = L.cut.nt1;
+    TH.halo = L.cut.halo;
   }
 }
 
@@ -716,10 +822,12 @@ int api_end(xg_kernel* k) {
 
 const int32_t* api_shape(xg_grid* g) { return g ? g->shape : nullptr; }
 
-// One launch of a blocked loop: `iters` iterations from level 0 into the scratch.
-int launch_blocked(xg_kernel* k, LoopPlan& L, xg_grid* G, const void* const* params, int iters, bool check) {
+// One launch of a blocked loop: `iters` iterations from level 0 into the scratch.  `check`:
+// the loop's checking launch (wave tiles: it runs no iterations, only follows the mask).
+int launch_blocked(xg_kernel* k, LoopPlan& L, xg_grid* G, const void* const* params, int64_t iters, bool check) {
   xg_tb_hdr TH;
-  fill_tb_hdr(k, L, TH, iters, k->d_fail);
+  if (L.d.nwave && check) fill_wave_check(k, L, TH, k->d_fail);
+  else fill_tb_hdr(k, L, TH, (int)iters, k->d_fail);
   const int m = L.d.nstmts;
   std::vector<std::vector<xg_gview>> refs((size_t)m);
   std::vector<void*> args;
@@ -733,9 +841,39 @@ int launch_blocked(xg_kernel* k, LoopPlan& L, xg_grid* G, const void* const* par
     args.push_back(refs[(size_t)j].data());
     args.push_back(const_cast<void*>(params[j]));
   }
-  const int64_t blocks = ceil_div(G->shape[0], L.d.core0) * ceil_div(G->shape[1], L.d.core1);
+  if (L.d.nwave && check)
+    return do_launch(k, -1, L.d.fn_wcheck, (int64_t)TH.nt0 * TH.nt1, kWaveCheckThreads, args.data());
   L.launches++;
+  if (L.d.nwave) {
+    const xg_wave_tile& w = L.d.wave[L.cut.tile];
+    return do_launch(k, -1, w.fn, L.cut.blocks(), L.cut.waves * 64, args.data(), (size_t)L.cut.waves * w.lds);
+  }
+  const int64_t blocks = ceil_div(G->shape[0], L.d.core0) * ceil_div(G->shape[1], L.d.core1);
   return do_launch(k, -1, check ? L.d.fn_check : L.d.fn, blocks, L.d.threads, args.data());
+}
+
+// The launches of `trip` iterations of a proven loop.
+int run_blocked(xg_kernel* k, LoopPlan& L, xg_grid* G, const void* const* params, int64_t trip) {
+  for (int64_t T; trip > 0; trip -= T) {
+    T = std::min<int64_t>(L.d.nwave ? L.cut.iters : L.d.tmax, trip);
+    if (int rc = launch_blocked(k, L, G, params, T, false)) return rc;
+    std::swap(G->levels[0], G->scratch);
+  }
+  return XG_OK;
+}
+
+// Run a plan's checking launch and read its answer (kCheckBytes).
+int check_blocked(xg_kernel* k, LoopPlan& L, xg_grid* G, const void* const* params, int64_t iters, int32_t* answer) {
+  if (!k->d_fail) {
+    void* p = nullptr;
+    if (int rc = dev_alloc(kCheckBytes, true, &p)) return rc;
+    k->d_fail = (int32_t*)p;
+  }
+  XG_HIP(hipMemsetAsync(k->d_fail, 0, kCheckBytes, g_dev.stream));
+  if (int rc = launch_blocked(k, L, G, params, iters, true)) return rc;
+  XG_HIP(hipMemcpyAsync(answer, k->d_fail, kCheckBytes, hipMemcpyDeviceToHost, g_dev.stream));
+  XG_HIP(hipStreamSynchronize(g_dev.stream));
+  return XG_OK;
 }
 
 int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params, int32_t n) {
@@ -779,15 +917,16 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
     account();
     return 1;
   }
-  if (!k->blocked || trip <= 0 || !L.d.fn) return 0;
+  if (!k->blocked || trip <= 0 || (!L.d.fn && !L.d.nwave)) return 0;
   xg_grid* G = k->grids[(size_t)L.d.grid_arg];
   if (!loop_blockable(k, L)) return 0;
   if (L.state < 0) return 0;
   // A check proves launches of up to the iterations it ran: the set of exact region
   // cells only shrinks from one iteration to the next, so a proof at T covers fewer
   // iterations, but a launch of more iterations than any check ran needs its own.
-  const int T0 = (int)std::min<int64_t>(L.d.tmax, trip);
-  const bool check = L.state == 0 || T0 > L.validated;
+  const int64_t tmax = std::min<int64_t>(L.d.tmax, trip);
+  // (wave tiles: one check per mask says what every number of iterations needs)
+  const bool check = L.state == 0 || (!L.d.nwave && tmax > L.validated);
   if (check && k->mode == kCapture) return 0;  // validation needs a synchronisation
   int rc = flush(k);
   if (rc) {
@@ -796,44 +935,38 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
   }
   int64_t done = 0;
   if (check) {
-    if (!k->d_fail) {
-      void* p = nullptr;
-      if (int e = dev_alloc(sizeof(int32_t), true, &p)) {
-        set_status(k, e);
-        return 1;
-      }
-      k->d_fail = (int32_t*)p;
-    }
-    int32_t h_fail = 0;
-    const int T = T0;
-    if (hipMemsetAsync(k->d_fail, 0, sizeof(int32_t), g_dev.stream) != hipSuccess ||
-        (rc = launch_blocked(k, L, G, params, T, true)) != XG_OK ||
-        hipMemcpyAsync(&h_fail, k->d_fail, sizeof(int32_t), hipMemcpyDeviceToHost, g_dev.stream) != hipSuccess ||
-        hipStreamSynchronize(g_dev.stream) != hipSuccess) {
-      set_status(k, rc ? rc : fail(XG_ERR_HIP, "blocked-loop validation failed"));
-      return 1;
-    }
-    if (h_fail) {  // some core cell depends on data outside its tile's halo: the scratch is discarded
-      L.state = -1;
-      return 0;
-    }
-    L.state = 1;
-    L.validated = std::max(L.validated, T);
-    std::swap(G->levels[0], G->scratch);
-    done = T;
-    L.iterations += T;
-  }
-  while (done < trip) {
-    const int T = (int)std::min<int64_t>(L.d.tmax, trip - done);
-    rc = launch_blocked(k, L, G, params, T, false);
-    if (rc) {
+    int32_t answer[XG_WAVE_MAX_ITERS];
+    if ((rc = check_blocked(k, L, G, params, tmax, answer))) {
       set_status(k, rc);
       return 1;
     }
-    std::swap(G->levels[0], G->scratch);
-    done += T;
-    L.iterations += T;
+    if (L.d.nwave) {
+      wave_answer(L, answer);
+    } else if (answer[0]) {  // some core cell depends on data outside its tile's halo: the scratch is discarded
+      L.state = -1;
+      return 0;
+    } else {   // the checking variant also ran these iterations
+      L.state = 1;
+      L.validated = std::max(L.validated, (int)tmax);
+      std::swap(G->levels[0], G->scratch);
+      done = tmax;
+      L.iterations += tmax;
+    }
   }
+  if (L.d.nwave) {
+    if (wave_outrun(L, trip)) {
+      L.state = -1;
+      return 0;
+    }
+    L.cut = wave_choose(L.d, {wave_shape(G, L)}, trip);
+    if (L.cut.waves == 0) return 0;
+    L.cut = wave_cut_for(L.d, L.cut, wave_shape(G, L));
+  }
+  if ((rc = run_blocked(k, L, G, params, trip - done))) {
+    set_status(k, rc);
+    return 1;
+  }
+  L.iterations += trip - done;
   account();
   return 1;
 }
@@ -1213,7 +1346,11 @@ int xg_kernel_create(int32_t nstmts, const xg_stmt_desc* stmts, int32_t ngroups,
     const xg_loop_desc& d = loops[i];
     bool ok = d.nstmts >= 1 && d.nstmts <= XG_LOOP_MAX_STMTS && d.grid_arg >= 0 && d.grid_arg < ngrids &&
               d.core0 > 0 && d.core1 > 0 && d.tmax >= 1 && d.halo >= 0 && d.threads >= 64 &&
-              d.threads <= 1024 && d.threads % 64 == 0;
+              d.threads <= 1024 && d.threads % 64 == 0 && d.nwave >= 0 && d.nwave <= XG_LOOP_MAX_WAVE;
+    for (int t = 0; ok && t < d.nwave; ++t)
+      ok = d.wave[t].rows >= 1 && d.wave[t].threads >= 64 && d.wave[t].threads <= 1024 &&
+           d.wave[t].threads % 64 == 0 && d.wave[t].lds >= 0 &&
+           d.wave[t].waves_per_simd >= 1 && d.wave_cols >= 64 && d.wave_cols % 64 == 0 && d.wave_elem > 0 && d.wave[t].fn && d.fn_wcheck;
     for (int j = 0; ok && j < d.nstmts; ++j)
       ok = d.sids[j] >= 0 && d.sids[j] < nstmts && k->stmts[(size_t)d.sids[j]].d.store_arg == d.grid_arg &&
            k->stmts[(size_t)d.sids[j]].d.dims == 2;
@@ -1288,22 +1425,17 @@ int xg_kernel_time_loop(xg_kernel* k, int32_t lid, int32_t trip, int32_t reps, d
   xg_grid* G = k->grids[(size_t)L.d.grid_arg];
   std::vector<const void*> ps;
   for (auto& p : L.last_params) ps.push_back(p.data());
-  // one trip = the launches a call makes for `trip` iterations (chunks of tmax)
+  // one trip = the launches a call makes for `trip` iterations
   auto run_trip = [&]() -> int {
-    for (int done = 0; done < trip;) {
-      const int T = std::min(L.d.tmax, trip - done);
-      int rc = launch_blocked(k, L, G, ps.data(), T, false);
-      if (rc) return rc;
-      std::swap(G->levels[0], G->scratch);
-      done += T;
-    }
-    return XG_OK;
+    if (L.d.nwave) L.cut = wave_cut_for(L.d, wave_choose(L.d, {wave_shape(G, L)}, trip), wave_shape(G, L));
+    return run_blocked(k, L, G, ps.data(), trip);
   };
-  const int64_t per_trip = ceil_div(trip, L.d.tmax);
   hipEvent_t e0, e1;
   XG_HIP(hipEventCreate(&e0));
   XG_HIP(hipEventCreate(&e1));
+  const int64_t before = L.launches;
   int rc = run_trip();
+  const int64_t per_trip = L.launches - before;
   if (!rc) {
     XG_HIP(hipEventRecord(e0, g_dev.stream));
     for (int i = 0; i < reps && !rc; ++i) rc = run_trip();

@@ -112,6 +112,21 @@ class GroupMeta:
 
 
 @dataclass
+class WaveTile:
+    """A wave-tile kernel of a blocked loop (see Emitter._tb_kernel_wave)."""
+    kernel: str
+    rows: int                     # region rows a wave holds
+    k: int                        # region columns a lane holds (64 * k columns)
+    threads: int                  # most work-items of a workgroup
+    lds: int                      # LDS bytes per wave: two halves of its first and last row, membership bits
+    waves_per_simd: int           # what its registers leave room for (launch bounds ask for it)
+
+    @property
+    def cols(self) -> int:
+        return 64 * self.k
+
+
+@dataclass
 class LoopMeta:
     """A `for` loop that may run temporally blocked (several iterations per launch)."""
     lid: int
@@ -128,6 +143,14 @@ class LoopMeta:
     alt: object = None            # LoopMeta of the same loop with the tile used on small grids
     alt_max_cells: int = 0        # ... on grids of at most this many cells
     batched: bool = True          # emit the batched variants (the small-grid tile has none)
+    # wave tiles: where a loop has any, they run it (every plan of it), and the kernels of
+    # the tile shape above are not built; the shape still names the loop's plans (by grid size)
+    waves: list = field(default_factory=list)
+
+    @property
+    def wave_check(self) -> str:
+        """The kernel that proves a wave-tile cut exact (batched: the same name and "b")."""
+        return f"xg_tb{self.lid}_chk"
 
 
 @dataclass
@@ -847,6 +870,7 @@ class Emitter:
         out.append(f"struct xg_r{sid} {{ xg_gview v[{nr}]; }};")
         # DV: the statement's uniform divisors were found to be exact powers of two for
         # this launch (dv_ok), so xg::udiv multiplies by their reciprocals
+        at = len(out)
         out.append(f"template <bool DV> struct xg_s{sid}_t {{")
         out.append(f"  typedef {T} T; typedef xg_r{sid} Refs; typedef xg_p{sid} Params;")
         out.append(f"  static constexpr int NDV = {len(udivs)};")
@@ -912,7 +936,8 @@ class Emitter:
             gts = {n: t for _, n, t in self.func.grid_args}
             out.append(f"  static constexpr int NPRE = {len(pre_slots)};")
             fields_ = " ".join(f"{device_type_name(gts[g].element)} v{i};" for i, (g, _, _) in enumerate(pre_slots))
-            out.append(f"  struct Pre {{ {fields_ or 'int32_t unused;'} }};")
+            out.insert(at, f"struct xg_e{sid} {{ {fields_ or 'int32_t unused;'} }};")
+            out.append(f"  typedef xg_e{sid} Pre;")
             out.append("  template <bool SAFE>")
             out.append("  __device__ static __forceinline__ void prefetch(Pre& pre, const Refs& R, const int32_t* sh, "
                        "int i0, int i1, int i2) {")
@@ -924,6 +949,31 @@ class Emitter:
                 o3 = [str(offs[d]) if d < gt.dimension else "0" for d in range(3)]
                 out.append(f"    pre.v{i} = xg::ld<{device_type_name(gt.element)}, {gt.dimension}, XG_OVERSTEP, SAFE>"
                            f"(R.v[{r}], sh, xc, {', '.join(o3)}, i0, i1, i2);")
+            out.append("  }")
+            # ... for K adjacent cells of a row from column i1 (SAFE: as one vector per load)
+            out.append("  template <bool SAFE, int K>")
+            out.append("  __device__ static __forceinline__ void prefetch_row(Pre* pre, const Refs& R, const int32_t* sh, "
+                       "int i0, int i1) {")
+            out.append("    if constexpr (!SAFE) {")
+            out.append("#pragma unroll")
+            out.append("      for (int k = 0; k < K; ++k) prefetch<false>(pre[k], R, sh, i0, i1 + k, 0);")
+            out.append("    } else {")
+            out.append(f"      const int64_t xc = xg::lin<{D}>(sh, i0, i1, 0);")
+            out.append("      (void)pre; (void)R; (void)xc;")
+            for i, (g, lvl, offs) in enumerate(pre_slots):
+                et = device_type_name(gts[g].element)
+                r = refs.index((g, lvl))
+                o3 = [str(offs[d]) if d < gts[g].dimension else "0" for d in range(3)]
+                if gts[g].dimension == D and et in ("float", "double"):
+                    out.append(f"      {{ const xg::vecu<{et}, K> w = *(xg::gptr<const xg::vecu<{et}, K>>)"
+                               f"(xg::gp<const {et}>(R.v[{r}].ptr) + xc + xg::off<{D}>(sh, {', '.join(o3)}));")
+                    out.append("#pragma unroll")
+                    out.append(f"        for (int k = 0; k < K; ++k) pre[k].v{i} = w[k]; }}")
+                else:
+                    out.append("#pragma unroll")
+                    out.append(f"      for (int k = 0; k < K; ++k) pre[k].v{i} = xg::ld<{et}, {gts[g].dimension}, "
+                               f"XG_OVERSTEP, true>(R.v[{r}], sh, xc + k, {', '.join(o3)}, i0, i1 + k, 0);")
+            out.append("    }")
             out.append("  }")
             out.append("  __device__ static __forceinline__ T value_rgp(const T* s, const Refs& R, const Params& P, "
                        "const Pre& pre) {")
@@ -1245,17 +1295,12 @@ class Emitter:
         body runs (read through the table's generic pointers they could alias the
         body's stores and would be re-read for every cell); the barrier lets the
         workgroup reuse its LDS for its next tile."""
-        loc = ["const xg_tb_hdr th = e.th;"]
-        for j, s in enumerate(L.stmts):
-            sid = s.stmt.sid
-            loc.append(f"const xg_r{sid} r{j} = *xg::cp<xg_r{sid}>(e.refs[{j}]);")
-            loc.append(f"const xg_p{sid} p{j} = *xg::cp<xg_p{sid}>(e.params[{j}]);")
-        bcall = ", ".join(["th"] + [f"r{j}, p{j}" for j in range(len(L.stmts))] + ["(int)t"])
+        loc, bcall = self._tb_entry_locals(L)
         for suffix, chk in (("_b", "false"), ("_chkb", "true")):
             out.append(f'extern "C" __global__ void {self._tb_bounds(L, chk == "true")} {L.kernel}{suffix}('
                        f"const xg_btent* __restrict__ E, const int32_t n, const int64_t total) "
                        f"{{ xg::for_batch_tiles(E, n, total, [&](const xg_btent& e, uint32_t t) "
-                       f"{{ {' '.join(loc)} {L.kernel}_body<{chk}, false>({bcall}); __syncthreads(); }}); }}")
+                       f"{{ {loc} {L.kernel}_body<{chk}, false>({bcall}); __syncthreads(); }}); }}")
 
     def _tb_kernel_reg(self, L: LoopMeta, out: list):
         """Blocked kernel of one loop.  A workgroup owns a core tile of the loop grid
@@ -1432,6 +1477,387 @@ class Emitter:
         if L.batched:
             self._tb_batched(L, out)
 
+    def _tb_kernel_wave(self, L: LoopMeta, V: WaveTile, out: list):
+        """Blocked kernel of one loop on a wave tile.  A workgroup of up to `threads`
+        work-items keeps a region of the loop's grid in registers for several
+        iterations of the body: wave w holds `rows` rows of 64 * k columns, lane c
+        columns k * c .. k * c + k - 1 of each (read and written as one vector).  A
+        read one row away comes from the lane's own registers, or through LDS where it
+        crosses into the next wave's rows; one column away, from the lane's other
+        columns or, over a DPP lane shift, its neighbour's.
+
+        What bounds it: vector issue.  A cavity sweep is 8 FP64 operations per cell (4
+        cycles per wave each) and here little else: inside the box of class 0 a cell is 10
+        instructions (7 FP64 where the divisor is a power of two, one product moved out of
+        the iterations, and 2 lane moves), with no test, select, index or LDS read per cell; the
+        LDS layout spends about 40, and its region fills the LDS where this one
+        fills registers.  50 cavity sweeps (1 launch = T iterations) with the LDS layout
+        and with this one: 2049^2 FP64 580 -> 242 us, FP32 459 -> 189 us, 1000^2 FP64
+        251 -> 135 us, 300^2 FP32 120 -> 81 us, 65^2 FP64 116 -> 81 us.
+
+        `rows` 8 and 4 measured: 8 rows read and exchange less per cell (2049^2 FP64 with
+        16 waves 46 us a launch against 50), 4 rows leave shorter chains to the small grids (65^2
+        to 1000^2: 1.2 to 1.3 times faster).  12 to 24 rows with fewer waves were 2 to 4 times
+        slower at 2049^2: the compiler spills there (edge tiles wait for scratch memory)."""
+        o = out.append
+        T = device_type_name(L.stmts[0].stmt.gtype.element)
+        m = len(L.stmts)
+        K, BR = V.k, V.rows
+        bits = BR * K
+        assert bits <= 64 and BR <= 32 and L.reach == 1
+        params = ["const xg_tb_hdr& TH"] + [f"const xg_r{s.stmt.sid}& R{j}, const xg_p{s.stmt.sid}& P{j}"
+                                            for j, s in enumerate(L.stmts)]
+        # reach of the loads that come from global memory (other grids / levels)
+        rl, rh = [0, 0], [0, 0]
+        for s in L.stmts:
+            for n in ir.walk(s.stmt.node.value):
+                if isinstance(n, ir.Cell) and not (n.grid.name == L.grid and n.level == 0):
+                    for d in range(2):
+                        rl[d] = max(rl[d], -n.offsets[d])
+                        rh[d] = max(rh[d], n.offsets[d])
+        o("template <bool DVOK>")
+        o(f"__device__ __forceinline__ void {V.kernel}_body({', '.join(params)}, const int tile) {{")
+        o(f"  typedef {T} T;")
+        o(f"  constexpr int BR = {BR}, K = {K}, RW = 64 * K;")
+        o(f"  typedef uint{32 if bits <= 32 else 64}_t MB;   /* a bit per cell of a lane */")
+        # the bands' edge rows, double buffered (alternate exchanges use alternate halves)
+        # (dynamic LDS, sized by the waves of the launch: V.lds bytes each)
+        o("  extern __shared__ __attribute__((aligned(16))) unsigned char wave_lds[];")
+        o("  typedef T Rows[2][RW];")
+        o("  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
+        o("  const int WV = blockDim.x >> 6, RH = WV * BR;")
+        o("  Rows* const ex = (Rows*)wave_lds;                 /* [2 WV]: half, wave; first and last row */")
+        o(f"  MB* const smb = (MB*)(ex + 2 * WV) + threadIdx.x * {m};   /* this lane's membership bits */")
+        o("  const int32_t* sh = TH.src.shape;")
+        o("  const int N0 = sh[0], N1 = sh[1];")
+        o("  const int t0 = tile / TH.nt1, t1 = tile - t0 * TH.nt1;")
+        o("  const xg::wave_axis A0(t0, TH.nt0, N0, RH, TH.halo), A1(t1, TH.nt1, N1, RW, TH.halo);")
+        o("  const int r0 = A0.start, c0 = A1.start;")
+        o("  const int gr = r0 + w * BR, gc = c0 + lane * K;   /* this wave's first row, this lane's first column */")
+        # a grid smaller than the region leaves region cells outside it: never members of a
+        # class, read at clamped addresses, and not written
+        o("  const bool full = r0 + RH <= N0 && c0 + RW <= N1;")
+        o("  const bool inbox = full && r0 >= TH.blo[0] && r0 + RH <= TH.bhi[0] && c0 >= TH.blo[1] && c0 + RW <= TH.bhi[1];")
+        o(f"  const bool safe = full && TH.uniform && r0 - {rl[0]} >= 0 && r0 + RH + {rh[0]} <= N0 && "
+          f"c0 - {rl[1]} >= 0 && c0 + RW + {rh[1]} <= N1;")
+        o("  const xg::gptr<const T> __restrict__ src = xg::gp<const T>(TH.src.ptr);")
+        o("  T V[BR][K];")
+        o("  if (full) {")
+        o("#pragma unroll")
+        o("    for (int q = 0; q < BR; ++q) {")
+        o("      const xg::vecu<T, K> x = *(xg::gptr<const xg::vecu<T, K>>)(src + ((int64_t)(gr + q) * N1 + gc));")
+        o("#pragma unroll")
+        o("      for (int k = 0; k < K; ++k) V[q][k] = x[k];")
+        o("    }")
+        o("  } else {")
+        o("#pragma unroll")
+        o("    for (int q = 0; q < BR; ++q)")
+        o("#pragma unroll")
+        o("      for (int k = 0; k < K; ++k) V[q][k] = src[(int64_t)min(gr + q, N0 - 1) * N1 + min(gc + k, N1 - 1)];")
+        o("  }")
+        o("  int xb = 0;                 /* exchange buffer half */")
+        o("  T U[K], D[K];               /* the rows above and below this wave's */")
+        o("  auto exchange = [&]() {")
+        o("    typedef xg::vecn<T, K> VT;")
+        o("    VT a, b;")
+        o("#pragma unroll")
+        o("    for (int k = 0; k < K; ++k) { a[k] = V[0][k]; b[k] = V[BR - 1][k]; }")
+        o("    Rows* const e = ex + xb * WV;")
+        o("    *(VT*)&e[w][0][lane * K] = a;")
+        o("    *(VT*)&e[w][1][lane * K] = b;")
+        o("    __syncthreads();")
+        o("    a = *(const VT*)&e[w > 0 ? w - 1 : 0][1][lane * K];")
+        o("    b = *(const VT*)&e[w < WV - 1 ? w + 1 : w][0][lane * K];")
+        o("#pragma unroll")
+        o("    for (int k = 0; k < K; ++k) { U[k] = a[k]; D[k] = b[k]; }")
+        o("    xb ^= 1;")
+        o("  };")
+        o("#pragma unroll")
+        o("  for (int k = 0; k < K; ++k) U[k] = D[k] = T(0);")
+        def gather(reads, down, ind):
+            """The statement's distinct reads of the loop grid, for column k of row q.  Every
+            lane of the wave runs them (lane shifts read other lanes' registers)."""
+            o(f"{ind}T s[{max(1, len(reads))}]; s[0] = T(0);")
+            row = {-1: "prev" if down else "next", 0: "cur", 1: "next" if down else "prev"}
+            for i, (d0, d1) in enumerate(reads):
+                a = row[d0]
+                if d1 == 0:
+                    o(f"{ind}s[{i}] = {a}[k];")
+                elif d1 > 0:
+                    o(f"{ind}if (k + 1 < K) s[{i}] = {a}[k + 1 < K ? k + 1 : 0]; else s[{i}] = xg::lane_shift<1>({a}[0]);")
+                else:
+                    o(f"{ind}if (k > 0) s[{i}] = {a}[k > 0 ? k - 1 : 0]; else s[{i}] = xg::lane_shift<-1>({a}[K - 1]);")
+
+        def cells(j, s, down, dv, rowtest=None, member=False):
+            """One statement over the wave's rows, downwards or upwards: the cells of a row
+            (where `rowtest` holds) from the old values (`prev`, the old row passed last, is
+            kept); `member`: stored where the lane's cell is a member."""
+            S = f"xg_s{s.stmt.sid}_t<{dv}>"
+            if s.stmt.sid in self._prefetched:
+                value = f"{S}::value_rgp(s, R{j}, P{j}, pre{j}[q][k])"
+            else:
+                value = f"{S}::template value_rg<false>(s, R{j}, P{j}, sh, gr + q, gc + k, 0)"
+            o("      T prev[K];")
+            o("#pragma unroll")
+            o(f"      for (int k = 0; k < K; ++k) prev[k] = {'U' if down else 'D'}[k];")
+            o("#pragma unroll")
+            o("      for (int r = 0; r < BR; ++r) {")
+            o(f"        const int q = {'r' if down else 'BR - 1 - r'};")
+            o("        T cur[K], next[K];")
+            o("#pragma unroll")
+            o("        for (int k = 0; k < K; ++k) {")
+            o("          cur[k] = V[q][k];")
+            o("          next[k] = " + ("q + 1 < BR ? V[q + 1 < BR ? q + 1 : q][k] : D[k];" if down else
+                                        "q > 0 ? V[q > 0 ? q - 1 : 0][k] : U[k];"))
+            o("        }")
+            o("        (void)prev; (void)next;")
+            if rowtest:
+                o(f"        if ({rowtest}) {{")
+            o("#pragma unroll")
+            o("        for (int k = 0; k < K; ++k) {")
+            gather(self._tb_reads[s.stmt.sid], down, "          ")
+            o(f"          const T x = {value};")
+            o(f"          V[q][k] = {'((mb >> (q * K + k)) & 1u) != 0u ? x : cur[k]' if member else 'x'};")
+            o("        }")
+            if rowtest:
+                o("        }")
+            o("#pragma unroll")
+            o("        for (int k = 0; k < K; ++k) prev[k] = cur[k];")
+            # the scheduler would start later rows early and run out of registers
+            o("        __builtin_amdgcn_sched_barrier(0);")
+            o("      }")
+
+        def prefetch():
+            for j, s in enumerate(L.stmts):
+                if s.stmt.sid in self._prefetched:
+                    S = f"xg_s{s.stmt.sid}"
+                    o(f"  typename {S}::Pre pre{j}[BR][K];")
+                    for cond, safe in (("if (safe)", "true"), ("else", "false")):
+                        o(f"  {cond} {{")
+                        o("#pragma unroll")
+                        o(f"    for (int q = 0; q < BR; ++q) {S}::template prefetch_row<{safe}, K>(pre{j}[q], R{j}, sh, "
+                          "gr + q, gc);")
+                        o("  }")
+
+        def iterations(body):
+            # Iterations run down the rows and up again in turn.  A new row is made where the old row
+            # passed last has just died, so rows move one register up in one iteration and back
+            # in the next; all downwards, the rows would be copied on every iteration (and the
+            # second copy of the region takes the registers of a wave per SIMD).  An odd count
+            # starts with one iteration on its own.
+            o("  if (TH.iters & 1) {")
+            body(False)
+            o("  }")
+            o("  for (int it = TH.iters >> 1; it > 0; --it) {")
+            body(True)
+            body(False)
+            o("  }")
+
+        def vertical(s):
+            return any(r[0] != 0 for r in self._tb_reads[s.stmt.sid])
+
+        def inner(down):
+            for j, s in enumerate(L.stmts):
+                if s.stmt.klass != 0:
+                    continue
+                o("    {")
+                if vertical(s):
+                    o("      exchange();")
+                cells(j, s, down, "DV")
+                o("    }")
+
+        def edge(down):
+            for j, s in enumerate(L.stmts):
+                if s.stmt.klass == 0:
+                    # run by every wave: rows move between registers, which a way round it would undo
+                    o("    {")
+                    if vertical(s):
+                        o("      exchange();")
+                    o(f"      const MB mb = smb[{j}];")
+                    cells(j, s, down, "DV", None, True)
+                    o("    }")
+                    continue
+                o(f"    if (any & {1 << j}u) {{")
+                if vertical(s):
+                    # members that read no row of another wave need no exchange
+                    o(f"      if (cross & {1 << j}u) exchange();")
+                o(f"      if (rb{j}) {{")
+                o(f"        const MB mb = smb[{j}];")
+                # opaque each time: the compiler would keep every row's test (a pair of scalar
+                # registers each) across the iterations, and spill them
+                o(f"        uint32_t rows = rb{j};")
+                o('        asm volatile("" : "+s"(rows));')
+                cells(j, s, down, "false", "(rows >> q) & 1u", True)
+                o("      }")
+                o("    }")
+
+        dvs = [f"xg_s{s.stmt.sid}::dv_ok(R{j}, P{j})" for j, s in enumerate(L.stmts) if self._dv.get(s.stmt.sid)]
+        # every uniform divisor has a reciprocal form in this launch
+        o(f"  const bool dv = {' && '.join(dvs) if dvs else 'false'};")
+        o("  (void)dv;")
+        def run(body):
+            o("  auto run = [&](auto dv_c) {")
+            o("  constexpr bool DV = decltype(dv_c)::value;   /* reciprocal form of uniform divisions */")
+            o("  (void)DV;")
+            prefetch()
+            iterations(body)
+            o("  };")
+            o("  if constexpr (DVOK) { if (dv) run(xg::bconst<true>()); else run(xg::bconst<false>()); }")
+            o("  else run(xg::bconst<false>());")
+
+        # A region inside the box of class 0 runs that class's statements on every cell: no mask
+        # is read, nothing is tested or selected.
+        o("  if (inbox) {")
+        run(inner)
+        o("  } else {")
+        # Elsewhere a bit per cell (smb) says where the lane's cells are members of each statement's
+        # class.  rb: the rows that some lane has members in; any: the statements some wave of
+        # the workgroup has members of; cross: those with members that read another wave's row.
+        for j in range(m):
+            o(f"  MB mb{j} = 0u;")
+            o(f"  uint32_t rb{j} = 0u;")
+        o("#pragma unroll 4")
+        o("  for (int q = 0; q < BR; ++q)")
+        o("#pragma unroll")
+        o("    for (int k = 0; k < K; ++k) {")
+        o("      const bool in = gr + q < N0 && gc + k < N1;")
+        o("      int32_t c = 0;")
+        o("      if (in && TH.mask) c = xg::gp<const int32_t>(TH.mask)[(int64_t)(gr + q) * N1 + gc + k];")
+        o("      const MB bit = in ? (MB)1u << (q * K + k) : (MB)0u;")
+        for j in range(m):
+            o(f"      if (c == TH.klass[{j}]) mb{j} |= bit;")
+        o("    }")
+        o("#pragma unroll 1")
+        o("  for (int q = 0; q < BR; ++q) {")
+        for j in range(m):
+            o(f"    if (__ballot(((mb{j} >> (q * K)) & {(1 << K) - 1}u) != 0u)) rb{j} |= 1u << q;")
+        o("  }")
+        o("  uint32_t any = 0u, cross = 0u;")
+        for j, s in enumerate(L.stmts):
+            o(f"  smb[{j}] = mb{j};")
+            o(f"  rb{j} = __builtin_amdgcn_readfirstlane(rb{j});")
+            o(f"  if (rb{j}) any |= {1 << j}u;")
+            for d0, test in ((-1, f"rb{j} & 1u"), (1, f"(rb{j} >> (BR - 1)) & 1u")):
+                if any(r[0] == d0 for r in self._tb_reads[s.stmt.sid]):
+                    o(f"  if ({test}) cross |= {1 << j}u;")
+        o("  any = __builtin_amdgcn_readfirstlane(xg::block_or(any | cross << 16));")
+        o("  cross = any >> 16;")
+        run(edge)
+        o("  }")
+        o("  const xg::gptr<T> __restrict__ dst = xg::gp<T>(TH.dst.ptr);")
+        o("#pragma unroll")
+        o("  for (int q = 0; q < BR; ++q) {")
+        o("    const int row = gr + q;")
+        o("    if (row < A0.w0 || row >= A0.w1) continue;")
+        o("    const xg::gptr<T> p = dst + ((int64_t)row * N1 + gc);")
+        o("    if (gc >= A1.w0 && gc + K <= A1.w1) {")
+        o("      xg::vecu<T, K> x;")
+        o("#pragma unroll")
+        o("      for (int k = 0; k < K; ++k) x[k] = V[q][k];")
+        o("      *(xg::gptr<xg::vecu<T, K>>)p = x;")
+        o("    } else {")
+        o("#pragma unroll")
+        o("      for (int k = 0; k < K; ++k)")
+        o("        if (gc + k >= A1.w0 && gc + k < A1.w1) p[k] = V[q][k];")
+        o("    }")
+        o("  }")
+        o("}")
+        kargs = ["const xg_tb_hdr TH"] + [f"const xg_r{s.stmt.sid} R{j}, const xg_p{s.stmt.sid} P{j}"
+                                          for j, s in enumerate(L.stmts)]
+        call = ", ".join(["TH"] + [f"R{j}, P{j}" for j in range(m)] + ["(int)xg::xcd_remap(blockIdx.x, gridDim.x)"])
+        bounds = f"__launch_bounds__({V.threads}) __attribute__((amdgpu_waves_per_eu({V.waves_per_simd})))"
+        o(f'extern "C" __global__ void {bounds} {V.kernel}({", ".join(kargs)}) {{ {V.kernel}_body<true>({call}); }}')
+        loc, bcall = self._tb_entry_locals(L)
+        o(f'extern "C" __global__ void {bounds} {V.kernel}_b(const xg_btent* __restrict__ E, const int32_t n, '
+          f"const int64_t total) {{ xg::for_batch_tiles(E, n, total, [&](const xg_btent& e, uint32_t t) "
+          f"{{ {loc} {V.kernel}_body<false>({bcall}); __syncthreads(); }}); }}")
+
+    @staticmethod
+    def _tb_entry_locals(L: LoopMeta) -> tuple:
+        """A batched blocked kernel's copies of its entry's structs, and the body's arguments."""
+        loc = ["const xg_tb_hdr th = e.th;"]
+        for j, s in enumerate(L.stmts):
+            sid = s.stmt.sid
+            loc.append(f"const xg_r{sid} r{j} = *xg::cp<xg_r{sid}>(e.refs[{j}]);")
+            loc.append(f"const xg_p{sid} p{j} = *xg::cp<xg_p{sid}>(e.params[{j}]);")
+        return " ".join(loc), ", ".join(["th"] + [f"r{j}, p{j}" for j in range(len(L.stmts))] + ["(int)t"])
+
+    def _tb_wave_check(self, L: LoopMeta, out: list):
+        """How far from a cell lie the initial values that its value depends on after each
+        of XG_WAVE_MAX_ITERS iterations (to the left, right, above or below, the largest
+        over the grid): TH.fail[i] for i + 1 iterations, the halo that a region needs
+        then, wherever the grid is cut; 255 where a member cell reads outside the grid
+        or the distance passes XG_WAVE_MAX_HALO.  Followed statement by statement; only
+        the mask decides, no field value is read, and it runs once per mask.  Inside the
+        box of class 0, where at most one statement runs, the distance is the number of
+        iterations (which the host takes as the least) and is not followed."""
+        o = out.append
+        m = len(L.stmts)
+        name = L.wave_check
+        o(f"__device__ __forceinline__ void {name}_body(const xg_tb_hdr& TH, const int tile) {{")
+        o("  constexpr int RH = XG_WAVE_CHECK_ROWS, RW = XG_WAVE_CHECK_COLS, NR = RH * RW;")
+        # extents of a cell: a byte each for left, right, above, below; 255: unknown
+        o("  __shared__ uint8_t mem[NR];")
+        o("  __shared__ uint32_t ext[2][NR];")
+        o("  __shared__ uint32_t far[XG_WAVE_MAX_ITERS];")
+        o("  if (threadIdx.x < XG_WAVE_MAX_ITERS) far[threadIdx.x] = 0u;")
+        o("  const int N0 = TH.src.shape[0], N1 = TH.src.shape[1];")
+        o("  const int t0 = tile / TH.nt1, t1 = tile - t0 * TH.nt1;")
+        o("  const xg::wave_axis A0(t0, TH.nt0, N0, RH, TH.halo), A1(t1, TH.nt1, N1, RW, TH.halo);")
+        if sum(s.stmt.klass == 0 for s in L.stmts) <= 1:
+            o("  if (A0.start >= TH.blo[0] && A0.start + RH <= TH.bhi[0] && A1.start >= TH.blo[1] && "
+              "A1.start + RW <= TH.bhi[1]) return;")
+        o("  for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
+        o("    const int r = A0.start + i / RW, c = A1.start + i % RW;")
+        o("    const bool in = r < N0 && c < N1;")
+        o("    uint32_t mb = 0u;")
+        o("    if (in) {")
+        o("      const int32_t k = TH.mask ? xg::gp<const int32_t>(TH.mask)[(int64_t)r * N1 + c] : 0;")
+        o("      mb = " + " | ".join(f"(k == TH.klass[{j}] ? {1 << j}u : 0u)" for j in range(m)) + ";")
+        o("    }")
+        o("    mem[i] = (uint8_t)mb;")
+        o("    ext[0][i] = in ? 0u : ~0u;")
+        o("  }")
+        o("  __syncthreads();")
+        o("  int cur = 0;")
+        o("  for (int it = 0; it < XG_WAVE_MAX_ITERS; ++it) {")
+        for j, s in enumerate(L.stmts):
+            reads = self._tb_reads[s.stmt.sid]
+            o("    for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
+            o("      uint32_t v = ext[cur][i];")
+            o(f"      if (mem[i] & {1 << j}u) {{")
+            o("        const int r = i / RW, c = i % RW;")
+            o("        (void)r; (void)c;")
+            o("        v = 0u;")
+            for d0, d1 in reads:
+                o(f"        v = xg::wave_extent(v, (r + ({d0}) >= 0 && r + ({d0}) < RH && c + ({d1}) >= 0 && "
+                  f"c + ({d1}) < RW) ? ext[cur][i + ({d0}) * RW + ({d1})] : ~0u, {d0}, {d1});")
+            o("      }")
+            o("      ext[cur ^ 1][i] = v;")
+            o("    }")
+            o("    __syncthreads();")
+            o("    cur ^= 1;")
+        o("    uint32_t most = 0u;")
+        o("    for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
+        o("      const int r = A0.start + i / RW, c = A1.start + i % RW;")
+        o("      if (r >= A0.w0 && r < A0.w1 && c >= A1.w0 && c < A1.w1)")
+        o("        for (int b = 0; b < 32; b += 8) most = max(most, (ext[cur][i] >> b) & 255u);")
+        o("    }")
+        o("    if (most > (uint32_t)it + 1u) atomicMax(&far[it], most > XG_WAVE_MAX_HALO ? 255u : most);")
+        o("  }")
+        o("  __syncthreads();")
+        o("  if (threadIdx.x < XG_WAVE_MAX_ITERS && far[threadIdx.x])")
+        o("    atomicMax((uint32_t*)TH.fail + threadIdx.x, far[threadIdx.x]);")
+        o("}")
+        # (the arguments of the loop's other launches, so the host builds them one way)
+        kargs = ["const xg_tb_hdr TH"] + [f"const xg_r{s.stmt.sid} R{j}, const xg_p{s.stmt.sid} P{j}"
+                                          for j, s in enumerate(L.stmts)]
+        o(f'extern "C" __global__ void __launch_bounds__(1024) {name}({", ".join(kargs)}) '
+          f"{{ {name}_body(TH, (int)blockIdx.x); }}")
+        o(f'extern "C" __global__ void __launch_bounds__(1024) {name}b(const xg_btent* __restrict__ E, const int32_t n, '
+          f"const int64_t total) {{ xg::for_batch_tiles(E, n, total, [&](const xg_btent& e, uint32_t t) "
+          f"{{ const xg_tb_hdr th = e.th; {name}_body(th, (int)t); __syncthreads(); }}); }}")
+
     def device_source(self, stmt_meta: list, groups: list, loops: list = ()) -> str:
         out = ["// generated by xgrid_amd for the MI355X backend", '#include "xgrid_device.h"',
                f"#define XG_OVERSTEP {OVERSTEP_CODE[self.overstep]}"]
@@ -1461,6 +1887,11 @@ class Emitter:
                            f"const xg_launch_hdr HB, const xg_r{b} RB, const xg_p{b} PB) "
                            f"{{ {body} }}")
         for L in loops:
+            if L.waves:
+                for V in L.waves:
+                    self._tb_kernel_wave(L, V, out)
+                self._tb_wave_check(L, out)
+                continue
             for V in (L, L.alt):
                 if V is not None:
                     (self._tb_kernel_reg if V.variant == "reg" else self._tb_kernel_lds)(V, out)
@@ -1764,6 +2195,10 @@ class Emitter:
     SMALL_GRID_SHAPE = (40, 64, 1024, 10, "lds")
     SMALL_GRID_MAX_CELLS = {4: 800 * 800, 8: 1300 * 1300}
 
+    # wave tiles (rows per wave, region columns, most work-items) of loops whose reads of the
+    # loop grid reach one cell
+    WAVE_TILES = ((8, 128, 1024), (4, 128, 1024))
+
     @classmethod
     def block_shape(cls, spec: str | None = None, elem: int = 8) -> tuple:
         """(core rows, region columns, work-items, most iterations per launch, variant)
@@ -1778,7 +2213,7 @@ class Emitter:
         parts = spec.split(",")
         r, c, t, m = (int(x) for x in parts[:4])
         v = parts[4].strip() if len(parts) > 4 else "lds"
-        if v not in ("lds", "reg"):
+        if v not in ("lds", "reg", "wave"):
             raise EmitError(f"unknown blocked-loop variant '{v}'")
         return r, c, t, m, v
 
@@ -1817,9 +2252,23 @@ class Emitter:
                 if L.alt is not None:
                     L.alt.batched = False
                     L.alt_max_cells = self.SMALL_GRID_MAX_CELLS[elem]
+                if reach == 1 and device_type_name(ms[0].stmt.gtype.element) in ("float", "double"):
+                    L.waves = [self._wave_tile(L, L.kernel + ("_s" if i else ""), br, cols, t)
+                               for i, (br, cols, t) in enumerate(self.WAVE_TILES)]
+                    if L.alt is not None:
+                        L.alt.waves = L.waves
             loops.append(L)
             self.used_shape = tuple(shape)
         return loops
+
+    @staticmethod
+    def _wave_tile(L: LoopMeta, name: str, rows: int, cols: int, threads: int) -> WaveTile:
+        elem = element_nbytes(L.stmts[0].stmt.gtype.element)
+        bits = 4 if rows * cols // 64 <= 32 else 8
+        # 122 / 74 registers hold the cavity's FP64 tiles of 8 / 4 rows, 86 / 55 its FP32 ones
+        waves = {8: {True: 6, False: 4}, 4: {True: 8, False: 5}}[elem][rows * cols <= 512]
+        return WaveTile(name, rows, cols // 64, threads, 2 * 2 * cols * elem + 64 * bits * len(L.stmts),
+                        max(waves, -(-threads // 256)))
 
     @staticmethod
     def _loop_meta(lid: int, node, ms: list, g: str, reach: int, shape: tuple, name: str):
@@ -1833,6 +2282,16 @@ class Emitter:
         cols = region_cols - 2 * halo
         if halo > 16 or cols < 16 or threads % 64 or threads > 1024:
             return None
+        if variant == "wave":
+            # rows: rows per wave; the plan's tile is the one a halo of 12 leaves
+            elem = device_type_name(ms[0].stmt.gtype.element)
+            if reach != 1 or elem not in ("float", "double") or rows > 32 or rows * region_cols > 4096 or region_cols % 64:
+                return None
+            L = LoopMeta(lid, node, ms, g, (rows * threads // 64 - 2 * halo, cols), halo, tmax, name, threads, reach, variant)
+            if L.core[0] < 1:
+                return None
+            L.waves = [Emitter._wave_tile(L, name, rows, region_cols, threads)]
+            return L
         if variant == "reg":
             waves = threads // 64
             if region_cols != 64 or reach < 1:
