@@ -75,6 +75,21 @@ typedef struct xg_group_desc {
   void* fn_b;                                /* batched: one workgroup per instance */
 } xg_group_desc;
 
+/* A run of consecutive statements that do not depend on each other (the reference runs
+ * them as separate nests, xgrid/lang/generator.py:369-374) and may run as one launch. */
+#define XG_FAN_SEGMENTS 8
+typedef struct xg_fan_desc {
+  int32_t first;
+  int32_t count;
+  int32_t nseg;                              /* its statements, a pair (fn_pair) being one segment */
+  int32_t seg_len[XG_FAN_SEGMENTS];          /* 1, or 2 for a pair */
+  int32_t seg_fill[XG_FAN_SEGMENTS];         /* statement whose (uniform) value a segment also stores in the
+                                                cells beside its class's rows, or -1 */
+  int32_t fill_cells;                        /* ... up to a multiple of this many columns */
+  int32_t fill_lo[3], fill_hi[3];            /* ... largest backward / forward read offset of that segment */
+  void* fn;                                  /* hipFunction_t taking (xg_fan, {hdr, refs, params} x count) */
+} xg_fan_desc;
+
 /* A `for` loop whose body is stencil statements on one 2-D grid, which may run
  * temporally blocked: `tmax` iterations per launch on core0 x core1 tiles with
  * a halo of `halo` cells kept in LDS (reference: the same statements as
@@ -184,6 +199,8 @@ void* xg_grid_level_ptr(xg_grid* g, int32_t level);
 int xg_kernel_create(int32_t nstmts, const xg_stmt_desc* stmts, int32_t ngroups,
                      const xg_group_desc* groups, int32_t nloops, const xg_loop_desc* loops,
                      int32_t ngrids, xg_kernel** out);
+/* The runs of independent statements of a kernel (none unless set). */
+int xg_kernel_set_fans(xg_kernel* k, int32_t nfans, const xg_fan_desc* fans);
 int xg_kernel_destroy(xg_kernel* k);
 /* Status of the last call made through the kernel's stub (0 or XG_ERR_*). */
 int xg_kernel_status(xg_kernel* k);

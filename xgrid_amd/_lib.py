@@ -44,6 +44,12 @@ class GroupDesc(Structure):
     _fields_ = [("first", c_int32), ("count", c_int32), ("fn", c_void_p), ("fn_b", c_void_p)]
 
 
+class FanDesc(Structure):
+    _fields_ = [("first", c_int32), ("count", c_int32), ("nseg", c_int32), ("seg_len", c_int32 * 8),
+                ("seg_fill", c_int32 * 8), ("fill_cells", c_int32), ("fill_lo", c_int32 * 3),
+                ("fill_hi", c_int32 * 3), ("fn", c_void_p)]
+
+
 XG_LOOP_MAX = 8
 
 
@@ -92,6 +98,7 @@ _SIGS = {
     "xg_grid_level_ptr": ([c_void_p, c_int32], c_void_p),
     "xg_kernel_create": ([c_int32, POINTER(StmtDesc), c_int32, POINTER(GroupDesc), c_int32, POINTER(LoopDesc),
                           c_int32, POINTER(c_void_p)], c_int),
+    "xg_kernel_set_fans": ([c_void_p, c_int32, POINTER(FanDesc)], c_int),
     "xg_kernel_destroy": ([c_void_p], c_int),
     "xg_kernel_status": ([c_void_p], c_int),
     "xg_kernel_set_options": ([c_void_p, c_int32, c_int32, c_int32], c_int),

@@ -18,7 +18,7 @@ from . import _lib
 from .analysis import analyze
 from .compilers import compile_device, compile_host, load_host
 from .config import get_config
-from .emit import Emitter, Lowered
+from .emit import Emitter, Lowered, read_reach
 from .grid import Grid
 from .types import Boolean, Floating, GridType, Integer, Pointer, Structure, Void, element_nbytes
 
@@ -139,6 +139,18 @@ class HipKernel:
             groups[i].first = g.first
             groups[i].count = g.count
             groups[i].fn = fn(g.kernel)
+        fans = (_lib.FanDesc * max(1, len(low.fans)))()
+        for i, f in enumerate(low.fans):
+            fans[i].first, fans[i].count, fans[i].nseg = f.first, f.count, len(f.segs)
+            for n, (seg, fill) in enumerate(zip(f.segs, f.fills)):
+                fans[i].seg_len[n] = len(seg)
+                fans[i].seg_fill[n] = -1 if fill is None else fill.stmt.sid
+                if fill is not None:
+                    fans[i].fill_cells = seg[0].tile3_cols // 64
+                    lo, hi = read_reach(seg[0].stmt)
+                    for a in range(3):
+                        fans[i].fill_lo[a], fans[i].fill_hi[a] = lo[a], hi[a]
+            fans[i].fn = fn(f.kernel)
         # loop plans: one per blockable loop (ids as in the stub), then the small-grid
         # tiles of those that have one
         alts = [L.alt for L in low.loops if L.alt is not None]
@@ -172,7 +184,7 @@ class HipKernel:
                 ld.alt_max_cells = L.alt_max_cells
                 nalt += 1
         self._nloops = len(low.loops) + len(alts)
-        self._descs, self._groups, self._loops = descs, groups, loops
+        self._descs, self._groups, self._loops, self._fans = descs, groups, loops, fans
         self.kernel = self.new_plan()
         self._finalizer.detach()
         self._finalizer = weakref.finalize(self, _release, self.lib, self.kernel, self._modules)
@@ -248,6 +260,7 @@ class HipKernel:
         _lib.check(self.lib.xg_kernel_create(len(low.stmts), self._descs, len(low.groups), self._groups,
                                              self._nloops, self._loops, len(low.grid_args), ctypes.byref(k)),
                    "xg_kernel_create")
+        _lib.check(self.lib.xg_kernel_set_fans(k, len(low.fans), self._fans), "xg_kernel_set_fans")
         return k.value
 
     def _param_size(self, m) -> int:

@@ -65,6 +65,15 @@ typedef struct xg_launch_hdr {
   xg_gview src;              /* pingpong source / two-phase temporary */
 } xg_launch_hdr;             /* 120 bytes */
 
+/* Independent statements in one launch: segment i (a statement, or a pair of them) has
+ * workgroups [begin[i], begin[i] + tiles[i]); begin[i] is a multiple of 8, so that a
+ * segment's tile map knows its workgroups' XCDs. */
+#define XG_FAN_MAX 8
+typedef struct xg_fan {
+  uint32_t begin[XG_FAN_MAX];
+  uint32_t tiles[XG_FAN_MAX];
+} xg_fan;                          /* 64 bytes */
+
 /* Temporally blocked loop: several iterations of a loop body of stencil
  * statements on one grid, per workgroup tile, in LDS. */
 #define XG_TB_MAX_STMTS 8

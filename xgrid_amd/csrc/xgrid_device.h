@@ -14,6 +14,8 @@
  *                   with its per-sweep malloc and copy-back, generator.py:312-352);
  *   run_phase2    - phase 2 of a two-phase statement: temporary -> store cells;
  *   run_block     - one workgroup walks a small class (chained boundary statements).
+ * Statements that do not depend on each other share a launch (a fan): each takes its own
+ * workgroups and runs as run_main, run_pair or run_fill.
  * Linear indices are row-major; for 1-D and square 2-D grids they coincide with
  * the reference's accessor (generator.py:158-182).
  *
@@ -330,9 +332,12 @@ __device__ __forceinline__ bool tile_safe(const xg_launch_hdr& H, const int32_t*
   return ok;
 }
 
-template <class S, int OV, bool MASKED, bool NT = false>
+/* FILL: the cells beside the class's rows, up to a multiple of CPL columns, take `fill` (the
+ * value another statement of the launch gives them) instead of keeping theirs. */
+template <class S, int OV, bool MASKED, bool NT = false, bool FILL = false>
 __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename S::Refs& R,
-                                          const typename S::Params& P, uint32_t tile, unsigned char* st3_lds) {
+                                          const typename S::Params& P, uint32_t tile, unsigned char* st3_lds,
+                                          const typename S::T fill = typename S::T()) {
   constexpr int D = S::D;
   typedef typename S::T T;
   typedef TileCells<D, S::CPL> TC;
@@ -401,7 +406,7 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
          * one cell to store and stores just that cell, with no read at all (FP64
          * heat 390 against 405 us); with four columns its up to three cells
          * cost more as single stores than the read (FP32 234 against 207 us). */
-        constexpr bool MERGE = MASKED || K > 2;
+        constexpr bool MERGE = !FILL && (MASKED || K > 2);
         vecn<T, K> old[NC / K];
         if (MERGE && row_fits) {
 #pragma unroll
@@ -425,17 +430,22 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
             any = any || tc.in[n + k];
           }
           if (!any) continue;
-          if (row_fits && (MERGE || all)) {
+          if (row_fits && (MERGE || FILL || all)) {
             const gptr<vecn<T, K>> dst =
                 (gptr<vecn<T, K>>)(gp<T>(H.out.ptr) + lin<3>(H.out.shape, tc.c[n][0], tc.c[n][1], col));
             vecn<T, K> w;
 #pragma unroll
-            for (int k = 0; k < K; ++k) w[k] = (!MERGE || tc.in[n + k]) ? v[n + k] : old[n / K][k];
+            for (int k = 0; k < K; ++k) {
+              if constexpr (FILL) w[k] = tc.in[n + k] ? v[n + k] : fill;
+              else w[k] = (!MERGE || tc.in[n + k]) ? v[n + k] : old[n / K][k];
+            }
             put<vecn<T, K>, NT>(dst, w);
           } else {
 #pragma unroll
-            for (int k = 0; k < K; ++k)
+            for (int k = 0; k < K; ++k) {
               if (tc.in[n + k]) store<S, OV, NT>(H, tc.c[n + k][0], tc.c[n + k][1], tc.c[n + k][2], v[n + k]);
+              else if (FILL && col + k < H.out.shape[2]) store<S, OV, NT>(H, tc.c[n][0], tc.c[n][1], col + k, fill);
+            }
           }
         }
         continue;
@@ -477,6 +487,15 @@ __device__ void run_main(const xg_launch_hdr& H, const typename S::Refs& R, cons
   } else {
     box_cells<S, OV, false>(H, R, P, tile, nullptr);
   }
+}
+
+/* Tile `tile` of a staged 3-D statement's box class, storing `fill` beside its rows. */
+template <class S, int OV>
+__device__ void run_fill(const xg_launch_hdr& H, const typename S::Refs& R, const typename S::Params& P, uint32_t tile,
+                         const typename S::T fill) {
+  __shared__ __attribute__((aligned(16))) unsigned char st3_lds[S::ST3_LDS];
+  if (H.dom.flags & XG_F_STREAM) box_cells<S, OV, false, true, true>(H, R, P, tile, st3_lds, fill);
+  else box_cells<S, OV, false, false, true>(H, R, P, tile, st3_lds, fill);
 }
 
 /* Two in-place statements over the same box in one tile walk (the runtime

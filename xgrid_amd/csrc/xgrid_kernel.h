@@ -99,6 +99,8 @@ struct Rec {
 struct xg_kernel {
   std::vector<xgi::StmtPlan> stmts;
   std::vector<xg_group_desc> groups;
+  std::vector<xg_fan_desc> fans;
+  std::vector<int32_t> fan_of;      // statement -> its fan, or -1 (empty: no fans)
   int32_t ngrids = 0;
   std::vector<xg_grid*> grids;
   int status = XG_OK;

@@ -405,6 +405,157 @@ int exec_pair(xg_kernel* k, int32_t a, const void* pa, const void* pb) {
   return do_launch(k, -1, d.fn_pair, blocks_for_dom(d.dims, H[0].dom), kThreads, args);
 }
 
+// The class of the cells beside the rows of a 3-D box class, up to a multiple of K columns
+// (kEdgeMixed: several, kEdgeNone: there are none).
+int32_t edge_class(const xg_grid* G, const ClassPlan& p, int K) {
+  int32_t& e = p.edge[K == 4];
+  if (e != kEdgeUnknown) return e;
+  const int32_t a = p.lo[2] / K * K, b = std::min<int32_t>(G->shape[2], (int32_t)ceil_div(p.hi[2], K) * K);
+  int32_t found = kEdgeNone;
+  for (int32_t i = p.lo[0]; i < p.hi[0] && found != kEdgeMixed; ++i)
+    for (int32_t j = p.lo[1]; j < p.hi[1] && found != kEdgeMixed; ++j) {
+      const int32_t* row = G->h_mask.empty() ? nullptr : G->h_mask.data() + ((int64_t)i * G->shape[1] + j) * G->shape[2];
+      for (int32_t c = a; c < b; ++c) {
+        if (c >= p.lo[2] && c < p.hi[2]) continue;
+        const int32_t v = row ? row[c] : 0;
+        if (found == kEdgeNone) found = v;
+        else if (found != v) found = kEdgeMixed;
+      }
+    }
+  return e = found;
+}
+
+// Does statement y depend on statement x of the same launch (or x read what y stores)?
+bool depends(xg_kernel* k, const StmtPlan& x, const StmtPlan& y) {
+  const xg_grid* X = k->grids[(size_t)x.d.store_arg];
+  const xg_grid* Y = k->grids[(size_t)y.d.store_arg];
+  for (int r = 0; r < y.d.nrefs; ++r)
+    if (y.d.ref_level[r] == 0 && k->grids[(size_t)y.d.ref_arg[r]] == X) return true;
+  for (int r = 0; r < x.d.nrefs; ++r)
+    if (x.d.ref_level[r] == 0 && k->grids[(size_t)x.d.ref_arg[r]] == Y) return true;
+  if (X != Y) return false;
+  auto shifted = [](const xg_stmt_desc& d) { return d.store_off[0] || d.store_off[1] || d.store_off[2]; };
+  return x.d.klass == y.d.klass || shifted(x.d) || shifted(y.d);
+}
+
+// Does every tile of a staged statement's box store the fill value beside its rows: reads inside
+// the grid (staged tiles), whole aligned lanes?
+bool fills_all(xg_kernel* k, const xg_fan_desc& f, const xg_stmt_desc& d) {
+  const xg_grid* G = k->grids[(size_t)d.store_arg];
+  const ClassPlan& p = G->plan(d.klass);
+  if (!uniform_refs(k, d) || ((uintptr_t)G->levels[0] & 15) || G->shape[2] % f.fill_cells) return false;
+  for (int a = 0; a < 3; ++a)
+    if (p.lo[a] < f.fill_lo[a] || p.hi[a] + f.fill_hi[a] > G->shape[a]) return false;
+  return d.klass == 0;
+}
+
+// The longest run of `run` from i (whole segments of one fan, in order) that may be one launch
+// on the grids bound to this call; `segs` gets its segment numbers.  0: fewer than two.
+size_t fan_run(xg_kernel* k, const std::vector<Pending>& run, size_t i, std::vector<int>& segs) {
+  segs.clear();
+  if (k->fan_of.empty()) return 0;
+  const int32_t fi = k->fan_of[(size_t)run[i].sid];
+  if (fi < 0) return 0;
+  const xg_fan_desc& f = k->fans[(size_t)fi];
+  int32_t seg = 0, at = f.first;
+  while (seg < f.nseg && at < run[i].sid) at += f.seg_len[seg++];
+  if (at != run[i].sid) return 0;   // the second statement of a pair
+  size_t j = i;
+  for (; seg < f.nseg; ++seg) {
+    const int32_t n = f.seg_len[seg];
+    if (j + (size_t)n > run.size()) break;
+    bool ok = true;
+    for (int32_t t = 0; t < n; ++t) {
+      const int32_t sid = run[j + (size_t)t].sid;
+      StmtPlan& sp = k->stmts[(size_t)sid];
+      ok = ok && sid == at + t && sid != k->timed_sid && effective_mode(k, sp) == XG_MODE_INPLACE;
+      for (size_t u = i; ok && u < j; ++u) ok = !depends(k, k->stmts[(size_t)run[u].sid], sp);
+    }
+    if (ok && n == 2) ok = pairable(k, at, at + 1);
+    if (!ok) break;
+    segs.push_back(seg);
+    j += (size_t)n;
+    at += n;
+  }
+  // a staged statement's lanes reach beside its rows: all those cells must take the fill
+  // statement's value in this launch
+  for (size_t s = 0; s < segs.size(); ++s) {
+    const int32_t fill = f.seg_fill[segs[s]];
+    if (fill < 0) continue;
+    int32_t sid = f.first;
+    for (int32_t q = 0; q < segs[s]; ++q) sid += f.seg_len[q];
+    const xg_stmt_desc& d = k->stmts[(size_t)sid].d;
+    const xg_grid* G = k->grids[(size_t)d.store_arg];
+    const ClassPlan& p = G->plan(d.klass);
+    const bool in = fill >= run[i].sid && fill < at;
+    const int32_t e = p.kind == XG_DOM_BOX ? edge_class(G, p, f.fill_cells) : kEdgeMixed;
+    if (!in || (e != kEdgeNone && e != k->stmts[(size_t)fill].d.klass)) return 0;
+  }
+  return segs.size() >= 2 ? j - i : 0;
+}
+
+int exec_fan(xg_kernel* k, const std::vector<Pending>& run, size_t i, size_t n, const std::vector<int>& segs) {
+  const xg_fan_desc& f = k->fans[(size_t)k->fan_of[(size_t)run[i].sid]];
+  static const uint8_t zeros[4096] = {0};
+  // buffers kept between calls (kernel arguments are copied at the launch)
+  thread_local std::vector<xg_launch_hdr> hdrs;
+  thread_local std::vector<std::vector<xg_gview>> refs;
+  thread_local std::vector<void*> args;
+  hdrs.resize((size_t)f.count);
+  if (refs.size() < (size_t)f.count) refs.resize((size_t)f.count);
+  xg_fan F;
+  std::memset(&F, 0, sizeof F);
+  args.clear();
+  args.push_back(&F);
+  for (int32_t q = 0; q < f.count; ++q) {
+    const int32_t sid = f.first + q;
+    const xg_stmt_desc& d = k->stmts[(size_t)sid].d;
+    xg_launch_hdr& H = hdrs[(size_t)q];
+    std::memset(&H, 0, sizeof H);
+    refs[(size_t)q].assign((size_t)std::max(1, d.nrefs), xg_gview{});
+    const void* params = zeros;
+    if (sid >= run[i].sid && sid < run[i].sid + (int32_t)n) {
+      const xg_grid* G = k->grids[(size_t)d.store_arg];
+      fill_dom(H.dom, G->plan(d.klass), G, d.klass);
+      fill_view(H.out, G, G->levels[0]);
+      H.dom.flags = (uniform_refs(k, d) ? XG_F_UNIFORM : 0) | stream_flag(G);
+      if (int rc = fill_refs(k, d, refs[(size_t)q])) return rc;
+      params = k->arena.data() + run[i + (size_t)(sid - run[i].sid)].off;
+    }
+    args.push_back(&H);
+    args.push_back(refs[(size_t)q].data());
+    args.push_back(const_cast<void*>(params));
+  }
+  // a list whose last cells another segment fills ends before them
+  for (int s : segs) {
+    const int32_t fill = f.seg_fill[s];
+    if (fill < 0) continue;
+    int32_t q = 0;
+    for (int32_t t = 0; t < s; ++t) q += f.seg_len[t];
+    const xg_stmt_desc& d = k->stmts[(size_t)fill].d;
+    xg_dom& dom = hdrs[(size_t)(fill - f.first)].dom;
+    if (dom.kind == XG_DOM_LIST && fills_all(k, f, k->stmts[(size_t)(f.first + q)].d))
+      dom.count = k->grids[(size_t)d.store_arg]->plan(d.klass).apart;
+  }
+  // workgroups of the last segment first; segments not in this run keep none (and begin where
+  // the one after them does)
+  int64_t blocks = 0;
+  for (int32_t s = f.nseg - 1; s >= 0; --s) {
+    F.begin[s] = (uint32_t)blocks;
+    if (std::find(segs.begin(), segs.end(), s) == segs.end()) continue;
+    int32_t q = 0;
+    for (int32_t t = 0; t < s; ++t) q += f.seg_len[t];
+    const xg_stmt_desc& d = k->stmts[(size_t)(f.first + q)].d;
+    const xg_dom& dom = hdrs[(size_t)q].dom;
+    const int64_t tiles = dom.kind == XG_DOM_EMPTY || dom.count == 0 ? 0 : blocks_for_dom(d.dims, dom, tile3_cols(d));
+    if (f.seg_len[s] == 2) k->n_fused += 2;
+    F.tiles[s] = (uint32_t)tiles;
+    blocks += ceil_div(tiles, 8) * 8;
+    if (blocks > 0x7fffffff) return fail(XG_ERR_ARG, "launch grid too large");
+  }
+  return do_launch(k, -1, f.fn, blocks, kThreads, args.data());
+}
+
 int flush(xg_kernel* k) {
   if (k->pending.empty()) return XG_OK;
   // the run takes the pending list's buffer and gives back its own (empty, with capacity):
@@ -431,8 +582,14 @@ int flush(xg_kernel* k) {
     const ClassPlan& p = G->plan(sp.d.klass);
     ok[i] = effective_mode(k, sp) == XG_MODE_INPLACE && p.count <= g_dev.fuse_max_cells;
   }
+  thread_local std::vector<int> segs;
   size_t i = 0;
   while (i < run.size() && rc == XG_OK) {
+    if (const size_t n = fan_run(k, run, i, segs)) {
+      rc = exec_fan(k, run, i, n, segs);
+      i += n;
+      continue;
+    }
     if (!ok[i]) {
       if (i + 1 < run.size() && !ok[i + 1] && pairable(k, run[i].sid, run[i + 1].sid)) {
         rc = exec_pair(k, run[i].sid, params_of(run[i]), params_of(run[i + 1]));
@@ -1280,8 +1437,19 @@ int xg_grid_set_mask(xg_grid* g, const int32_t* mask) {
       auto it = lists.find(mask[i]);
       if (it != lists.end()) it->second.push_back((int32_t)i);
     }
+    const ClassPlan& inner = g->plan(0);
+    const int32_t K = D == 3 && inner.kind == XG_DOM_BOX && (g->elem == 4 || g->elem == 8) ? 16 / g->elem : 0;
     for (auto& kv : lists) {
       ClassPlan& p = g->plans[kv.first];
+      p.apart = p.count;
+      if (K) {   // the cells beside the rows of class 0's box go last (each part in order)
+        const int32_t a = inner.lo[2] / K * K, b = (int32_t)ceil_div(inner.hi[2], K) * K;
+        auto apart = [&](int32_t c) {
+          const int32_t i2 = c % s2, r = c / s2, i1 = r % s1, i0 = r / s1;
+          return i0 < inner.lo[0] || i0 >= inner.hi[0] || i1 < inner.lo[1] || i1 >= inner.hi[1] || i2 < a || i2 >= b;
+        };
+        p.apart = std::stable_partition(kv.second.begin(), kv.second.end(), apart) - kv.second.begin();
+      }
       void* d = nullptr;
       if (int rc = dev_alloc(kv.second.size() * sizeof(int32_t), false, &d)) return rc;
       p.d_list = (int32_t*)d;
@@ -1370,6 +1538,29 @@ int xg_kernel_create(int32_t nstmts, const xg_stmt_desc* stmts, int32_t ngroups,
   k->exec_count.assign((size_t)nstmts, 0);
   k->last_params.assign((size_t)nstmts, std::vector<uint8_t>());
   *out = k;
+  return XG_OK;
+}
+
+int xg_kernel_set_fans(xg_kernel* k, int32_t nfans, const xg_fan_desc* fans) {
+  if (!k || nfans < 0 || (nfans > 0 && !fans)) return fail(XG_ERR_ARG, "invalid fans");
+  std::vector<int32_t> of(k->stmts.size(), -1);
+  for (int i = 0; i < nfans; ++i) {
+    const xg_fan_desc& f = fans[i];
+    bool ok = f.fn && f.first >= 0 && f.count >= 2 && f.first + f.count <= (int32_t)k->stmts.size() && f.nseg >= 2 &&
+              f.nseg <= XG_FAN_SEGMENTS && f.nseg <= XG_FAN_MAX;
+    int32_t n = 0;
+    for (int s = 0; ok && s < f.nseg; ++s) {
+      ok = (f.seg_len[s] == 1 || f.seg_len[s] == 2) &&
+           (f.seg_fill[s] < 0 || (f.seg_fill[s] >= f.first && f.seg_fill[s] < f.first + f.count &&
+                                  (f.fill_cells == 2 || f.fill_cells == 4)));
+      n += f.seg_len[s];
+    }
+    for (int q = 0; ok && q < f.count; ++q) ok = of[(size_t)(f.first + q)] < 0;
+    if (!ok || n != f.count) return fail(XG_ERR_ARG, "invalid fan description " + std::to_string(i));
+    for (int q = 0; q < f.count; ++q) of[(size_t)(f.first + q)] = i;
+  }
+  k->fans.assign(fans, fans + nfans);
+  k->fan_of = nfans ? of : std::vector<int32_t>();
   return XG_OK;
 }
 
