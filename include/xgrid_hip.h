@@ -279,10 +279,10 @@ int xg_grid_norm_diff(xg_grid* a, int32_t level_a, int32_t type_a, xg_grid* b, i
 /* No counterpart in the reference.  For callers that cannot allocate (tight
  * serving loops, harnesses that forbid hipMalloc): xg_grid_norm_diff with the
  * same arguments and results, but it allocates nothing, not even on its first
- * call.  Its partials live in a static device array of 1024 partials + 1
- * result (16,400 bytes per GPU, held until the process ends; its address is
- * looked up by xg_init).  Any class size fits: at most 1024 workgroups each
- * reduce a strided slice.  Every call on a GPU shares that GPU's array, so
+ * call.  Its partials live in a static device array of 512 partials (8,192
+ * bytes per GPU, held until the process ends; its address is looked up by
+ * xg_init) and its result in pinned host memory that xg_init allocates.  Any
+ * class size fits: at most 512 workgroups each reduce a strided slice.  Every call on a GPU shares that GPU's array, so
  * calls that overlap on one GPU (several host threads at once) race.
  * Synchronises the backend stream. */
 int xg_grid_norm_diff_noalloc(xg_grid* a, int32_t level_a, int32_t type_a, xg_grid* b, int32_t level_b,
