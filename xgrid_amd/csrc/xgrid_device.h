@@ -63,14 +63,24 @@ template <class T>
 __device__ __forceinline__ gptr<T> gp(const void* p) {
   return (gptr<T>)(p);
 }
-/* K adjacent elements read or written as one access (staged 3-D tiles: K
- * elements of 16 bytes together, only at addresses that are multiples of 16). */
+/* K adjacent elements read or written as one access at a multiple of their size. */
 template <class T, int K>
 using vecn = T __attribute__((ext_vector_type(K)));
-/* The same at any multiple of the element's size (global memory takes 16-byte
- * accesses at any multiple of 4 bytes; LDS does not). */
+/* The same at any multiple of one element's size: global memory takes 16-byte
+ * accesses at any multiple of 4 bytes (LDS does not).  The under-aligned type is a local
+ * typedef because a template argument drops its alignment. */
 template <class T, int K>
-using vecu = T __attribute__((ext_vector_type(K), aligned(sizeof(T))));
+__device__ __forceinline__ vecn<T, K> get_u(gptr<const T> p) {
+  typedef T V __attribute__((ext_vector_type(K), aligned(sizeof(T))));
+  return *(const V __attribute__((address_space(1)))*)p;
+}
+template <class T, int K, bool NT = false>
+__device__ __forceinline__ void put_u(gptr<T> p, const vecn<T, K>& v) {
+  typedef T V __attribute__((ext_vector_type(K), aligned(sizeof(T))));
+  V __attribute__((address_space(1)))* q = (V __attribute__((address_space(1)))*)p;
+  if constexpr (NT) __builtin_nontemporal_store((V)v, q);
+  else *q = (V)v;
+}
 /* The views and parameter blocks a batch table points to are written by the
  * host before the launch and only read by kernels: reading them through the
  * constant address space lets uniform reads be scalar loads into SGPRs, as
@@ -332,6 +342,17 @@ __device__ __forceinline__ bool tile_safe(const xg_launch_hdr& H, const int32_t*
   return ok;
 }
 
+/* The K values at `back` and beyond in q, the last one repeated (back >= 0). */
+template <int K, class T>
+__device__ __forceinline__ void pick(T (&q)[K], int back) {
+#pragma unroll
+  for (int s = 1; s < K; ++s)
+    if (back >= s) {
+#pragma unroll
+      for (int k = 0; k + 1 < K; ++k) q[k] = q[k + 1];
+    }
+}
+
 /* FILL: the cells beside the class's rows, up to a multiple of CPL columns, take `fill` (the
  * value another statement of the launch gives them) instead of keeping theirs. */
 template <class S, int OV, bool MASKED, bool NT = false, bool FILL = false>
@@ -356,7 +377,9 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
     }
     T v[NC];
     bool pairs = false;   /* store a lane's CPL columns with one 16-byte store */
-    if (tile_safe<S>(H, tc.tlo, tc.thi)) {
+    bool safe = tile_safe<S>(H, tc.tlo, tc.thi);
+    if constexpr (D == 3 && S::ST3) safe = safe && H.out.shape[2] >= S::CPL;
+    if (safe) {
       if constexpr (D == 3 && S::ST3) {
         /* Staged 3-D tile: each array's columns of the tile's planes are read
          * once into registers; column neighbours come over DPP lane shifts and
@@ -373,10 +396,10 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
         if (Tile<D>::CH > 1) __syncthreads();  /* the next chunk rewrites the LDS copy */
         /* In a safe tile every stored cell lies inside the grid, so with no store
          * offset and no scratch destination the store is a plain one at the cell's
-         * index, and a lane's CPL adjacent columns (16 bytes) are one store where
-         * the base is 16-byte aligned and the row pitch a multiple of CPL. */
+         * index, and a lane's CPL adjacent columns (16 bytes) are one store, at
+         * whatever alignment the row has. */
         if constexpr (S::CPL * sizeof(T) == 16 && S::SO0 == 0 && S::SO1 == 0 && S::SO2 == 0)
-          pairs = !(H.dom.flags & XG_F_TO_TMP) && ((uint64_t)H.out.ptr & 15) == 0 && (H.out.shape[2] % S::CPL) == 0;
+          pairs = !(H.dom.flags & XG_F_TO_TMP);
       } else {
 #pragma unroll
         for (int n = 0; n < NC; ++n) v[n] = S::template value<true>(R, P, H.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
@@ -418,7 +441,7 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
               any = any || tc.in[n + k];
             }
             if (any && !all)
-              old[n / K] = *(gptr<const vecn<T, K>>)(gp<T>(H.out.ptr) + lin<3>(H.out.shape, tc.c[n][0], tc.c[n][1], col));
+              old[n / K] = get_u<T, K>(gp<const T>(H.out.ptr) + lin<3>(H.out.shape, tc.c[n][0], tc.c[n][1], col));
           }
         }
 #pragma unroll
@@ -431,15 +454,14 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
           }
           if (!any) continue;
           if (row_fits && (MERGE || FILL || all)) {
-            const gptr<vecn<T, K>> dst =
-                (gptr<vecn<T, K>>)(gp<T>(H.out.ptr) + lin<3>(H.out.shape, tc.c[n][0], tc.c[n][1], col));
+            const gptr<T> dst = gp<T>(H.out.ptr) + lin<3>(H.out.shape, tc.c[n][0], tc.c[n][1], col);
             vecn<T, K> w;
 #pragma unroll
             for (int k = 0; k < K; ++k) {
               if constexpr (FILL) w[k] = tc.in[n + k] ? v[n + k] : fill;
               else w[k] = (!MERGE || tc.in[n + k]) ? v[n + k] : old[n / K][k];
             }
-            put<vecn<T, K>, NT>(dst, w);
+            put_u<T, K, NT>(dst, w);
           } else {
 #pragma unroll
             for (int k = 0; k < K; ++k) {

@@ -72,13 +72,13 @@ struct ClassPlan {
   int32_t hi[3] = {1, 1, 1};
   int32_t* d_list = nullptr;
   // The class of the cells beside a 3-D box's rows, up to a multiple of 2 or 4 columns
-  // (edge_class): kEdgeUnknown until asked for, kEdgeMixed where they differ.
+  // (edge_is): kEdgeUnknown until read from the mask, kEdgeMixed where they differ.
   mutable int32_t edge[2] = {INT32_MIN, INT32_MIN};
   // A 3-D list keeps the cells beside the rows of class 0's box (up to a multiple of 16 bytes)
   // at its end: `apart` entries come before them.
   int64_t apart = 0;
 };
-constexpr int32_t kEdgeUnknown = INT32_MIN, kEdgeMixed = INT32_MIN + 1, kEdgeNone = INT32_MIN + 2;
+constexpr int32_t kEdgeUnknown = INT32_MIN, kEdgeMixed = INT32_MIN + 1;
 
 struct xg_grid {
   int32_t dims = 1;

@@ -20,11 +20,12 @@ constexpr int64_t kFuseMaxCells = 4096;  // default of g_dev.fuse_max_cells (XGR
 // of host time against 6.3.  A small cavity is three launches and over 60 us of device time,
 // which hides either.
 constexpr int64_t kGraphMinLaunches = 3;
-// Store grids larger than the 256 MB last-level cache (Infinity Cache) take non-temporal
-// stores in 3-D box tiles: no later launch can find their cells in cache anyway.  The
-// 512^3 heat update moves the same bytes with them and runs 5-6 % faster (the write
-// stream drains faster); smaller grids keep plain stores for the next statement.
-constexpr size_t kStreamBytes = (size_t)256 << 20;
+// Store grids of which two levels do not fit the 256 MB last-level cache (Infinity Cache) take
+// non-temporal stores in 3-D box tiles: by the time the next update reads a cell it has left the
+// cache anyway, and the write stream drains faster.  The line lies where both ways meet (heat
+// update, us, plain / non-temporal): 125 MiB FP32 59 / 67, 128 MiB FP64 47 / 54, 141 MiB FP64
+// 66 / 64, 141 MiB FP32 86 / 82, 178 MiB 97 / 92, 200 MB FP64 97 / 89.
+constexpr size_t kStreamBytes = (size_t)128 << 20;
 // Freed grid memory the device pool keeps for reuse (beyond it, memory goes back at
 // the next synchronisation).
 constexpr uint64_t kPoolKeepBytes = (uint64_t)16 << 30;

@@ -405,24 +405,30 @@ int exec_pair(xg_kernel* k, int32_t a, const void* pa, const void* pb) {
   return do_launch(k, -1, d.fn_pair, blocks_for_dom(d.dims, H[0].dom), kThreads, args);
 }
 
-// The class of the cells beside the rows of a 3-D box class, up to a multiple of K columns
-// (kEdgeMixed: several, kEdgeNone: there are none).
-int32_t edge_class(const xg_grid* G, const ClassPlan& p, int K) {
-  int32_t& e = p.edge[K == 4];
-  if (e != kEdgeUnknown) return e;
+// Are the cells beside the rows of class 0's 3-D box, up to a multiple of K columns, all of
+// class `klass`?  The mask's plan knows how many of a list's cells are there.  Where the wall is
+// no list (small grids, thick walls) the mask is read, once; over many rows that costs more than
+// the launch it saves (262,144 cold rows of a 512^3 mask: 50 ms).
+constexpr int64_t kEdgeRows = 4096;
+bool edge_is(const xg_grid* G, const ClassPlan& p, int K, int32_t klass) {
   const int32_t a = p.lo[2] / K * K, b = std::min<int32_t>(G->shape[2], (int32_t)ceil_div(p.hi[2], K) * K);
-  int32_t found = kEdgeNone;
-  for (int32_t i = p.lo[0]; i < p.hi[0] && found != kEdgeMixed; ++i)
-    for (int32_t j = p.lo[1]; j < p.hi[1] && found != kEdgeMixed; ++j) {
-      const int32_t* row = G->h_mask.empty() ? nullptr : G->h_mask.data() + ((int64_t)i * G->shape[1] + j) * G->shape[2];
-      for (int32_t c = a; c < b; ++c) {
-        if (c >= p.lo[2] && c < p.hi[2]) continue;
-        const int32_t v = row ? row[c] : 0;
-        if (found == kEdgeNone) found = v;
-        else if (found != v) found = kEdgeMixed;
-      }
-    }
-  return e = found;
+  const int64_t rows = (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
+  const int64_t cells = rows * ((p.lo[2] - a) + (b - p.hi[2]));
+  if (cells == 0) return true;
+  const ClassPlan& w = G->plan(klass);
+  if (w.kind == XG_DOM_LIST) return w.count - w.apart == cells;
+  if (rows > kEdgeRows || G->h_mask.empty()) return false;
+  int32_t& e = p.edge[K == 4];
+  if (e == kEdgeUnknown) {
+    const int32_t* m = G->h_mask.data();
+    auto at = [&](int32_t i, int32_t j) { return m + ((int64_t)i * G->shape[1] + j) * G->shape[2]; };
+    e = at(p.lo[0], p.lo[1])[a < p.lo[2] ? a : p.hi[2]];
+    for (int32_t i = p.lo[0]; i < p.hi[0] && e != kEdgeMixed; ++i)
+      for (int32_t j = p.lo[1]; j < p.hi[1] && e != kEdgeMixed; ++j)
+        for (int32_t c = a; c < b; ++c)
+          if ((c < p.lo[2] || c >= p.hi[2]) && at(i, j)[c] != e) e = kEdgeMixed;
+  }
+  return e == klass;
 }
 
 // Does statement y depend on statement x of the same launch (or x read what y stores)?
@@ -438,12 +444,12 @@ bool depends(xg_kernel* k, const StmtPlan& x, const StmtPlan& y) {
   return x.d.klass == y.d.klass || shifted(x.d) || shifted(y.d);
 }
 
-// Does every tile of a staged statement's box store the fill value beside its rows: reads inside
-// the grid (staged tiles), whole aligned lanes?
+// Does every tile of a staged statement's box store the fill value beside its rows: is every
+// tile staged (box_cells)?
 bool fills_all(xg_kernel* k, const xg_fan_desc& f, const xg_stmt_desc& d) {
   const xg_grid* G = k->grids[(size_t)d.store_arg];
   const ClassPlan& p = G->plan(d.klass);
-  if (!uniform_refs(k, d) || ((uintptr_t)G->levels[0] & 15) || G->shape[2] % f.fill_cells) return false;
+  if (!uniform_refs(k, d) || G->shape[2] < f.fill_cells) return false;
   for (int a = 0; a < 3; ++a)
     if (p.lo[a] < f.fill_lo[a] || p.hi[a] + f.fill_hi[a] > G->shape[a]) return false;
   return d.klass == 0;
@@ -488,8 +494,8 @@ size_t fan_run(xg_kernel* k, const std::vector<Pending>& run, size_t i, std::vec
     const xg_grid* G = k->grids[(size_t)d.store_arg];
     const ClassPlan& p = G->plan(d.klass);
     const bool in = fill >= run[i].sid && fill < at;
-    const int32_t e = p.kind == XG_DOM_BOX ? edge_class(G, p, f.fill_cells) : kEdgeMixed;
-    if (!in || (e != kEdgeNone && e != k->stmts[(size_t)fill].d.klass)) return 0;
+    if (!in || d.klass != 0 || p.kind != XG_DOM_BOX || !edge_is(G, p, f.fill_cells, k->stmts[(size_t)fill].d.klass))
+      return 0;
   }
   return segs.size() >= 2 ? j - i : 0;
 }

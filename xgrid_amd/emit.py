@@ -473,9 +473,7 @@ class _St3Plan:
     A lane holds 16 bytes of each row (CPL = 2 columns of 8-byte elements, 4 of
     4-byte ones), so a wave reads 1 KB of a row at a time: the 512^3 FP64 7-point
     update measured 376 us against 534 us with one column per lane in a probe.
-    Where a tile lies inside the row and the array is 16-byte aligned with a row
-    pitch that is a multiple of CPL, a lane's columns are one 16-byte load;
-    otherwise one element at a time.  XGRID_STAGE3_COLS=1 selects one column per
+    A lane's columns are one 16-byte load at any alignment.  XGRID_STAGE3_COLS=1 selects one column per
     lane, XGRID_STAGE3_F32=0 leaves 4-byte arrays unstaged."""
 
     NP, ROWS = 4, 4
@@ -579,10 +577,14 @@ class _St3Plan:
         out.append(f"  struct St3 {{ {' '.join(fields)} }};")
         out.append("  __device__ static __forceinline__ void st3_load(St3& st, unsigned char* lds, const Refs& R, "
                    "const int32_t* sh, int p0, int r0, int c0) {")
-        # In a tile whose columns all lie inside the row (`full`: every tile but a
-        # partial last one) a lane's columns need no clamp; where their address is a
-        # multiple of 16 bytes they are read as one 16-byte load.  (Marking the wave's
-        # row uniform with readfirstlane made the FP64 heat kernel spill.)
+        # A lane's columns are one 16-byte load at whatever alignment the row has (read
+        # element by element, as two loads per lane in FP64 and four in FP32, odd pitches took
+        # 409 us at 400x400x399 FP64 and 238 us at 400x400x401 FP32 for the heat update; 244 and
+        # 128 us so).  In a tile whose columns
+        # all lie inside the row (`full`: every tile but a partial last one) they need no
+        # clamp; elsewhere the load is moved back into the row and the columns picked from
+        # it (a staged tile's rows hold at least K cells: box_cells).  (Marking the
+        # wave's row uniform with readfirstlane made the FP64 heat kernel spill.)
         # 8-byte tiles load at a raised wave priority, so a wave that starts its
         # tile issues its loads ahead of other waves' arithmetic (512^3 FP64
         # update 385.3-385.6 against 389.4-390.4 us; FP32 slower, 205-207 against 204)
@@ -595,32 +597,30 @@ class _St3Plan:
         out.append("    const int64_t row = min(r0 + wr, sh[1] - 1);")
         out.append(f"    const int cl = c0 + lane * {K};")
         out.append(f"    const bool full = c0 + {C} <= sh[2];")
-        out.append("    (void)lds; (void)P1; (void)P0; (void)cl; (void)full;")
+        out.append(f"    const int cb = min(cl, sh[2] - {K}), back = cl - cb;")
+        out.append("    (void)lds; (void)P1; (void)P0; (void)cl; (void)full; (void)cb; (void)back;")
         for j in sorted(self.planes):
             t = self.types[j]
             out.append(f"    const xg::gptr<const {t}> g{j} = xg::gp<const {t}>(R.v[{j}].ptr);")
             if K * self._size(j) == 16:
-                # a lane's columns at a 16-byte aligned address: a 16-byte aligned base,
-                # a row pitch that is a multiple of K (then every plane pitch is) and
-                # column multiples of K
-                out.append(f"    if (full && ((uint64_t)R.v[{j}].ptr & 15) == 0 && (P1 % {K}) == 0) {{")
                 out.append("#pragma unroll")
-                out.append(f"      for (int u = 0; u < {self.window(j)}; ++u) {{")
-                out.append(f"        const xg::gptr<const {t}> rp = g{j} + (xg::st3_plane(p0 + u + {self.pmin(j)}, sh) * P0 + row * P1);")
-                out.append(f"        const xg::vecn<{t}, {K}> v = *(xg::gptr<const xg::vecn<{t}, {K}>>)(rp + cl);")
+                out.append(f"    for (int u = 0; u < {self.window(j)}; ++u) {{")
+                out.append(f"      const xg::gptr<const {t}> rp = g{j} + (xg::st3_plane(p0 + u + {self.pmin(j)}, sh) * P0 + row * P1);")
+                out.append(f"      const xg::vecn<{t}, {K}> v = xg::get_u<{t}, {K}>(rp + cb);")
                 out.append("#pragma unroll")
-                out.append(f"        for (int k = 0; k < {K}; ++k) st.q{j}[u][k] = v[k];")
-                out.append("      }")
-                out.append("    } else {")
+                out.append(f"      for (int k = 0; k < {K}; ++k) st.q{j}[u][k] = v[k];")
+                out.append("    }")
+                out.append("    if (!full) {")
+                out.append("#pragma unroll")
+                out.append(f"      for (int u = 0; u < {self.window(j)}; ++u) xg::pick<{K}>(st.q{j}[u], back);")
+                out.append("    }")
             else:
-                out.append("    {")
-            out.append("#pragma unroll")
-            out.append(f"      for (int u = 0; u < {self.window(j)}; ++u) {{")
-            out.append(f"        const xg::gptr<const {t}> rp = g{j} + (xg::st3_plane(p0 + u + {self.pmin(j)}, sh) * P0 + row * P1);")
-            out.append("#pragma unroll")
-            out.append(f"        for (int k = 0; k < {K}; ++k) st.q{j}[u][k] = rp[min(cl + k, sh[2] - 1)];")
-            out.append("      }")
-            out.append("    }")
+                out.append("#pragma unroll")
+                out.append(f"    for (int u = 0; u < {self.window(j)}; ++u) {{")
+                out.append(f"      const xg::gptr<const {t}> rp = g{j} + (xg::st3_plane(p0 + u + {self.pmin(j)}, sh) * P0 + row * P1);")
+                out.append("#pragma unroll")
+                out.append(f"      for (int k = 0; k < {K}; ++k) st.q{j}[u][k] = rp[min(cl + k, sh[2] - 1)];")
+                out.append("    }")
         if self.xg:
             out.append("    const bool edge = lane == 0 || lane == 63;")
             out.append(f"    const int64_t ecol = lane == 0 ? max(c0 - 1, 0) : min(c0 + {C}, sh[2] - 1);")
@@ -643,9 +643,9 @@ class _St3Plan:
                        f"st.q{j}[n + {o0 - self.pmin(j)}][k];")
             # the halo rows above and below the tile: 2 x NP rows of C columns over 256 work-items
             if K * self._size(j) == 16:
-                # K columns per work-item, one 16-byte load, where aligned as above,
-                # straight into LDS: a wave loads one halo row (64 lanes x 16 bytes =
-                # C columns), so its LDS row is the same for the whole wave
+                # K columns per work-item, one 16-byte load, a wave per halo row (64 lanes
+                # x 16 bytes = C columns); where aligned (a 16-byte aligned base, a row
+                # pitch that is a multiple of K) straight into LDS, else through registers
                 out.append(f"      if (full && ((uint64_t)R.v[{j}].ptr & 15) == 0 && (P1 % {K}) == 0) {{")
                 out.append("#pragma unroll")
                 out.append(f"        for (int h = 0; h < {2 * NP * 64 // 256}; ++h) {{")
@@ -657,17 +657,35 @@ class _St3Plan:
                 out.append("        }")
                 lds_dma = True
                 out.append("      } else {")
+                nh = 2 * NP * 64 // 256
+                out.append(f"        xg::vecn<{t}, {K}> hv[{nh}];")
+                out.append("#pragma unroll")
+                out.append(f"        for (int h = 0; h < {nh}; ++h) {{")
+                out.append(f"          const int e = wr * 64 + h * 256, pl = (e / 64) % {NP}, hr = e / {64 * NP};")
+                out.append(f"          const int64_t gr = min(max(hr ? r0 + {self.ROWS} : r0 - 1, 0), sh[1] - 1);")
+                out.append(f"          hv[h] = xg::get_u<{t}, {K}>"
+                           f"(g{j} + (xg::st3_plane(p0 + pl + {o0}, sh) * P0 + gr * P1 + cb));")
+                out.append("        }")
+                out.append("#pragma unroll")
+                out.append(f"        for (int h = 0; h < {nh}; ++h) {{")
+                out.append(f"          const int e = wr * 64 + h * 256, pl = (e / 64) % {NP}, hr = e / {64 * NP};")
+                out.append(f"          {t} w[{K}];")
+                out.append("#pragma unroll")
+                out.append(f"          for (int k = 0; k < {K}; ++k) w[k] = hv[h][k];")
+                out.append(f"          if (!full) xg::pick<{K}>(w, back);")
+                out.append("#pragma unroll")
+                out.append(f"          for (int k = 0; k < {K}; ++k) L[(pl * {R2} + (hr ? {R2 - 1} : 0)) * {C} + lane * {K} + k] = w[k];")
+                out.append("        }")
+                out.append("      }")
             else:
-                out.append("      {")
-            out.append("#pragma unroll")
-            out.append(f"      for (int h = 0; h < {2 * NP * C // 256}; ++h) {{")
-            out.append(f"        const int e = threadIdx.x + h * 256, cc = e % {C}, pl = (e / {C}) % {NP}, "
-                       f"hr = e / {C * NP};")
-            out.append(f"        const int64_t gr = min(max(hr ? r0 + {self.ROWS} : r0 - 1, 0), sh[1] - 1);")
-            out.append(f"        L[(pl * {R2} + (hr ? {R2 - 1} : 0)) * {C} + cc] = "
-                       f"g{j}[xg::st3_plane(p0 + pl + {o0}, sh) * P0 + gr * P1 + min(c0 + cc, sh[2] - 1)];")
-            out.append("      }")
-            out.append("      }")
+                out.append("#pragma unroll")
+                out.append(f"      for (int h = 0; h < {2 * NP * C // 256}; ++h) {{")
+                out.append(f"        const int e = threadIdx.x + h * 256, cc = e % {C}, pl = (e / {C}) % {NP}, "
+                           f"hr = e / {C * NP};")
+                out.append(f"        const int64_t gr = min(max(hr ? r0 + {self.ROWS} : r0 - 1, 0), sh[1] - 1);")
+                out.append(f"        L[(pl * {R2} + (hr ? {R2 - 1} : 0)) * {C} + cc] = "
+                           f"g{j}[xg::st3_plane(p0 + pl + {o0}, sh) * P0 + gr * P1 + min(c0 + cc, sh[2] - 1)];")
+                out.append("      }")
             out.append("    }")
             off += NP * R2 * C * self._size(j)
         if lds_dma:
@@ -990,7 +1008,7 @@ class Emitter:
                 r = refs.index((g, lvl))
                 o3 = [str(offs[d]) if d < gts[g].dimension else "0" for d in range(3)]
                 if gts[g].dimension == D and et in ("float", "double"):
-                    out.append(f"      {{ const xg::vecu<{et}, K> w = *(xg::gptr<const xg::vecu<{et}, K>>)"
+                    out.append(f"      {{ const xg::vecn<{et}, K> w = xg::get_u<{et}, K>"
                                f"(xg::gp<const {et}>(R.v[{r}].ptr) + xc + xg::off<{D}>(sh, {', '.join(o3)}));")
                     out.append("#pragma unroll")
                     out.append(f"        for (int k = 0; k < K; ++k) pre[k].v{i} = w[k]; }}")
@@ -1571,7 +1589,7 @@ class Emitter:
         o("  if (full) {")
         o("#pragma unroll")
         o("    for (int q = 0; q < BR; ++q) {")
-        o("      const xg::vecu<T, K> x = *(xg::gptr<const xg::vecu<T, K>>)(src + ((int64_t)(gr + q) * N1 + gc));")
+        o("      const xg::vecn<T, K> x = xg::get_u<T, K>(src + ((int64_t)(gr + q) * N1 + gc));")
         o("#pragma unroll")
         o("      for (int k = 0; k < K; ++k) V[q][k] = x[k];")
         o("    }")
@@ -1777,10 +1795,10 @@ class Emitter:
         o("    if (row < A0.w0 || row >= A0.w1) continue;")
         o("    const xg::gptr<T> p = dst + ((int64_t)row * N1 + gc);")
         o("    if (gc >= A1.w0 && gc + K <= A1.w1) {")
-        o("      xg::vecu<T, K> x;")
+        o("      xg::vecn<T, K> x;")
         o("#pragma unroll")
         o("      for (int k = 0; k < K; ++k) x[k] = V[q][k];")
-        o("      *(xg::gptr<xg::vecu<T, K>>)p = x;")
+        o("      xg::put_u<T, K>(p, x);")
         o("    } else {")
         o("#pragma unroll")
         o("      for (int k = 0; k < K; ++k)")
