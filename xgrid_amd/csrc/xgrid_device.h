@@ -815,19 +815,20 @@ struct wave_axis {
   }
 };
 
-/* Extents (cells to the left, right, above and below, a byte each) of a value that
- * depends on what `v` says and on the cell (d0, d1) away, whose own extents are `x`;
- * 255 stays 255. */
-__device__ __forceinline__ uint32_t wave_extent(uint32_t v, uint32_t x, int d0, int d1) {
-  const int d[4] = {-d1, d1, -d0, d0};
-  uint32_t r = 0u;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int e = (int)((x >> (8 * b)) & 255u), o = (int)((v >> (8 * b)) & 255u);
-    r |= (uint32_t)max(o, e == 255 ? 255 : min(max(e + d[b], 0), 254)) << (8 * b);
+/* How far the initial values that a cell's value depends on lie to its left, right, above and
+ * below (16 bits each; adding a cell per statement to `unknown` stays far from their end). */
+struct wave_ext {
+  typedef short two __attribute__((ext_vector_type(2)));
+  two h, v;
+  __device__ static __forceinline__ wave_ext none() { return {two{0, 0}, two{0, 0}}; }
+  __device__ static __forceinline__ wave_ext unknown() { return {two{0x4000, 0x4000}, two{0x4000, 0x4000}}; }
+  /* this cell's value also depends on that of the cell (d0, d1) away, whose distances are x */
+  __device__ __forceinline__ void reads(const wave_ext& x, short d0, short d1) {
+    h = __builtin_elementwise_max(h, (two)(x.h + two{(short)-d1, d1}));
+    v = __builtin_elementwise_max(v, (two)(x.v + two{(short)-d0, d0}));
   }
-  return r;
-}
+  __device__ __forceinline__ int most() const { return max(max(h[0], h[1]), max(v[0], v[1])); }
+};
 
 /* ---- batched launches ---------------------------------------------------
  * Global tile g of a batched launch belongs to the entry whose range

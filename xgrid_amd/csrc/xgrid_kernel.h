@@ -83,6 +83,12 @@ struct LoopPlan : LoopProof {
   xg_loop_desc d;
   std::vector<LoopProof> others;   // other masks' proofs, most recent first
   WaveCut cut;                     // wave tiles: the cut of the launches being made
+  // wave tiles: the cut last chosen for one grid, and what it was chosen for (choosing takes the
+  // host 13 us, as long as two launches)
+  WaveCut chosen;
+  int32_t chosen_n0 = 0, chosen_n1 = 0;
+  int64_t chosen_trip = 0;
+  uint8_t chosen_reach[XG_WAVE_MAX_ITERS] = {};
   int64_t launches = 0, iterations = 0;
   std::vector<std::vector<uint8_t>> last_params;
 };

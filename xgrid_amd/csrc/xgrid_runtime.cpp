@@ -734,6 +734,21 @@ WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes,
   return best;
 }
 
+// The cut for one grid (waves = 0: none), chosen again only if something it depends on changed.
+static void wave_cut_plain(LoopPlan& L, const xg_grid* G, int64_t trip) {
+  if (L.chosen_trip != trip || L.chosen_n0 != G->shape[0] || L.chosen_n1 != G->shape[1] ||
+      std::memcmp(L.chosen_reach, L.reach, sizeof L.reach) != 0) {
+    const WaveShape s = wave_shape(G, L);
+    L.chosen = wave_choose(L.d, {s}, trip);
+    if (L.chosen.waves) L.chosen = wave_cut_for(L.d, L.chosen, s);
+    L.chosen_trip = trip;
+    L.chosen_n0 = s.n0;
+    L.chosen_n1 = s.n1;
+    std::memcpy(L.chosen_reach, L.reach, sizeof L.reach);
+  }
+  L.cut = L.chosen;
+}
+
 void fill_wave_check(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int32_t* answer) {
   fill_tb_hdr(k, L, TH, XG_WAVE_MAX_ITERS, answer);
   const xg_grid* G = k->grids[(size_t)L.d.grid_arg];
@@ -1121,9 +1136,8 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
       L.state = -1;
       return 0;
     }
-    L.cut = wave_choose(L.d, {wave_shape(G, L)}, trip);
+    wave_cut_plain(L, G, trip);
     if (L.cut.waves == 0) return 0;
-    L.cut = wave_cut_for(L.d, L.cut, wave_shape(G, L));
   }
   if ((rc = run_blocked(k, L, G, params, trip - done))) {
     set_status(k, rc);
@@ -1624,7 +1638,7 @@ int xg_kernel_time_loop(xg_kernel* k, int32_t lid, int32_t trip, int32_t reps, d
   for (auto& p : L.last_params) ps.push_back(p.data());
   // one trip = the launches a call makes for `trip` iterations
   auto run_trip = [&]() -> int {
-    if (L.d.nwave) L.cut = wave_cut_for(L.d, wave_choose(L.d, {wave_shape(G, L)}, trip), wave_shape(G, L));
+    if (L.d.nwave) wave_cut_plain(L, G, trip);
     return run_blocked(k, L, G, ps.data(), trip);
   };
   hipEvent_t e0, e1;

@@ -1834,15 +1834,22 @@ class Emitter:
         or the distance passes XG_WAVE_MAX_HALO.  Followed statement by statement; only
         the mask decides, no field value is read, and it runs once per mask.  Inside the
         box of class 0, where at most one statement runs, the distance is the number of
-        iterations (which the host takes as the least) and is not followed."""
+        iterations (which the host takes as the least) and is not followed.
+
+        The workgroup's integer work bounds it; a work-item keeps its cells' distances in
+        registers and each statement touches its members only.  (Distances of a byte in two LDS
+        copies, every read tested against the region: 237 us for a 65^2 cavity sweep's mask,
+        102 us so.)"""
         o = out.append
         m = len(L.stmts)
         name = L.wave_check
         o(f"__device__ __forceinline__ void {name}_body(const xg_tb_hdr& TH, const int tile) {{")
-        o("  constexpr int RH = XG_WAVE_CHECK_ROWS, RW = XG_WAVE_CHECK_COLS, NR = RH * RW;")
-        # extents of a cell: a byte each for left, right, above, below; 255: unknown
-        o("  __shared__ uint8_t mem[NR];")
-        o("  __shared__ uint32_t ext[2][NR];")
+        # a work-item keeps NC cells of one column, RS rows apart; the copy in LDS has a border
+        # of cells that are never known, so a read needs no test
+        o("  constexpr int RH = XG_WAVE_CHECK_ROWS, RW = XG_WAVE_CHECK_COLS, PW = RW + 2;")
+        o("  constexpr int RS = 1024 / RW, NC = RH / RS;")
+        o("  static_assert(RS * RW == 1024 && NC * RS == RH && NC <= 32, \"1024 work-items hold the region\");")
+        o("  __shared__ xg::wave_ext ext[(RH + 2) * PW];")
         o("  __shared__ uint32_t far[XG_WAVE_MAX_ITERS];")
         o("  if (threadIdx.x < XG_WAVE_MAX_ITERS) far[threadIdx.x] = 0u;")
         o("  const int N0 = TH.src.shape[0], N1 = TH.src.shape[1];")
@@ -1851,43 +1858,57 @@ class Emitter:
         if sum(s.stmt.klass == 0 for s in L.stmts) <= 1:
             o("  if (A0.start >= TH.blo[0] && A0.start + RH <= TH.bhi[0] && A1.start >= TH.blo[1] && "
               "A1.start + RW <= TH.bhi[1]) return;")
-        o("  for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
-        o("    const int r = A0.start + i / RW, c = A1.start + i % RW;")
-        o("    const bool in = r < N0 && c < N1;")
-        o("    uint32_t mb = 0u;")
-        o("    if (in) {")
-        o("      const int32_t k = TH.mask ? xg::gp<const int32_t>(TH.mask)[(int64_t)r * N1 + c] : 0;")
-        o("      mb = " + " | ".join(f"(k == TH.klass[{j}] ? {1 << j}u : 0u)" for j in range(m)) + ";")
-        o("    }")
-        o("    mem[i] = (uint8_t)mb;")
-        o("    ext[0][i] = in ? 0u : ~0u;")
+        o("  for (int i = threadIdx.x; i < (RH + 2) * PW; i += 1024) ext[i] = xg::wave_ext::unknown();")
+        o("  const int tr = threadIdx.x / RW, tc = threadIdx.x % RW, col = A1.start + tc;")
+        o("  xg::wave_ext* const mine = ext + (tr + 1) * PW + tc + 1;")
+        o("  xg::wave_ext own[NC];")
+        o(f"  uint32_t win = 0u, in = 0u, mem[{m}] = {{}};   // bit k: cell k")
+        o("#pragma unroll")
+        o("  for (int k = 0; k < NC; ++k) {")
+        o("    const int r = A0.start + tr + k * RS;")
+        o("    own[k] = xg::wave_ext::unknown();")
+        o("    if (r >= N0 || col >= N1) continue;")
+        o("    const int32_t kl = TH.mask ? xg::gp<const int32_t>(TH.mask)[(int64_t)r * N1 + col] : 0;")
+        for j in range(m):
+            o(f"    mem[{j}] |= (kl == TH.klass[{j}] ? 1u : 0u) << k;")
+        o("    in |= 1u << k;")
+        o("    if (r >= A0.w0 && r < A0.w1 && col >= A1.w0 && col < A1.w1) win |= 1u << k;")
+        o("    own[k] = xg::wave_ext::none();")
         o("  }")
         o("  __syncthreads();")
-        o("  int cur = 0;")
+        o("#pragma unroll")
+        o("  for (int k = 0; k < NC; ++k)")
+        o("    if (in >> k & 1u) mine[k * RS * PW] = own[k];")
+        o("  __syncthreads();")
         o("  for (int it = 0; it < XG_WAVE_MAX_ITERS; ++it) {")
+        # (bits tested where they are used, not kept as lane masks over the iterations: those spill)
+        o("    " + " ".join(f'asm volatile("" : "+v"(mem[{j}]));' for j in range(m)) + ' asm volatile("" : "+v"(win));')
         for j, s in enumerate(L.stmts):
             reads = self._tb_reads[s.stmt.sid]
-            o("    for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
-            o("      uint32_t v = ext[cur][i];")
-            o(f"      if (mem[i] & {1 << j}u) {{")
-            o("        const int r = i / RW, c = i % RW;")
-            o("        (void)r; (void)c;")
-            o("        v = 0u;")
+            assert all(abs(d0) <= 1 and abs(d1) <= 1 for d0, d1 in reads)
+            o(f"    if (mem[{j}]) {{")
+            o("#pragma unroll")
+            o("      for (int k = 0; k < NC; ++k)")
+            o(f"        if (mem[{j}] >> k & 1u) {{")
+            o("          xg::wave_ext v = xg::wave_ext::none();")
             for d0, d1 in reads:
-                o(f"        v = xg::wave_extent(v, (r + ({d0}) >= 0 && r + ({d0}) < RH && c + ({d1}) >= 0 && "
-                  f"c + ({d1}) < RW) ? ext[cur][i + ({d0}) * RW + ({d1})] : ~0u, {d0}, {d1});")
-            o("      }")
-            o("      ext[cur ^ 1][i] = v;")
+                o(f"          v.reads(mine[(k * RS + ({d0})) * PW + ({d1})], {d0}, {d1});")
+            o("          own[k] = v;")
+            o("        }")
             o("    }")
             o("    __syncthreads();")
-            o("    cur ^= 1;")
-        o("    uint32_t most = 0u;")
-        o("    for (int i = threadIdx.x; i < NR; i += blockDim.x) {")
-        o("      const int r = A0.start + i / RW, c = A1.start + i % RW;")
-        o("      if (r >= A0.w0 && r < A0.w1 && c >= A1.w0 && c < A1.w1)")
-        o("        for (int b = 0; b < 32; b += 8) most = max(most, (ext[cur][i] >> b) & 255u);")
-        o("    }")
-        o("    if (most > (uint32_t)it + 1u) atomicMax(&far[it], most > XG_WAVE_MAX_HALO ? 255u : most);")
+            o(f"    if (mem[{j}]) {{")
+            o("#pragma unroll")
+            o("      for (int k = 0; k < NC; ++k)")
+            o(f"        if (mem[{j}] >> k & 1u) mine[k * RS * PW] = own[k];")
+            o("    }")
+            o("    __syncthreads();")
+        o("    xg::wave_ext top = xg::wave_ext::none();")
+        o("#pragma unroll")
+        o("    for (int k = 0; k < NC; ++k)")
+        o("      if (win >> k & 1u) top.reads(own[k], 0, 0);")
+        o("    const int most = top.most();")
+        o("    if (most > it + 1) atomicMax(&far[it], most > XG_WAVE_MAX_HALO ? 255u : (uint32_t)most);")
         o("  }")
         o("  __syncthreads();")
         o("  if (threadIdx.x < XG_WAVE_MAX_ITERS && far[threadIdx.x])")
