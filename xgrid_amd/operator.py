@@ -20,7 +20,6 @@ from .types import BaseType
 # (this thread-local one), never into Operator._ir: what the first call parses is
 # decided then, under the configuration and globals in force at that time.
 _private = threading.local()
-_Grid = None                     # xgrid_amd.grid.Grid, imported on the first kernel call
 _ir_lock = threading.RLock()     # a parse parses the operators it calls
 
 CustomTypecheck = Callable[[list], BaseType]
@@ -52,19 +51,13 @@ class Operator:
 
     def __call__(self, *args: Any) -> Any:
         if self.mode == "kernel":
-            global _Grid
             if self.native is None:
                 from .backend import build_kernel
                 if self._precompiled is not None:
                     self._precompiled.wait()      # its code objects are then in the cache
                 self.native, self.depth = build_kernel(self)
-            if _Grid is None:
-                from .grid import Grid as _Grid
-            depth, tick = self.depth, self.tick
-            for arg in args:
-                if isinstance(arg, _Grid):
-                    arg._op_invoke(depth, tick)
-            return self.native(*args)
+            native = self.native
+            return native.call(native, args, self.depth, self.tick)
         if self.mode == "function":
             return self.func(*args)
         raise RuntimeError(f"Invalid call to non-kernel or non-function ({self.mode}) operator '{self.name}'")
