@@ -228,6 +228,7 @@ class _ExprC:
         # device statements: divisor texts of the per-cell divisions by a launch-uniform
         # value, which are emitted as xg::udiv<DV> (see _uniform_division)
         self.udivs = udivs
+        self.quot = False             # emit them as q.div<number> instead (xg::Quot)
         self.hoisted = hoisted or {}  # id(node) -> text of its host-computed value
         self.fold_pow = fold_pow      # host text with the device's pow folds (hoisted values)
 
@@ -273,6 +274,8 @@ class _ExprC:
             d = self(e.right)
             if d not in self.udivs:
                 self.udivs.append(d)
+            if self.quot:
+                return f"q.template div<{self.udivs.index(d)}>({self(e.left)}, {d})"
             return f"xg::udiv<DV>({self(e.left)}, {d})"
         return f"({self(e.left)} {e.op} {self(e.right)})"
 
@@ -747,6 +750,7 @@ class Emitter:
         self.functions = []            # user operators reachable from the kernel (dependency order)
         self.device_functions = []     # those reachable from stencil expressions
         self._prefetched = set()       # blocked-loop statements whose other-grid loads are prefetched
+        self._quot = set()             # ... that have a form with corrected quotients (xg::Quot)
         self._tb_reads = {}            # blocked-loop statement -> its loop-grid read offsets, in slot order
         self._fan_list = []            # FanMeta of the kernel (device_source)
         self._st3_waves = {}           # staged statement -> launch attribute of its kernels
@@ -885,7 +889,7 @@ class Emitter:
             st3[0] = plan3
             expr_st3 = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
             st3[0] = None
-        expr_tb = expr_pre = expr_lds = expr_lds_pre = None
+        expr_tb = expr_pre = expr_quot = expr_lds = expr_lds_pre = None
         if tb is not None:
             in_reg[0] = True
             expr_tb = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
@@ -897,6 +901,10 @@ class Emitter:
                 pre_mode[0] = True
                 in_reg[0] = True
                 expr_pre = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
+                if udivs:
+                    x = _ExprC(True, cell, name, grid_info, udivs, hoisted)
+                    x.quot = True
+                    expr_quot = x(st.node.value)
                 in_reg[0] = False
                 in_lds[0] = True
                 expr_lds_pre = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
@@ -1023,6 +1031,21 @@ class Emitter:
             out.append("    (void)s; (void)R; (void)P; (void)pre;")
             out.append(f"    return {expr_pre};")
             out.append("  }")
+            if expr_quot is not None:
+                out.append(f"  typedef xg::Divisors<{len(udivs)}> Divs; typedef xg::Quot<{len(udivs)}> Quot;")
+                out.append("  __device__ static __forceinline__ Divs divisors(const Refs& R, const Params& P) {")
+                out.append("    (void)R; (void)P;")
+                out.append("    Divs d;")
+                for i, d in enumerate(udivs):
+                    out.append(f"    d.template set<{i}>({d});")
+                out.append("    return d;")
+                out.append("  }")
+                out.append("  __device__ static __forceinline__ T value_rgq(const T* s, const Refs& R, const Params& P, "
+                           "const Pre& pre, Quot& q) {")
+                out.append("    (void)s; (void)R; (void)P; (void)pre;")
+                out.append(f"    return {expr_quot};")
+                out.append("  }")
+                self._quot.add(sid)
             out.append("  template <bool CHECK, int RHH, int RWW>")
             out.append("  __device__ static __forceinline__ T value_pre(const T* lds, const uint8_t* vld, bool& ok, "
                        "int lr, int lc, const Refs& R, const Params& P, const Pre& pre) {")
@@ -1584,8 +1607,13 @@ class Emitter:
         o("  const bool inbox = full && r0 >= TH.blo[0] && r0 + RH <= TH.bhi[0] && c0 >= TH.blo[1] && c0 + RW <= TH.bhi[1];")
         o(f"  const bool safe = full && TH.uniform && r0 - {rl[0]} >= 0 && r0 + RH + {rh[0]} <= N0 && "
           f"c0 - {rl[1]} >= 0 && c0 + RW + {rh[1]} <= N1;")
-        o("  const xg::gptr<const T> __restrict__ src = xg::gp<const T>(TH.src.ptr);")
         o("  T V[BR][K];")
+        o("  auto load = [&]() {")
+        # (an address of its own each time: values kept from one load for the next would take
+        # the registers that hold the rows)
+        o("  uint64_t at = (uint64_t)TH.src.ptr;")
+        o('  asm volatile("" : "+s"(at));')
+        o("  const xg::gptr<const T> src = (xg::gptr<const T>)at;")
         o("  if (full) {")
         o("#pragma unroll")
         o("    for (int q = 0; q < BR; ++q) {")
@@ -1599,6 +1627,8 @@ class Emitter:
         o("#pragma unroll")
         o("      for (int k = 0; k < K; ++k) V[q][k] = src[(int64_t)min(gr + q, N0 - 1) * N1 + min(gc + k, N1 - 1)];")
         o("  }")
+        o("  };")
+        o("  load();")
         o("  int xb = 0;                 /* exchange buffer half */")
         o("  T U[K], D[K];               /* the rows above and below this wave's */")
         o("  auto exchange = [&]() {")
@@ -1660,7 +1690,12 @@ class Emitter:
             o("#pragma unroll")
             o("        for (int k = 0; k < K; ++k) {")
             gather(self._tb_reads[s.stmt.sid], down, "          ")
-            o(f"          const T x = {value};")
+            if dv == "DV" and s.stmt.sid in self._quot:
+                o("          T x;")
+                o(f"          if constexpr (QT) x = {S}::value_rgq(s, R{j}, P{j}, pre{j}[q][k], qt{j});")
+                o(f"          else x = {value};")
+            else:
+                o(f"          const T x = {value};")
             o(f"          V[q][k] = {'((mb >> (q * K + k)) & 1u) != 0u ? x : cur[k]' if member else 'x'};")
             o("        }")
             if rowtest:
@@ -1739,15 +1774,30 @@ class Emitter:
         # every uniform divisor has a reciprocal form in this launch
         o(f"  const bool dv = {' && '.join(dvs) if dvs else 'false'};")
         o("  (void)dv;")
+        quots = [(j, s.stmt.sid) for j, s in enumerate(L.stmts) if s.stmt.sid in self._quot]
+        for j, sid in quots:
+            o(f"  const xg_s{sid}::Divs dq{j} = xg_s{sid}::divisors(R{j}, P{j});")
+
         def run(body):
-            o("  auto run = [&](auto dv_c) {")
-            o("  constexpr bool DV = decltype(dv_c)::value;   /* reciprocal form of uniform divisions */")
-            o("  (void)DV;")
+            o("  auto run = [&](auto mode) -> bool {")
+            o("  /* the form of uniform divisions: 0 divide, 1 reciprocal, 2 corrected quotient */")
+            o("  constexpr bool DV = decltype(mode)::value == 1, QT = decltype(mode)::value == 2;")
+            o("  (void)DV; (void)QT;")
             prefetch()
+            for j, sid in quots:
+                o(f"  xg_s{sid}::Quot qt{j}(dq{j});")
             iterations(body)
+            o(f"  return {' && '.join(f'qt{j}.doubt == 0' for j, _ in quots) or 'true'};")
             o("  };")
-            o("  if constexpr (DVOK) { if (dv) run(xg::bconst<true>()); else run(xg::bconst<false>()); }")
-            o("  else run(xg::bconst<false>());")
+            o("  bool done = false;")
+            o("  if constexpr (DVOK) if (dv) done = run(xg::iconst<1>());")
+            if quots:
+                o(f"  if (!done && {' && '.join(f'dq{j}.ok' for j, _ in quots)}) {{")
+                o("    const bool sure = run(xg::iconst<2>());")
+                o("    done = !__builtin_amdgcn_readfirstlane(xg::block_or(sure ? 0u : 1u));")
+                o("    if (!done) load();")
+                o("  }")
+            o("  if (!done) run(xg::iconst<0>());")
 
         # A region inside the box of class 0 runs that class's statements on every cell: no mask
         # is read, nothing is tested or selected.
