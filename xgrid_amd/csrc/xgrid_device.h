@@ -43,7 +43,8 @@ namespace xg {
 
 /* Workgroup tile: 256 work-items, NC cells each per chunk, CH chunks in turn.
  *   1-D: 1024 consecutive cells (work-item t: t, t+256, t+512, t+768)
- *   2-D: 4 rows x 64 columns (one cell per work-item)
+ *   2-D: 4 rows x 64 columns (one cell per work-item), or x 64 times the columns that 16 bytes
+ *        hold for the statements that read rows so (CPL, TileCells)
  *   3-D: XG_TILE3_CHUNKS x 4 planes x 4 rows x 64 columns (work-item (r, c):
  *        planes 0..3 of each chunk, chunk after chunk); column tiles are
  *        aligned to multiples of 64 columns, so the first may start below lo */
@@ -237,14 +238,14 @@ __device__ __forceinline__ void unlin(const int32_t* shape, int64_t c, int& i0, 
 
 /* This workgroup's tile of the box [lo, hi): the NC cells of this work-item,
  * whether each is inside the box, and the tile's extent clipped to the box.
- * CPL (3-D only): columns per work-item.  A tile is 64 * CPL columns wide and
+ * CPL (2-D and 3-D): columns per work-item.  A tile is 64 * CPL columns wide and
  * work-item (r, c) holds columns CPL * c .. CPL * c + CPL - 1 of each of its
- * planes: cell n is plane n / CPL, column CPL * c + n % CPL (statements whose
- * staged loads read 16 bytes of a row per lane: CPL = 2 for 8-byte elements,
- * 4 for 4-byte ones). */
+ * planes: cell n is plane n / CPL, column CPL * c + n % CPL (16 bytes of a row
+ * per lane: CPL = 2 for 8-byte elements, 4 for 4-byte ones). */
 template <int D, int CPL = 1>
 struct TileCells {
-  static constexpr int NC = Tile<D>::NC * (D == 3 ? CPL : 1);
+  static constexpr int NC = Tile<D>::NC * (D >= 2 ? CPL : 1);
+  static constexpr int E1 = Tile<D>::E1 * (D == 2 ? CPL : 1);
   static constexpr int E2 = Tile<D>::E2 * (D == 3 ? CPL : 1);
   int c[NC][3];
   bool in[NC];
@@ -264,7 +265,7 @@ struct TileCells {
      * the tile. */
     const int a2 = D > 2 ? (lo[2] & ~(E2 - 1)) : 0;
     if (D == 2) {
-      const int n1 = (hi[1] - lo[1] + TL::E1 - 1) / TL::E1;
+      const int n1 = (hi[1] - lo[1] + E1 - 1) / E1;
       t0 = (int)tile / n1;
       t1 = (int)tile - t0 * n1;
     } else if (D == 3) {
@@ -292,12 +293,12 @@ struct TileCells {
       t2 = (int)(r2 - b * n2);
     }
     tlo[0] = lo[0] + t0 * (TL::E0 * TL::CH) + chunk * TL::E0;
-    tlo[1] = D > 1 ? lo[1] + t1 * TL::E1 : 0;
+    tlo[1] = D > 1 ? lo[1] + t1 * E1 : 0;
     const int c2 = a2 + t2 * E2;      /* first column of the (aligned) 3-D tile */
     col0 = c2;
     tlo[2] = D > 2 ? max(c2, lo[2]) : 0;
     thi[0] = min(tlo[0] + TL::E0, hi[0]);
-    thi[1] = D > 1 ? min(tlo[1] + TL::E1, hi[1]) : 1;
+    thi[1] = D > 1 ? min(tlo[1] + E1, hi[1]) : 1;
     thi[2] = D > 2 ? min(c2 + E2, hi[2]) : 1;
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
@@ -306,8 +307,8 @@ struct TileCells {
         c[n][1] = 0;
         c[n][2] = 0;
       } else if (D == 2) {
-        c[n][0] = tlo[0] + (tid >> 6) + 4 * n;  /* NC = 1: one row per wave */
-        c[n][1] = tlo[1] + (tid & 63);
+        c[n][0] = tlo[0] + (tid >> 6);  /* one row per wave */
+        c[n][1] = tlo[1] + (tid & 63) * CPL + n;
         c[n][2] = 0;
       } else {
         c[n][0] = tlo[0] + n / CPL;
@@ -328,7 +329,42 @@ struct TileCells {
       if (D > 2) c[n][2] = max(min(c[n][2], thi[2] - 1), tlo[2]);
     }
   }
+
+  /* The same for a 2-D tile at least CPL columns wide, a work-item's cells kept adjacent (one
+   * address, and vector loads): a lane that ends past the tile moves back as a whole, and
+   * the cells it passes on the way are another lane's. */
+  __device__ __forceinline__ void slide_to_tile() {
+    const int first = c[0][1], start = min(first, thi[1] - CPL), row = min(c[0][0], thi[0] - 1);
+    const bool row_in = c[0][0] < thi[0];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      c[n][0] = row;
+      c[n][1] = start + n;
+      in[n] = row_in && start + n >= first;
+    }
+  }
 };
+
+/* Store a lane's 2-D cells, computed for adjacent columns (slide_to_tile): where all are its own
+ * and the statement stores them where they are, as one vector. */
+template <class S, int OV, class TC>
+__device__ __forceinline__ void store_row(const xg_launch_hdr& H, const TC& tc, const typename S::T* v) {
+  typedef typename S::T T;
+  constexpr int K = TC::NC;
+  bool all = tc.in[0];
+#pragma unroll
+  for (int n = 1; n < K; ++n) all = all && tc.in[n];
+  if (S::SO0 == 0 && S::SO1 == 0 && all && !(H.dom.flags & XG_F_TO_TMP)) {
+    vecn<T, K> w;
+#pragma unroll
+    for (int n = 0; n < K; ++n) w[n] = v[n];
+    put_u<T, K>(gp<T>(H.out.ptr) + lin<2>(H.out.shape, tc.c[0][0], tc.c[0][1], 0), w);
+  } else {
+#pragma unroll
+    for (int n = 0; n < K; ++n)
+      if (tc.in[n]) store<S, OV>(H, tc.c[n][0], tc.c[n][1], tc.c[n][2], v[n]);
+  }
+}
 
 /* Do the tile's cells, the statement's loads and its store all lie inside the
  * grid, with every view of the grid shape (so no clamp or wrap is needed)? */
@@ -369,7 +405,14 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
     /* A work-item evaluates all its cells without branching, so their loads are
      * in flight together: a cell past the tile's edge is evaluated at the
      * nearest cell inside the tile (a valid address) and not stored. */
-    tc.clamp_to_tile();
+    constexpr bool WIDE = D == 2 && S::CPL > 1;
+    const bool wide = WIDE && tc.thi[1] - tc.tlo[1] >= S::CPL;   /* the lane's cells are adjacent */
+    if constexpr (WIDE) {
+      if (wide) tc.slide_to_tile();
+      else tc.clamp_to_tile();
+    } else {
+      tc.clamp_to_tile();
+    }
     if (MASKED) {
 #pragma unroll
       for (int n = 0; n < NC; ++n)
@@ -379,7 +422,7 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
     bool pairs = false;   /* store a lane's CPL columns with one 16-byte store */
     bool safe = tile_safe<S>(H, tc.tlo, tc.thi);
     if constexpr (D == 3 && S::ST3) safe = safe && H.out.shape[2] >= S::CPL;
-    if (safe) {
+    if (safe && (!WIDE || wide)) {
       if constexpr (D == 3 && S::ST3) {
         /* Staged 3-D tile: each array's columns of the tile's planes are read
          * once into registers; column neighbours come over DPP lane shifts and
@@ -400,6 +443,10 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
          * whatever alignment the row has. */
         if constexpr (S::CPL * sizeof(T) == 16 && S::SO0 == 0 && S::SO1 == 0 && S::SO2 == 0)
           pairs = !(H.dom.flags & XG_F_TO_TMP);
+      } else if constexpr (WIDE) {
+        S::value_row(v, R, P, H.out.shape, tc.c[0][0], tc.c[0][1]);
+        store_row<S, OV>(H, tc, v);
+        continue;
       } else {
 #pragma unroll
         for (int n = 0; n < NC; ++n) v[n] = S::template value<true>(R, P, H.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
@@ -531,20 +578,38 @@ __device__ void run_pair(const xg_launch_hdr& HA, const typename SA::Refs& RA, c
                          const xg_launch_hdr& HB, const typename SB::Refs& RB, const typename SB::Params& PB,
                          uint32_t tile) {
   constexpr int D = SA::D;
-  static_assert(SB::D == D, "paired statements share one tile");
+  static_assert(SB::D == D && SB::CPL == SA::CPL, "paired statements share one tile");
   for (int ch = 0; ch < Tile<D>::CH; ++ch) {
-    TileCells<D> tc(HA.dom.lo, HA.dom.hi, tile, ch);
+    typedef TileCells<D, SA::CPL> TC;
+    TC tc(HA.dom.lo, HA.dom.hi, tile, ch);
     if (tc.tlo[0] >= HA.dom.hi[0]) break;
-    constexpr int NC = TileCells<D>::NC;
-    tc.clamp_to_tile();  /* evaluate every cell without branching (see box_cells) */
+    constexpr int NC = TC::NC;
+    constexpr bool WIDE = D == 2 && SA::CPL > 1;
+    const bool wide = WIDE && tc.thi[1] - tc.tlo[1] >= SA::CPL;
+    /* evaluate every cell without branching (see box_cells) */
+    if constexpr (WIDE) {
+      if (wide) tc.slide_to_tile();
+      else tc.clamp_to_tile();
+    } else {
+      tc.clamp_to_tile();
+    }
     typename SA::T va[NC];
     typename SB::T vb[NC];
-    if (tile_safe<SA>(HA, tc.tlo, tc.thi) && tile_safe<SB>(HB, tc.tlo, tc.thi)) {
+    if (tile_safe<SA>(HA, tc.tlo, tc.thi) && tile_safe<SB>(HB, tc.tlo, tc.thi) && (!WIDE || wide)) {
+      if constexpr (WIDE) {
+        SA::value_row(va, RA, PA, HA.out.shape, tc.c[0][0], tc.c[0][1]);
+        if constexpr (FWD) SB::value_row_fwd(vb, RB, PB, HB.out.shape, tc.c[0][0], tc.c[0][1], va);
+        else SB::value_row(vb, RB, PB, HB.out.shape, tc.c[0][0], tc.c[0][1]);
+        store_row<SA, OV>(HA, tc, va);
+        store_row<SB, OV>(HB, tc, vb);
+        continue;
+      } else {
 #pragma unroll
-      for (int n = 0; n < NC; ++n) {
-        va[n] = SA::template value<true>(RA, PA, HA.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
-        if constexpr (FWD) vb[n] = SB::template value_fwd<true>(RB, PB, HB.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2], va[n]);
-        else vb[n] = SB::template value<true>(RB, PB, HB.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
+        for (int n = 0; n < NC; ++n) {
+          va[n] = SA::template value<true>(RA, PA, HA.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
+          if constexpr (FWD) vb[n] = SB::template value_fwd<true>(RB, PB, HB.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2], va[n]);
+          else vb[n] = SB::template value<true>(RB, PB, HB.out.shape, tc.c[n][0], tc.c[n][1], tc.c[n][2]);
+        }
       }
     } else {
 #pragma unroll

@@ -232,7 +232,7 @@ int fill_refs(xg_kernel* k, const xg_stmt_desc& d, std::vector<xg_gview>& refs) 
 // workgroups covering the box [lo, hi) with the tile of a D-dimensional statement
 int64_t tiles_for(int D, const int32_t* lo, const int32_t* hi, int cols3) {
   if (D == 1) return ceil_div(hi[0] - lo[0], 1024);
-  if (D == 2) return ceil_div(hi[0] - lo[0], 4) * ceil_div(hi[1] - lo[1], 64);
+  if (D == 2) return ceil_div(hi[0] - lo[0], 4) * ceil_div(hi[1] - lo[1], cols3);
   // column tiles of cols3 (64, 128 or 256) columns start at multiples of cols3 (TileCells in xgrid_device.h)
   return ceil_div(hi[0] - lo[0], 4 * XG_TILE3_CHUNKS) * ceil_div(hi[1] - lo[1], 4) *
          ceil_div(hi[2] - (lo[2] & ~(cols3 - 1)), cols3);
@@ -243,7 +243,7 @@ int64_t blocks_for_dom(int D, const xg_dom& dom, int cols3) {
   return tiles_for(D, dom.lo, dom.hi, cols3);
 }
 
-// 64 columns per lane-row of a 3-D tile times the columns each lane holds (1, 2 or 4)
+// 64 columns per lane-row of a 2-D or 3-D tile times the columns each lane holds (1, 2 or 4)
 int tile3_cols(const xg_stmt_desc& d) { return d.tile3_cols == 128 || d.tile3_cols == 256 ? d.tile3_cols : 64; }
 
 int do_launch(xg_kernel* k, int32_t sid, void* fn, int64_t blocks, int threads, void** args, size_t lds = 0) {
@@ -402,7 +402,7 @@ int exec_pair(xg_kernel* k, int32_t a, const void* pa, const void* pb) {
   void* args[6] = {&H[0], refs[0].data(), const_cast<void*>(pa), &H[1], refs[1].data(), const_cast<void*>(pb)};
   k->n_fused += 2;
   const xg_stmt_desc& d = k->stmts[(size_t)a].d;
-  return do_launch(k, -1, d.fn_pair, blocks_for_dom(d.dims, H[0].dom), kThreads, args);
+  return do_launch(k, -1, d.fn_pair, blocks_for_dom(d.dims, H[0].dom, tile3_cols(d)), kThreads, args);
 }
 
 // Are the cells beside the rows of class 0's 3-D box, up to a multiple of K columns, all of

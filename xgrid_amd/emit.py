@@ -830,6 +830,52 @@ class Emitter:
                 plan.add(refs.index((n.grid.name, n.level)), tuple(n.offsets))
         return plan if plan.usable() else None
 
+    def _value_row(self, st: StencilStmt, refs: list, grids: dict, row_groups: list, lower, fwd_type) -> list:
+        """The values of a 2-D lane's adjacent cells, in a tile that is safe.  The elements
+        that the cells read of one row are read once, as vectors where there are K of them."""
+        K = self._cpl2(st)
+        row_groups[0] = groups = {}
+        expr = lower()
+        row_groups[0] = None
+        o = ["  __device__ static __forceinline__ void value_row" + ("_fwd" if fwd_type else "") +
+             "(T* v, const Refs& R, const Params& P, const int32_t* sh, int i0, int i1" +
+             (f", const {fwd_type}* fwd) {{" if fwd_type else ") {"),
+             "    const int64_t xc = xg::lin<2>(sh, i0, i1, 0);",
+             "    (void)R; (void)P; (void)sh; (void)xc; (void)i0; (void)i1;"]
+        for n, ((g, lvl, row), cols) in enumerate(groups.items()):
+            et = device_type_name(grids[g].element)
+            lo, hi = min(cols), max(cols) + K - 1
+            need = sorted({c + k for c in cols for k in range(K)})
+            bases = []
+            if et in ("float", "double", "int32_t"):
+                left = set(need)
+                for b in [0] + need:
+                    if all(b + k in left for k in range(K)):
+                        bases.append(b)
+                        left -= {b + k for k in range(K)}
+                need = sorted(left)
+            o.append(f"    constexpr int O{n} = {-lo};")
+            o.append(f"    {et} a{n}[{hi - lo + 1}];")
+            o.append(f"    const xg::gptr<const {et}> p{n} = xg::gp<const {et}>(R.v[{refs.index((g, lvl))}].ptr) + xc + "
+                     f"xg::off<2>(sh, {row}, 0, 0);")
+            for b in bases:
+                o.append(f"    {{ const xg::vecn<{et}, {K}> w = xg::get_u<{et}, {K}>(p{n} + {b}); " +
+                         " ".join(f"a{n}[{b - lo + k}] = w[{k}];" for k in range(K)) + " }")
+            for c in need:
+                o.append(f"    a{n}[{c - lo}] = p{n}[{c}];")
+        o += ["#pragma unroll", f"    for (int k = 0; k < {K}; ++k) v[k] = {expr};", "  }"]
+        return o
+
+    @staticmethod
+    def _cpl2(st: StencilStmt) -> int:
+        """Columns a work-item holds in a 2-D tile: 16 bytes of a row.  With one cell, the
+        issue of about 200 vector instructions per wave bounded these statements, addresses above
+        all (a 64-bit one per load).  One and 16 bytes: the cavity's two pairs at 2049^2
+        23.5 and 27 -> 14.5 and 18 us FP32, 37 and 40 -> 33 and 33 us FP64 (5.1 TB/s),
+        1100 x 1537 FP64 diffusion 8.2 -> 6.1 us; 65^2 and 300^2 cavity calls 1 to 2 % slower
+        (a wave's own chain is longer)."""
+        return {"float": 4, "double": 2}.get(device_type_name(st.gtype.element), 1) if st.dimension == 2 else 1
+
     def _device_stmt(self, st: StencilStmt, refs: list, params: list, out: list, tb: LoopMeta | None = None,
                      fwd_from: str | None = None, meta: StmtMeta | None = None):
         sid = st.sid
@@ -844,11 +890,22 @@ class Emitter:
         pre_slots: list = []  # (grid, level, offsets) of each prefetched load
         rd_slots: list = []   # distinct (row, column) offsets of the loop grid's level-0 reads
         st3 = [None]          # while lowering value_st3: the staged 3-D plan (see _plan_st3)
+        row_groups = [None]   # while lowering value_row: {(grid, level, row offset): column offsets}
         fwd = [False]         # while lowering value_fwd: time-0 loads of `fwd_from` at the cell are `fwd`
 
         def cell(e: ir.Cell) -> str:
             if fwd[0] and e.grid.name == fwd_from and e.level == 0 and not any(e.offsets):
-                return "fwd"
+                return "fwd" if row_groups[0] is None else "fwd[k]"
+            if row_groups[0] is not None:
+                gt = grids[e.grid.name]
+                if gt.dimension == D:
+                    key = (e.grid.name, e.level, e.offsets[0])
+                    row_groups[0].setdefault(key, set()).add(e.offsets[1])
+                    return f"a{list(row_groups[0]).index(key)}[k + O{list(row_groups[0]).index(key)} + {e.offsets[1]}]"
+                o3 = [str(e.offsets[d]) if d < gt.dimension else "0" for d in range(3)]
+                r = refs.index((e.grid.name, e.level))
+                return (f"xg::ld<{device_type_name(gt.element)}, {gt.dimension}, XG_OVERSTEP, true>(R.v[{r}], sh, xc + k, "
+                        f"{', '.join(o3)}, i0, i1 + k, 0)")
             if st3[0] is not None:
                 acc = st3[0].access(refs.index((e.grid.name, e.level)), tuple(e.offsets))
                 if acc is not None:
@@ -944,10 +1001,10 @@ class Emitter:
         else:
             out.append("  static constexpr bool ST3 = false;")
             out.append("  static constexpr int ST3_LDS = 0;")
-            out.append("  static constexpr int CPL = 1;")
+            out.append(f"  static constexpr int CPL = {self._cpl2(st)};")
         if meta is not None:
-            # the host sizes this statement's 3-D launches by its tile width
-            meta.tile3_cols = plan3.COLS if expr_st3 is not None else 64
+            # the host sizes this statement's 2-D and 3-D launches by its tile width
+            meta.tile3_cols = plan3.COLS if expr_st3 is not None else 64 * self._cpl2(st)
         if fwd_from is not None:
             # the same expression with its time-0 loads of `fwd_from` at the cell taken from the
             # value the paired statement just computed for that cell
@@ -962,6 +1019,14 @@ class Emitter:
             out.append("    (void)R; (void)P; (void)sh; (void)xc; (void)i0; (void)i1; (void)i2; (void)fwd;")
             out.append(f"    return {expr_fwd};")
             out.append("  }")
+        if self._cpl2(st) > 1:
+            plain = lambda: _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
+            out.extend(self._value_row(st, refs, grids, row_groups, plain, None))
+            if fwd_from is not None:
+                fwd[0] = True
+                out.extend(self._value_row(st, refs, grids, row_groups, plain,
+                                           device_type_name(grids[fwd_from].element)))
+                fwd[0] = False
         if expr_tb is not None:
             # the same expression with the loop grid's level-0 reads taken from s[], the values
             # at the statement's distinct offsets (gathered from registers by the blocked kernel)
@@ -2433,7 +2498,7 @@ class Emitter:
             sa, sb = a.stmt, b.stmt
             ok = (a.group >= 0 and a.group == b.group and b.group_pos == a.group_pos + 1 and
                   sa.mode == "inplace" and sb.mode == "inplace" and
-                  sa.dimension == sb.dimension and sa.dimension in (1, 2) and
+                  sa.dimension == sb.dimension and sa.dimension in (1, 2) and self._cpl2(sa) == self._cpl2(sb) and
                   not any(sa.store_offsets) and not any(sb.store_offsets) and sa.grid != sb.grid and
                   (sb.grid, 0) not in a.refs)
             # b may read a's store at time 0 only at its own cell: that value is forwarded
@@ -2471,18 +2536,21 @@ class Emitter:
         def uniform(m):
             return not any(isinstance(n, (ir.Cell, ir.Call)) for n in ir.walk(m.stmt.node.value)) and not m.refs
 
+        def is_staged(m):
+            return m.stmt.dimension == 3 and m.tile3_cols != 64
+
         fans = []
 
         def close(run):
             fills = []
-            staged = [s[0] for s in run if s[0].tile3_cols != 64]
+            staged = [s[0] for s in run if is_staged(s[0])]
             for seg in run:
                 fill = None
-                if seg[0].tile3_cols != 64:
+                if is_staged(seg[0]):
                     fill = next((t[0] for t in run if len(t) == 1 and t is not seg and uniform(t[0]) and
                                  t[0].stmt.grid == seg[0].stmt.grid and not any(seg[0].stmt.store_offsets)), None)
                 fills.append(fill)
-            if len(staged) > 1 or any(f is None and s[0].tile3_cols != 64 for s, f in zip(run, fills)):
+            if len(staged) > 1 or any(f is None and is_staged(s[0]) for s, f in zip(run, fills)):
                 return
             if len(run) >= 2:
                 fans.append(FanMeta(f"xg_m{len(fans)}", list(run), fills))
