@@ -971,6 +971,32 @@ struct wave_axis {
   }
 };
 
+/* The wave tile (t0, t1) of workgroup b of nb = nt0 * nt1: tiles on the grid's edges first, spread
+ * over the XCDs, then the inner ones, a contiguous run per XCD.  An edge tile, which tests its
+ * cells, takes nearly three times as long as an inner one: row by row, a few XCDs had
+ * the top and bottom rows and the last workgroups to start were edge tiles. */
+struct wave_order {
+  int t0, t1;
+  __device__ __forceinline__ wave_order(uint32_t b, uint32_t nb, int nt0, int nt1) {
+    if (nt0 < 3 || nt1 < 3) {
+      const int t = (int)xcd_remap(b, nb);
+      t0 = t / nt1;
+      t1 = t - t0 * nt1;
+      return;
+    }
+    const uint32_t edge = 2u * (uint32_t)(nt0 + nt1 - 2);
+    if (b < edge) {
+      const int e = (int)xcd_remap(b, edge), s = e - 2 * nt1;
+      t0 = s >= 0 ? 1 + (s >> 1) : (e < nt1 ? 0 : nt0 - 1);
+      t1 = s >= 0 ? (s & 1) * (nt1 - 1) : (e < nt1 ? e : e - nt1);
+    } else {
+      const int t = (int)xcd_remap(b - edge, nb - edge), q = t / (nt1 - 2);
+      t0 = 1 + q;
+      t1 = 1 + t - q * (nt1 - 2);
+    }
+  }
+};
+
 /* How far the initial values that a cell's value depends on lie to its left, right, above and
  * below (16 bits each; adding a cell per statement to `unknown` stays far from their end). */
 struct wave_ext {

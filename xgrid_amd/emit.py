@@ -1648,7 +1648,7 @@ class Emitter:
                         rl[d] = max(rl[d], -n.offsets[d])
                         rh[d] = max(rh[d], n.offsets[d])
         o("template <bool DVOK>")
-        o(f"__device__ __forceinline__ void {V.kernel}_body({', '.join(params)}, const int tile) {{")
+        o(f"__device__ __forceinline__ void {V.kernel}_body({', '.join(params)}, const int t0, const int t1) {{")
         o(f"  typedef {T} T;")
         o(f"  constexpr int BR = {BR}, K = {K}, RW = 64 * K;")
         o(f"  typedef uint{32 if bits <= 32 else 64}_t MB;   /* a bit per cell of a lane */")
@@ -1662,7 +1662,6 @@ class Emitter:
         o(f"  MB* const smb = (MB*)(ex + 2 * WV) + threadIdx.x * {m};   /* this lane's membership bits */")
         o("  const int32_t* sh = TH.src.shape;")
         o("  const int N0 = sh[0], N1 = sh[1];")
-        o("  const int t0 = tile / TH.nt1, t1 = tile - t0 * TH.nt1;")
         o("  const xg::wave_axis A0(t0, TH.nt0, N0, RH, TH.halo), A1(t1, TH.nt1, N1, RW, TH.halo);")
         o("  const int r0 = A0.start, c0 = A1.start;")
         o("  const int gr = r0 + w * BR, gc = c0 + lane * K;   /* this wave's first row, this lane's first column */")
@@ -1923,13 +1922,15 @@ class Emitter:
         o("}")
         kargs = ["const xg_tb_hdr TH"] + [f"const xg_r{s.stmt.sid} R{j}, const xg_p{s.stmt.sid} P{j}"
                                           for j, s in enumerate(L.stmts)]
-        call = ", ".join(["TH"] + [f"R{j}, P{j}" for j in range(m)] + ["(int)xg::xcd_remap(blockIdx.x, gridDim.x)"])
+        call = ", ".join(["TH"] + [f"R{j}, P{j}" for j in range(m)] + ["at.t0", "at.t1"])
         bounds = f"__launch_bounds__({V.threads}) __attribute__((amdgpu_waves_per_eu({V.waves_per_simd})))"
-        o(f'extern "C" __global__ void {bounds} {V.kernel}({", ".join(kargs)}) {{ {V.kernel}_body<true>({call}); }}')
+        o(f'extern "C" __global__ void {bounds} {V.kernel}({", ".join(kargs)}) '
+          f"{{ const xg::wave_order at(blockIdx.x, gridDim.x, TH.nt0, TH.nt1); {V.kernel}_body<true>({call}); }}")
         loc, bcall = self._tb_entry_locals(L)
         o(f'extern "C" __global__ void {bounds} {V.kernel}_b(const xg_btent* __restrict__ E, const int32_t n, '
           f"const int64_t total) {{ xg::for_batch_tiles(E, n, total, [&](const xg_btent& e, uint32_t t) "
-          f"{{ {loc} {V.kernel}_body<false>({bcall}); __syncthreads(); }}); }}")
+          f"{{ {loc} const int t0 = (int)t / th.nt1; {V.kernel}_body<false>({bcall[:-len('(int)t')]}t0, (int)t - t0 * th.nt1); "
+          "__syncthreads(); }); }")
 
     @staticmethod
     def _tb_entry_locals(L: LoopMeta) -> tuple:
