@@ -57,6 +57,8 @@ typedef struct xg_stmt_desc {
   int32_t pair_fwd;                          /* fn_pair forwards this store to the next statement */
   int32_t tile3_cols;                        /* 2-D and 3-D fn_main: columns per tile (64, or 128 / 256 for
                                                 16 bytes of a row per lane); 0 means 64 */
+  int32_t flat_planes;                       /* 3-D fn_main: planes per work-item of a flat launch (0: none) */
+  int32_t reach_lo[3], reach_hi[3];          /* how far loads reach below and above the cell, by axis */
   void* fn_main;                             /* hipFunction_t of the class kernel */
   void* fn_pingpong;                         /* hipFunction_t of the Jacobi sweep (PINGPONG) */
   void* fn_phase2;                           /* hipFunction_t storing a temporary (two-phase) */

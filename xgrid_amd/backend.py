@@ -134,6 +134,8 @@ class HipKernel:
             d.fn_pair = fn(m.pair) if m.pair else None
             d.pair_fwd = int(m.pair_fwd)
             d.tile3_cols = m.tile3_cols
+            d.flat_planes = m.flat_planes
+            d.reach_lo[:], d.reach_hi[:] = read_reach(m.stmt)
         groups = (_lib.GroupDesc * max(1, len(low.groups)))()
         for i, g in enumerate(low.groups):
             groups[i].first = g.first

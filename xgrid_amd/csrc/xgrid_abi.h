@@ -40,6 +40,7 @@ typedef __hip_internal::uint64_t uint64_t;
 #define XG_F_TO_TMP 2    /* phase 1 of a two-phase statement: value -> src[cell] (no store offset) */
 #define XG_F_UNIFORM 4   /* every loaded view has the store grid's rank and shape */
 #define XG_F_STREAM 8    /* in place, two levels of the store grid exceed the last-level cache: 3-D box tiles store non-temporally */
+#define XG_F_FLAT 16     /* 3-D box class in place: work-items in one run over its rows (flat_cells) */
 
 typedef struct xg_gview {
   void* ptr;                 /* element 0 of one time level */

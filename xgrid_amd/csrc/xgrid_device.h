@@ -526,6 +526,58 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
   }
 }
 
+/* Work-items in one run over the rows of the class's box, each with CPL adjacent columns on
+ * FLAT planes, every read a vector load (L1 and L2 hold the rows and planes that work-items
+ * share).  For boxes whose rows leave many lanes of the staged tiles idle; the host has
+ * checked that every read lies inside the grid.  The last work-item of a row and the last
+ * planes move back into the box as a whole and store their own cells only.
+ * Bound by memory: 300x300x140 FP64 heat 6.3 TB/s (staged 4.3, where a tenth of the lanes
+ * of every second tile hold cells).  Two planes per work-item: four leave too few waves (250x333x301
+ * FP32 45 us against 37), one reads more from L2 (300x300x140 FP64 37 us against 32). */
+template <class S, int OV, bool NT, bool FILL = false>
+__device__ void flat_cells(const xg_launch_hdr& H, const typename S::Refs& R, const typename S::Params& P, uint32_t tile,
+                           const typename S::T fill = typename S::T()) {
+  typedef typename S::T T;
+  constexpr int K = S::CPL, NP = S::FLAT;
+  const int32_t* lo = H.dom.lo;
+  const int32_t* hi = H.dom.hi;
+  const uint32_t groups = (uint32_t)(hi[2] - lo[2] + K - 1) / K, items = (uint32_t)(hi[1] - lo[1]) * groups;
+  /* bands of 32 workgroups, inside a band plane chunks slowest: a chunk's halo planes were read
+   * 128 KB per plane earlier, and are still in this XCD's L2 */
+  constexpr uint32_t B = 32;
+  const uint32_t per = (items + XG_THREADS - 1) / XG_THREADS, chunks = (uint32_t)(hi[0] - lo[0] + NP - 1) / NP;
+  const uint32_t band = tile / (B * chunks), wide = min(B, per - band * B), rest = tile - band * B * chunks;
+  const uint32_t t0 = rest / wide, f = (band * B + rest - t0 * wide) * XG_THREADS + threadIdx.x;
+  if (f >= items) return;
+  const uint32_t r = f / groups;
+  const int row = lo[1] + (int)r, first = lo[2] + (int)(f - r * groups) * K, p0 = lo[0] + (int)t0 * NP;
+  const int start = min(first, hi[2] - K), plane = min(p0, hi[0] - NP);
+  T v[NP][K];
+  S::value_flat(v, R, P, H.out.shape, plane, row, start);
+  const gptr<T> out = gp<T>(H.out.ptr);
+#pragma unroll
+  for (int n = 0; n < NP; ++n) {
+    if (plane + n < p0) continue;
+    const int64_t at = lin<3>(H.out.shape, plane + n, row, 0);
+    if (start == first) {
+      vecn<T, K> w;
+#pragma unroll
+      for (int k = 0; k < K; ++k) w[k] = v[n][k];
+      put_u<T, K, NT>(out + at + start, w);
+    } else {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (start + k >= first) put<T, NT>(out + at + start + k, v[n][k]);
+    }
+    if (FILL) {   /* the cells that staged lanes store beside the row */
+      if (first == lo[2])
+        for (int c = lo[2] & ~(K - 1); c < lo[2]; ++c) put<T, NT>(out + at + c, fill);
+      if (first + K >= hi[2])
+        for (int c = hi[2]; c < min((hi[2] + K - 1) & ~(K - 1), H.out.shape[2]); ++c) put<T, NT>(out + at + c, fill);
+    }
+  }
+}
+
 /* Tile `tile` of `ntiles` of the statement's class (a list class: a slice of
  * the list, strided over the tiles). */
 template <class S, int OV>
@@ -541,6 +593,12 @@ __device__ void run_main(const xg_launch_hdr& H, const typename S::Refs& R, cons
       apply<S, OV>(H, R, P, i0, i1, i2);
     }
   } else if constexpr (D == 3 && S::ST3) {
+    if constexpr (S::FLAT > 0)
+      if (dom.flags & XG_F_FLAT) {
+        if (dom.flags & XG_F_STREAM) flat_cells<S, OV, true>(H, R, P, tile);
+        else flat_cells<S, OV, false>(H, R, P, tile);
+        return;
+      }
     /* one LDS copy for the box variants (staged 3-D loads) */
     __shared__ __attribute__((aligned(16))) unsigned char st3_lds[S::ST3_LDS];
     if (dom.kind == XG_DOM_MASKED) box_cells<S, OV, true>(H, R, P, tile, st3_lds);
@@ -562,6 +620,12 @@ __device__ void run_main(const xg_launch_hdr& H, const typename S::Refs& R, cons
 template <class S, int OV>
 __device__ void run_fill(const xg_launch_hdr& H, const typename S::Refs& R, const typename S::Params& P, uint32_t tile,
                          const typename S::T fill) {
+  if constexpr (S::FLAT > 0)
+    if (H.dom.flags & XG_F_FLAT) {
+      if (H.dom.flags & XG_F_STREAM) flat_cells<S, OV, true, true>(H, R, P, tile, fill);
+      else flat_cells<S, OV, false, true>(H, R, P, tile, fill);
+      return;
+    }
   __shared__ __attribute__((aligned(16))) unsigned char st3_lds[S::ST3_LDS];
   if (H.dom.flags & XG_F_STREAM) box_cells<S, OV, false, true, true>(H, R, P, tile, st3_lds, fill);
   else box_cells<S, OV, false, false, true>(H, R, P, tile, st3_lds, fill);

@@ -246,6 +246,32 @@ int64_t blocks_for_dom(int D, const xg_dom& dom, int cols3) {
 // 64 columns per lane-row of a 2-D or 3-D tile times the columns each lane holds (1, 2 or 4)
 int tile3_cols(const xg_stmt_desc& d) { return d.tile3_cols == 128 || d.tile3_cols == 256 ? d.tile3_cols : 64; }
 
+// XG_F_FLAT if a staged statement's in-place launch over the box `dom` is better flat (flat_cells):
+// if too few lanes of the staged tiles, 128 columns wide in FP64 and 256 in FP32, hold cells of
+// it.  Grids that the last-level cache holds are better flat below nine tenths, larger ones
+// below six, since a flat launch reads halo planes from memory more often.  Heat updates, us,
+// staged / flat, with the share of lanes held: 400x400x60 FP32 (0.23) 43 / 17, 300x300x115 (0.44)
+// 39 / 18, FP64 (0.88) 33 / 28, 250x333x301 FP32 (0.58) 48 / 37, 256^3 FP32 (0.99) 24 / 26; larger
+// ones: 400x400x270 FP32 (0.52) 113 / 88, 450x450x150 FP64 (0.58) 136 / 116, 400x400x270 FP64
+// (0.70) 159 / 173, 250x333x301 FP64 (0.78) 92 / 101.
+int32_t flat_flag(const xg_stmt_desc& d, const xg_dom& dom, const int32_t* shape) {
+  const int K = tile3_cols(d) / 64;
+  if (d.dims != 3 || d.flat_planes <= 0 || dom.kind != XG_DOM_BOX || !(dom.flags & XG_F_UNIFORM)) return 0;
+  for (int a = 0; a < 3; ++a)
+    if (dom.lo[a] < d.reach_lo[a] || dom.hi[a] + d.reach_hi[a] > shape[a]) return 0;
+  const int64_t cols = dom.hi[2] - dom.lo[2], rows = dom.hi[1] - dom.lo[1];
+  if (cols < K || dom.hi[0] - dom.lo[0] < d.flat_planes || rows * ceil_div(cols, K) > 0x7fffffff) return 0;
+  const int64_t lanes = ceil_div(dom.hi[2] - (dom.lo[2] & ~(64 * K - 1)), 64 * K) * 64 * K;
+  return cols * 10 < lanes * (dom.flags & XG_F_STREAM ? 6 : 9) ? XG_F_FLAT : 0;
+}
+
+// Workgroups of a statement's fn_main over its class.
+int64_t main_blocks(const xg_stmt_desc& d, const xg_dom& dom) {
+  if (!(dom.flags & XG_F_FLAT)) return blocks_for_dom(d.dims, dom, tile3_cols(d));
+  const int64_t items = (dom.hi[1] - dom.lo[1]) * ceil_div(dom.hi[2] - dom.lo[2], tile3_cols(d) / 64);
+  return ceil_div(dom.hi[0] - dom.lo[0], d.flat_planes) * ceil_div(items, kThreads);
+}
+
 int do_launch(xg_kernel* k, int32_t sid, void* fn, int64_t blocks, int threads, void** args, size_t lds = 0) {
   if (blocks <= 0) return XG_OK;
   if (blocks > 0x7fffffff) return fail(XG_ERR_ARG, "launch grid too large");
@@ -284,8 +310,9 @@ int exec_stmt(xg_kernel* k, int32_t sid, const void* params) {
   H.dom.flags = uni;
   if (mode == XG_MODE_INPLACE) {
     H.dom.flags |= stream_flag(G);  // 3-D box tiles of large grids store non-temporally
+    H.dom.flags |= flat_flag(d, H.dom, G->shape);
     fill_view(H.out, G, G->levels[0]);
-    return do_launch(k, sid, d.fn_main, blocks_for_dom(d.dims, H.dom, tile3_cols(d)), kThreads, args);
+    return do_launch(k, sid, d.fn_main, main_blocks(d, H.dom), kThreads, args);
   }
   if (!G->scratch) return fail(XG_ERR_STATE, "scratch buffer missing");
   if (mode == XG_MODE_PINGPONG) {
@@ -525,6 +552,7 @@ int exec_fan(xg_kernel* k, const std::vector<Pending>& run, size_t i, size_t n, 
       fill_dom(H.dom, G->plan(d.klass), G, d.klass);
       fill_view(H.out, G, G->levels[0]);
       H.dom.flags = (uniform_refs(k, d) ? XG_F_UNIFORM : 0) | stream_flag(G);
+      H.dom.flags |= flat_flag(d, H.dom, G->shape);
       if (int rc = fill_refs(k, d, refs[(size_t)q])) return rc;
       params = k->arena.data() + run[i + (size_t)(sid - run[i].sid)].off;
     }
@@ -553,7 +581,7 @@ int exec_fan(xg_kernel* k, const std::vector<Pending>& run, size_t i, size_t n, 
     for (int32_t t = 0; t < s; ++t) q += f.seg_len[t];
     const xg_stmt_desc& d = k->stmts[(size_t)(f.first + q)].d;
     const xg_dom& dom = hdrs[(size_t)q].dom;
-    const int64_t tiles = dom.kind == XG_DOM_EMPTY || dom.count == 0 ? 0 : blocks_for_dom(d.dims, dom, tile3_cols(d));
+    const int64_t tiles = dom.kind == XG_DOM_EMPTY || dom.count == 0 ? 0 : main_blocks(d, dom);
     if (f.seg_len[s] == 2) k->n_fused += 2;
     F.tiles[s] = (uint32_t)tiles;
     blocks += ceil_div(tiles, 8) * 8;

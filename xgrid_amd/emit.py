@@ -88,6 +88,7 @@ class StmtMeta:
     pair_fwd: bool = False        # ... with the next one's loads of this store (own cell, time 0) forwarded
     fwd_from: str | None = None   # (second of a forwarding pair) the grid whose time-0 loads are forwarded
     hoisted: list = field(default_factory=list)   # [Hoist]: launch-uniform subexpressions computed by the host
+    flat_planes: int = 0          # planes a work-item of a flat 3-D launch holds (0: no such launches)
     tile3_cols: int = 64          # columns of a 3-D tile of this statement's run_main kernels
 
 
@@ -830,19 +831,12 @@ class Emitter:
                 plan.add(refs.index((n.grid.name, n.level)), tuple(n.offsets))
         return plan if plan.usable() else None
 
-    def _value_row(self, st: StencilStmt, refs: list, grids: dict, row_groups: list, lower, fwd_type) -> list:
-        """The values of a 2-D lane's adjacent cells, in a tile that is safe.  The elements
-        that the cells read of one row are read once, as vectors where there are K of them."""
-        K = self._cpl2(st)
-        row_groups[0] = groups = {}
-        expr = lower()
-        row_groups[0] = None
-        o = ["  __device__ static __forceinline__ void value_row" + ("_fwd" if fwd_type else "") +
-             "(T* v, const Refs& R, const Params& P, const int32_t* sh, int i0, int i1" +
-             (f", const {fwd_type}* fwd) {{" if fwd_type else ") {"),
-             "    const int64_t xc = xg::lin<2>(sh, i0, i1, 0);",
-             "    (void)R; (void)P; (void)sh; (void)xc; (void)i0; (void)i1;"]
-        for n, ((g, lvl, row), cols) in enumerate(groups.items()):
+    @staticmethod
+    def _row_loads(groups: dict, refs: list, grids: dict, K: int) -> list:
+        """Each row's elements (groups: (grid, level, plane and row offsets) -> column offsets of the K
+        cells' reads), read once: as vectors where there are K of them, else one by one."""
+        o = []
+        for n, ((g, lvl, *row), cols) in enumerate(groups.items()):
             et = device_type_name(grids[g].element)
             lo, hi = min(cols), max(cols) + K - 1
             need = sorted({c + k for c in cols for k in range(K)})
@@ -857,12 +851,48 @@ class Emitter:
             o.append(f"    constexpr int O{n} = {-lo};")
             o.append(f"    {et} a{n}[{hi - lo + 1}];")
             o.append(f"    const xg::gptr<const {et}> p{n} = xg::gp<const {et}>(R.v[{refs.index((g, lvl))}].ptr) + xc + "
-                     f"xg::off<2>(sh, {row}, 0, 0);")
+                     f"xg::off<{len(row) + 1}>(sh, {', '.join(map(str, row))}, {'0, 0' if len(row) == 1 else 0});")
             for b in bases:
                 o.append(f"    {{ const xg::vecn<{et}, {K}> w = xg::get_u<{et}, {K}>(p{n} + {b}); " +
                          " ".join(f"a{n}[{b - lo + k}] = w[{k}];" for k in range(K)) + " }")
             for c in need:
                 o.append(f"    a{n}[{c - lo}] = p{n}[{c}];")
+        return o
+
+    def _value_flat(self, st: StencilStmt, refs: list, grids: dict, row_groups: list, row_plane: list, K: int,
+                    lower) -> list:
+        """The values of K adjacent cells of a row on FLAT_PLANES planes, every read a load (flat_cells)."""
+        row_groups[0] = groups = {}
+        exprs = []
+        for n in range(self.FLAT_PLANES):
+            row_plane[0] = n
+            exprs.append(lower())
+        row_groups[0], row_plane[0] = None, 0
+        o = [f"  static constexpr int FLAT = {self.FLAT_PLANES};",
+             "  __device__ static __forceinline__ void value_flat(T (&v)[FLAT][CPL], const Refs& R, const Params& P, "
+             "const int32_t* sh, int i0, int i1, int i2) {",
+             "    const int64_t xc = xg::lin<3>(sh, i0, i1, i2);",
+             "    (void)R; (void)P; (void)sh; (void)xc; (void)i0; (void)i1; (void)i2;"]
+        o += self._row_loads(groups, refs, grids, K)
+        for n, e in enumerate(exprs):
+            o += ["#pragma unroll", f"    for (int k = 0; k < {K}; ++k) v[{n}][k] = {e};"]
+        return o + ["  }"]
+
+    FLAT_PLANES = 2
+
+    def _value_row(self, st: StencilStmt, refs: list, grids: dict, row_groups: list, lower, fwd_type) -> list:
+        """The values of a 2-D lane's adjacent cells, in a tile that is safe.  The elements
+        that the cells read of one row are read once, as vectors where there are K of them."""
+        K = self._cpl2(st)
+        row_groups[0] = groups = {}
+        expr = lower()
+        row_groups[0] = None
+        o = ["  __device__ static __forceinline__ void value_row" + ("_fwd" if fwd_type else "") +
+             "(T* v, const Refs& R, const Params& P, const int32_t* sh, int i0, int i1" +
+             (f", const {fwd_type}* fwd) {{" if fwd_type else ") {"),
+             "    const int64_t xc = xg::lin<2>(sh, i0, i1, 0);",
+             "    (void)R; (void)P; (void)sh; (void)xc; (void)i0; (void)i1;"]
+        o += self._row_loads(groups, refs, grids, K)
         o += ["#pragma unroll", f"    for (int k = 0; k < {K}; ++k) v[k] = {expr};", "  }"]
         return o
 
@@ -890,7 +920,8 @@ class Emitter:
         pre_slots: list = []  # (grid, level, offsets) of each prefetched load
         rd_slots: list = []   # distinct (row, column) offsets of the loop grid's level-0 reads
         st3 = [None]          # while lowering value_st3: the staged 3-D plan (see _plan_st3)
-        row_groups = [None]   # while lowering value_row: {(grid, level, row offset): column offsets}
+        row_groups = [None]   # while lowering value_row, value_flat: {(grid, level, row offset): column offsets}
+        row_plane = [0]       # ... and the plane of the work-item's cells
         fwd = [False]         # while lowering value_fwd: time-0 loads of `fwd_from` at the cell are `fwd`
 
         def cell(e: ir.Cell) -> str:
@@ -899,13 +930,16 @@ class Emitter:
             if row_groups[0] is not None:
                 gt = grids[e.grid.name]
                 if gt.dimension == D:
-                    key = (e.grid.name, e.level, e.offsets[0])
-                    row_groups[0].setdefault(key, set()).add(e.offsets[1])
-                    return f"a{list(row_groups[0]).index(key)}[k + O{list(row_groups[0]).index(key)} + {e.offsets[1]}]"
+                    up = (e.offsets[0] + row_plane[0],) if D == 3 else ()
+                    key = (e.grid.name, e.level, *up, e.offsets[D - 2])
+                    row_groups[0].setdefault(key, set()).add(e.offsets[D - 1])
+                    n = list(row_groups[0]).index(key)
+                    return f"a{n}[k + O{n} + {e.offsets[D - 1]}]"
+                # (never run: a tile is safe only where all views have the store grid's shape)
                 o3 = [str(e.offsets[d]) if d < gt.dimension else "0" for d in range(3)]
                 r = refs.index((e.grid.name, e.level))
                 return (f"xg::ld<{device_type_name(gt.element)}, {gt.dimension}, XG_OVERSTEP, true>(R.v[{r}], sh, xc + k, "
-                        f"{', '.join(o3)}, i0, i1 + k, 0)")
+                        f"{', '.join(o3)}, i0, i1, 0)")
             if st3[0] is not None:
                 acc = st3[0].access(refs.index((e.grid.name, e.level)), tuple(e.offsets))
                 if acc is not None:
@@ -972,6 +1006,7 @@ class Emitter:
             self._tb_reads[sid] = list(rd_slots)
         so = list(st.store_offsets) + [0] * (3 - len(st.store_offsets))
         rl, rh = read_reach(st)
+        flat = 0
         nr = max(1, len(refs))
         out.append(f"// statement {sid}: {st.node.loc}")
         out.append(f"struct xg_p{sid} {{ {param_fields(meta, device_type_name)} }};")
@@ -998,11 +1033,19 @@ class Emitter:
         out.append("  }")
         if expr_st3 is not None:
             out.extend(plan3.members(expr_st3))
+            if plan3.cpl * plan3.esize == 16 and not any(so):
+                out.extend(self._value_flat(st, refs, grids, row_groups, row_plane, plan3.cpl,
+                                            lambda: _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)))
+                flat = self.FLAT_PLANES
+            else:
+                out.append("  static constexpr int FLAT = 0;")
         else:
             out.append("  static constexpr bool ST3 = false;")
+            out.append("  static constexpr int FLAT = 0;")
             out.append("  static constexpr int ST3_LDS = 0;")
             out.append(f"  static constexpr int CPL = {self._cpl2(st)};")
         if meta is not None:
+            meta.flat_planes = flat
             # the host sizes this statement's 2-D and 3-D launches by its tile width
             meta.tile3_cols = plan3.COLS if expr_st3 is not None else 64 * self._cpl2(st)
         if fwd_from is not None:
