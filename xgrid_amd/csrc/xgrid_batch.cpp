@@ -512,7 +512,7 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
       ok.push_back(t);
       shapes.push_back(wave_shape(k->grids[(size_t)ld.grid_arg], L));
     }
-    const WaveCut cut = ok.empty() ? WaveCut{} : wave_choose(ld, shapes, trip);
+    const WaveCut cut = ok.empty() ? WaveCut{} : wave_choose(ld, shapes, trip, true);
     for (size_t i = 0; i < ok.size(); ++i) {
       if (cut.waves) b->inst[(size_t)idx[(size_t)ok[i]]].k->loops[(size_t)lid].cut = wave_cut_for(ld, cut, shapes[i]);
       else plain.push_back(ok[i]);

@@ -166,8 +166,8 @@ struct WaveShape {
 };
 inline WaveShape wave_shape(const xg_grid* G, const LoopProof& p) { return {G->shape[0], G->shape[1], p.reach}; }
 // The tile, waves and iterations with which the launches for `trip` iterations run all `shapes`
-// (one batch).  waves = 0: no tile holds the loop.
-WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip);
+// (`batch`: as one batched launch).  waves = 0: no tile holds the loop.
+WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip, bool batch);
 // ... with the halo and tile counts of one grid.
 WaveCut wave_cut_for(const xg_loop_desc& d, WaveCut c, const WaveShape& s);
 // Header of a mask's checking launch, and what its answer (XG_WAVE_MAX_ITERS numbers) says.

@@ -708,14 +708,34 @@ WaveCut wave_cut_for(const xg_loop_desc& d, WaveCut c, const WaveShape& s) {
   return c;
 }
 
-// Estimated time of one launch of wave tiles, for choosing among cuts: memory traffic, and per
-// round of resident workgroups the iterations, each with the serial chain of one wave's
-// cells, the workgroup's exchange, and the cells of the waves that share a SIMD.  Fitted to
-// cavity sweeps of 65^2 to 2049^2 in both precisions, both tiles and 2 to 16 waves: the
-// cut it picks is within 8 % of the best of about 60 measured ones, mostly the best.
+// Estimated time of one launch of wave tiles, for choosing among cuts (less what is the same for
+// all): memory traffic, and per round of resident workgroups the iterations, each with the
+// serial chain of one wave's cells, the workgroup's exchange, and the cells of the waves
+// that share a SIMD.  Rounds need not be whole, since edge tiles, the long ones, start first.  A
+// workgroup alone on its unit reads and writes with nothing to run beside it: its traffic counts
+// more.  Fitted to cavity steps of 130^2 to 2049^2 in both precisions, both tiles, 5 to 16
+// waves and 5 to 13 iterations (1600 cuts): of those, what it picks is within 5 % of the best,
+// mostly the best.  (With whole rounds, fitted before edge tiles started first, within 34 %:
+// 1700^2 FP64 284 us a step against 235, FP32 255 against 196, 2049^2 FP64 343 against 297.)
 static double wave_launch_us(const xg_loop_desc& d, const WaveCut& c, int64_t blocks) {
   const xg_wave_tile& t = d.wave[c.tile];
   const double cells = (double)t.rows * d.wave_cols / 64;   // of a lane
+  const int64_t cus = std::max(1, g_dev.cus);
+  int64_t per_cu = std::max<int64_t>(1, 4 * t.waves_per_simd / c.waves);
+  if (t.lds > 0) per_cu = std::max<int64_t>(1, std::min<int64_t>(per_cu, 163840 / ((int64_t)c.waves * t.lds)));
+  const double at_once = (double)std::min(per_cu, ceil_div(std::min(blocks, cus * per_cu), cus));
+  const double iteration = 0.0004 + 0.0158 * c.waves + 0.0529 * cells + 0.00165 * cells * std::max(1.0, at_once * c.waves / 4);
+  const double rounds = std::max(1.0, (double)blocks / (double)(cus * per_cu));
+  const double traffic = 3.3e-5 * (double)blocks * c.waves * cells * d.wave_elem / 4 * (per_cu == 1 ? 1.72 : 1.0);
+  return 2.28 + traffic + c.iters * rounds * iteration;
+}
+
+// The same for a batch, whose tiles start instance by instance: whole rounds, the last one as long
+// as its workgroups take.  Fitted like the above, before edge tiles started first in plain
+// launches (16 mixed instances of sides 64 to 1024 FP64: 222 us a step by this estimate, 236 by that).
+static double wave_batch_us(const xg_loop_desc& d, const WaveCut& c, int64_t blocks) {
+  const xg_wave_tile& t = d.wave[c.tile];
+  const double cells = (double)t.rows * d.wave_cols / 64;
   const int64_t cus = std::max(1, g_dev.cus);
   int64_t per_cu = std::max<int64_t>(1, 4 * t.waves_per_simd / c.waves);
   if (t.lds > 0) per_cu = std::max<int64_t>(1, std::min<int64_t>(per_cu, 163840 / ((int64_t)c.waves * t.lds)));
@@ -728,7 +748,7 @@ static double wave_launch_us(const xg_loop_desc& d, const WaveCut& c, int64_t bl
   return 5.0 + 4.42e-5 * (double)blocks * c.waves * cells * d.wave_elem / 4 + c.iters * its;
 }
 
-WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip) {
+WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes, int64_t trip, bool batch) {
   WaveCut best;
   double best_us = 0.0;
   for (int32_t t = 0; t < d.nwave; ++t)
@@ -752,7 +772,7 @@ WaveCut wave_choose(const xg_loop_desc& d, const std::vector<WaveShape>& shapes,
         c.iters = (int32_t)T;
         int64_t blocks = 0;
         for (const WaveShape& s : shapes) blocks += wave_cut_for(d, c, s).blocks();
-        const double us = (double)ceil_div(trip, T) * wave_launch_us(d, c, blocks);
+        const double us = (double)ceil_div(trip, T) * (batch ? wave_batch_us(d, c, blocks) : wave_launch_us(d, c, blocks));
         if (best.waves == 0 || us < best_us) {
           best = c;
           best_us = us;
@@ -767,7 +787,7 @@ static void wave_cut_plain(LoopPlan& L, const xg_grid* G, int64_t trip) {
   if (L.chosen_trip != trip || L.chosen_n0 != G->shape[0] || L.chosen_n1 != G->shape[1] ||
       std::memcmp(L.chosen_reach, L.reach, sizeof L.reach) != 0) {
     const WaveShape s = wave_shape(G, L);
-    L.chosen = wave_choose(L.d, {s}, trip);
+    L.chosen = wave_choose(L.d, {s}, trip, false);
     if (L.chosen.waves) L.chosen = wave_cut_for(L.d, L.chosen, s);
     L.chosen_trip = trip;
     L.chosen_n0 = s.n0;
