@@ -229,7 +229,10 @@ class _ExprC:
         # device statements: divisor texts of the per-cell divisions by a launch-uniform
         # value, which are emitted as xg::udiv<DV> (see _uniform_division)
         self.udivs = udivs
-        self.quot = False             # emit them as q.div<number> instead (xg::Quot)
+        # ... those whose divisions are emitted as q.div<number> instead (xg::Quot): not below a
+        # condition, where a lane may not run them (a ballot would miss it)
+        self.quots = None
+        self.below = 0                # conditions around the node being emitted
         self.hoisted = hoisted or {}  # id(node) -> text of its host-computed value
         self.fold_pow = fold_pow      # host text with the device's pow folds (hoisted values)
 
@@ -275,16 +278,26 @@ class _ExprC:
             d = self(e.right)
             if d not in self.udivs:
                 self.udivs.append(d)
-            if self.quot:
-                return f"q.template div<{self.udivs.index(d)}>({self(e.left)}, {d})"
+            if self.quots is not None and not self.below:
+                if d not in self.quots:
+                    self.quots.append(d)
+                return f"q.template div<{self.quots.index(d)}>({self(e.left)}, {d})"
             return f"xg::udiv<DV>({self(e.left)}, {d})"
-        return f"({self(e.left)} {e.op} {self(e.right)})"
+        left = self(e.left)
+        return f"({left} {e.op} {self._arm(e.right) if e.op in ('&&', '||') else self(e.right)})"
 
     def e_Un(self, e):
         return f"({e.op} {self(e.operand)})"
 
+    def _arm(self, e) -> str:
+        """An operand that some lanes may not evaluate."""
+        self.below += 1
+        text = self(e)
+        self.below -= 1
+        return text
+
     def e_Select(self, e):
-        return f"({self(e.cond)} ? {self(e.then)} : {self(e.orelse)})"
+        return f"({self(e.cond)} ? {self._arm(e.then)} : {self._arm(e.orelse)})"
 
     def e_Cast(self, e):
         tn = device_type_name(e.type) if self.device else ctype_name(e.type)
@@ -981,6 +994,7 @@ class Emitter:
             expr_st3 = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
             st3[0] = None
         expr_tb = expr_pre = expr_quot = expr_lds = expr_lds_pre = None
+        quots: list = []      # divisors of expr_quot's corrected quotients
         if tb is not None:
             in_reg[0] = True
             expr_tb = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
@@ -994,7 +1008,7 @@ class Emitter:
                 expr_pre = _ExprC(True, cell, name, grid_info, udivs, hoisted)(st.node.value)
                 if udivs:
                     x = _ExprC(True, cell, name, grid_info, udivs, hoisted)
-                    x.quot = True
+                    x.quots = quots
                     expr_quot = x(st.node.value)
                 in_reg[0] = False
                 in_lds[0] = True
@@ -1139,12 +1153,12 @@ class Emitter:
             out.append("    (void)s; (void)R; (void)P; (void)pre;")
             out.append(f"    return {expr_pre};")
             out.append("  }")
-            if expr_quot is not None:
-                out.append(f"  typedef xg::Divisors<{len(udivs)}> Divs; typedef xg::Quot<{len(udivs)}> Quot;")
+            if quots:
+                out.append(f"  typedef xg::Divisors<{len(quots)}> Divs; typedef xg::Quot<{len(quots)}> Quot;")
                 out.append("  __device__ static __forceinline__ Divs divisors(const Refs& R, const Params& P) {")
                 out.append("    (void)R; (void)P;")
                 out.append("    Divs d;")
-                for i, d in enumerate(udivs):
+                for i, d in enumerate(quots):
                     out.append(f"    d.template set<{i}>({d});")
                 out.append("    return d;")
                 out.append("  }")
