@@ -11,12 +11,13 @@ fallback: without the library or a GPU this raises.
 from __future__ import annotations
 
 import ctypes
+import os
 import weakref
 from ctypes import c_void_p
 
 from . import _lib
 from .analysis import analyze
-from .compilers import compile_device, compile_host, load_host
+from .compilers import compile_device, compile_host, kernel_scratch, load_host
 from .config import get_config
 from .emit import Emitter, Lowered, read_reach
 from .grid import Grid
@@ -29,12 +30,36 @@ class KernelError(RuntimeError):
     pass
 
 
-def lower_kernel(op, block_shape: tuple | None = None) -> Lowered:
+def lower_kernel(op, block_shape: tuple | None = None, fits: dict | None = None) -> Lowered:
     cfg = get_config()
     info = analyze(op.ir)
     if not cfg.parallel and any(st.implicit for st in info.stmts):
         raise KernelError("Unable to perform implicit operation while parallel is off")
-    return Emitter(info, cfg.overstep, cfg.comment, macro=op.macro, block_shape=block_shape).lower(), info
+    return Emitter(info, cfg.overstep, cfg.comment, macro=op.macro, block_shape=block_shape, fits=fits).lower(), info
+
+
+def compile_kernel(op, block_shape: tuple | None = None) -> tuple:
+    """Lower a kernel and compile its device code, with blocked loops on wave tiles only where
+    the code object says that they fit (Emitter.FIT_FULL): each loop whose 4-row tile spills registers is
+    built anew the next way.  A loop that fits, such as the cavity's, takes one compile.
+    Returns (lowered kernel, analysis, code object path)."""
+    cfg = get_config()
+    fits: dict = {}
+    given = block_shape is not None or os.environ.get("XGRID_TB_SHAPE")   # tiles asked for are built
+    while True:
+        low, info = lower_kernel(op, block_shape, fits)
+        path = compile_device(low.device_src, cfg.cacheroot, cfg.fp_contract)
+        loops = [] if given else [L for L in low.loops if L.waves]
+        scratch = kernel_scratch(path) if loops else {}
+        again = [L for L in loops if scratch[L.waves[-1].kernel] > 0]
+        if not again:
+            break
+        for L in again:
+            fits[L.lid] = fits.get(L.lid, Emitter.FIT_FULL) + 1
+    for L in loops:
+        if fits.get(L.lid) == Emitter.FIT_ROOM and scratch[L.waves[0].kernel] > Emitter.ROOM_8_ROWS_SCRATCH:
+            del L.waves[0]           # (the list is the small-grid plan's too)
+    return low, info, path
 
 
 def _ctype_of(t):
@@ -78,12 +103,11 @@ class HipKernel:
         self.cfg = cfg                   # options are those in force when the kernel was built
         self.op = op
         self.lib = _lib.ensure_device(cfg.device)
-        low, info = lower_kernel(op, block_shape)
+        low, info, self.code_object = compile_kernel(op, block_shape)
         self.block_shape = tuple(block_shape) if block_shape is not None else low.block_shape
         self.lowered = low
         self.info = info
         self.depth = info.depth
-        self.code_object = compile_device(low.device_src, cfg.cacheroot, cfg.fp_contract)
         self.stub_path = compile_host(low.stub_src, cfg.cacheroot, cfg.cc, cfg.opt_level)
         mod = c_void_p()
         _lib.check(self.lib.xg_module_load(self.code_object.encode(), ctypes.byref(mod)), "xg_module_load")

@@ -14,6 +14,7 @@ import ctypes
 import hashlib
 import os
 import shutil
+import struct
 import subprocess
 import tempfile
 import threading
@@ -74,6 +75,30 @@ def compile_device(src: str, cacheroot: str, fp_contract: bool = False) -> str:
     if rc != 0:
         raise CompileError(_lib.last_error())
     return path
+
+
+def kernel_scratch(path: str) -> dict:
+    """Scratch bytes per work-item (spilled registers) of each kernel of a code object: the
+    private_segment_fixed_size of its kernel descriptor, the symbol `<kernel>.kd` (AMDGPU code
+    object ABI: 64 bytes, the size at byte 4)."""
+    with open(path, "rb") as f:
+        b = f.read()
+    (at,) = struct.unpack_from("<Q", b, 0x28)
+    size, count = struct.unpack_from("<HH", b, 0x3a)
+    # name, type, flags, addr, offset, size, link, info, align, entsize
+    sections = [struct.unpack_from("<IIQQQQIIQQ", b, at + i * size) for i in range(count)]
+    out = {}
+    for s in sections:
+        if s[1] not in (2, 11):      # symbol tables
+            continue
+        names = sections[s[6]][4]
+        for o in range(s[4], s[4] + s[5], 24):
+            name, _, _, where, addr, _ = struct.unpack_from("<IBBHQQ", b, o)
+            name = b[names + name:b.index(b"\0", names + name)].decode()
+            if name.endswith(".kd") and where < count:
+                desc = sections[where][4] + addr - sections[where][3]
+                out[name[:-3]] = struct.unpack_from("<I", b, desc + 4)[0]
+    return out
 
 
 def find_cc(candidates) -> str:

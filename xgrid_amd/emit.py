@@ -136,7 +136,8 @@ class WaveTile:
     k: int                        # region columns a lane holds (64 * k columns)
     threads: int                  # most work-items of a workgroup
     lds: int                      # LDS bytes per wave: two halves of its first and last row, membership bits
-    waves_per_simd: int           # what its registers leave room for (launch bounds ask for it)
+    waves_per_simd: int           # what the cavity's registers leave room for (the cut estimate's occupancy)
+    asked: int                    # waves per SIMD that the kernel is compiled for
 
     @property
     def cols(self) -> int:
@@ -752,8 +753,10 @@ class _St3Plan:
 
 class Emitter:
     def __init__(self, info: KernelInfo, overstep: str = "none", comment: bool = False,
-                 entry: str = "xg_entry", macro: list | None = None, block_shape: tuple | None = None):
+                 entry: str = "xg_entry", macro: list | None = None, block_shape: tuple | None = None,
+                 fits: dict | None = None):
         self.info = info
+        self.fits = fits or {}         # loop -> how its wave tiles are built (FIT_*; default: FIT_FULL)
         self.shape = tuple(block_shape) if block_shape is not None else None   # None: by element size
         self.used_shape = None         # the shape the blockable loops were built with
         self.macro = list(macro or [])
@@ -1980,7 +1983,7 @@ class Emitter:
         kargs = ["const xg_tb_hdr TH"] + [f"const xg_r{s.stmt.sid} R{j}, const xg_p{s.stmt.sid} P{j}"
                                           for j, s in enumerate(L.stmts)]
         call = ", ".join(["TH"] + [f"R{j}, P{j}" for j in range(m)] + ["at.t0", "at.t1"])
-        bounds = f"__launch_bounds__({V.threads}) __attribute__((amdgpu_waves_per_eu({V.waves_per_simd})))"
+        bounds = f"__launch_bounds__({V.threads}) __attribute__((amdgpu_waves_per_eu({V.asked})))"
         o(f'extern "C" __global__ void {bounds} {V.kernel}({", ".join(kargs)}) '
           f"{{ const xg::wave_order at(blockIdx.x, gridDim.x, TH.nt0, TH.nt1); {V.kernel}_body<true>({call}); }}")
         loc, bcall = self._tb_entry_locals(L)
@@ -2439,6 +2442,24 @@ class Emitter:
     # wave tiles (rows per wave, region columns, most work-items) of loops whose reads of the
     # loop grid reach one cell
     WAVE_TILES = ((8, 128, 1024), (4, 128, 1024))
+    # How a loop's wave tiles are built.  Beside the rows a lane keeps in registers, for all
+    # iterations, what the body reads of other grids and what the compiler moves out of the
+    # iterations; a tile that spills waits for scratch memory (all six arrays of a
+    # variable-coefficient Poisson sweep: 7.1 ms for 50 sweeps of 2049^2 FP64, 1.7 ms with the region in LDS).
+    #   FIT_FULL   for the waves per SIMD that the cavity's registers leave room for (_wave_tile)
+    #   FIT_ROOM   for the waves of one workgroup only: 128 registers
+    #   FIT_NONE   no wave tiles: the region in LDS
+    # The first under which the 4-row tile spills nothing is taken (backend.compile_kernel).  50
+    # sweeps, us, FIT_FULL / FIT_ROOM / LDS: three other values a cell 300^2 FP64 75 / 52 / 68, 2049^2
+    # 853 / 327 / 475, two and two quotients 600^2 FP32 150 / 96 / 114, 2049^2 578 / 394 / 764.
+    FIT_FULL, FIT_ROOM, FIT_NONE = 0, 1, 2
+    # Bodies that are better in LDS whatever the registers: more than three values of other grids a cell
+    # in the statements of class 0 (four, 600^2 FP64: 87 us, 82 with LDS), or more than one in a wall's,
+    # whose rows every tile on the grid's edge then keeps as well (three, 600^2 FP64: 139 and 113 us).
+    WAVE_MAX_VALUES, WAVE_MAX_WALL_VALUES = 3, 1
+    # Most values, walls and all, for which FIT_ROOM keeps the 8-row tile, and the scratch bytes it may take
+    # then: 2049^2 FP64 with and without it, two values 289 and 370 us, three 846 and 358.
+    ROOM_8_ROWS_VALUES, ROOM_8_ROWS_SCRATCH = 2, 512
 
     @classmethod
     def block_shape(cls, spec: str | None = None, elem: int = 8) -> tuple:
@@ -2493,9 +2514,13 @@ class Emitter:
                 if L.alt is not None:
                     L.alt.batched = False
                     L.alt_max_cells = self.SMALL_GRID_MAX_CELLS[elem]
-                if reach == 1 and device_type_name(ms[0].stmt.gtype.element) in ("float", "double"):
-                    L.waves = [self._wave_tile(L, L.kernel + ("_s" if i else ""), br, cols, t)
-                               for i, (br, cols, t) in enumerate(self.WAVE_TILES)]
+                fit = self.fits.get(L.lid, self.FIT_FULL)
+                if reach == 1 and fit != self.FIT_NONE and device_type_name(ms[0].stmt.gtype.element) in ("float", "double"):
+                    inner, walls = self._other_values(ms, g)
+                    if inner <= self.WAVE_MAX_VALUES and max(walls, default=0) <= self.WAVE_MAX_WALL_VALUES:
+                        L.waves = [self._wave_tile(L, L.kernel + ("_s" if i else ""), br, cols, t, fit)
+                                   for i, (br, cols, t) in enumerate(self.WAVE_TILES)
+                                   if i or fit == self.FIT_FULL or inner + sum(walls) <= self.ROOM_8_ROWS_VALUES]
                     if L.alt is not None:
                         L.alt.waves = L.waves
             loops.append(L)
@@ -2503,13 +2528,29 @@ class Emitter:
         return loops
 
     @staticmethod
-    def _wave_tile(L: LoopMeta, name: str, rows: int, cols: int, threads: int) -> WaveTile:
+    def _other_values(ms: list, g: str) -> tuple:
+        """The values per cell that a loop's statements read of other grids and levels: of class 0's
+        statements together, and of each other statement."""
+        inner, walls = 0, []
+        for m in ms:
+            n = len({(c.grid.name, c.level, tuple(c.offsets)) for c in ir.walk(m.stmt.node.value)
+                     if isinstance(c, ir.Cell) and not (c.grid.name == g and c.level == 0)})
+            if m.stmt.klass == 0:
+                inner += n
+            else:
+                walls.append(n)
+        return inner, walls
+
+    @staticmethod
+    def _wave_tile(L: LoopMeta, name: str, rows: int, cols: int, threads: int, fit: int = 0) -> WaveTile:
         elem = element_nbytes(L.stmts[0].stmt.gtype.element)
         bits = 4 if rows * cols // 64 <= 32 else 8
         # 122 / 74 registers hold the cavity's FP64 tiles of 8 / 4 rows, 86 / 55 its FP32 ones
         waves = {8: {True: 6, False: 4}, 4: {True: 8, False: 5}}[elem][rows * cols <= 512]
+        least = -(-threads // 256)      # those of one workgroup
+        waves = max(waves, least)
         return WaveTile(name, rows, cols // 64, threads, 2 * 2 * cols * elem + 64 * bits * len(L.stmts),
-                        max(waves, -(-threads // 256)))
+                        waves, waves if fit == Emitter.FIT_FULL else least)
 
     @staticmethod
     def _loop_meta(lid: int, node, ms: list, g: str, reach: int, shape: tuple, name: str):

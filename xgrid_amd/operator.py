@@ -141,15 +141,14 @@ class Precompile:
 
     def _run(self):
         import time
-        from .backend import lower_kernel
-        from .compilers import compile_device, compile_host
+        from .backend import compile_kernel
+        from .compilers import compile_host
         from .config import thread_config
         t0 = time.perf_counter()
         try:
             _private.table = {}
             with thread_config(self.cfg):
-                low, _ = lower_kernel(self.op)
-                compile_device(low.device_src, self.cfg.cacheroot, self.cfg.fp_contract)
+                low, _, _ = compile_kernel(self.op)
                 compile_host(low.stub_src, self.cfg.cacheroot, self.cfg.cc, self.cfg.opt_level)
         except Exception as e:          # reported by the first call's own build
             self.error = e
