@@ -672,10 +672,15 @@ int finish_capture(xg_batch* b, BatchGraph* g) {
     XG_HIP(hipMemcpyAsync(dev, b->arena.data(), b->arena.size(), hipMemcpyHostToDevice, g_dev.stream));
     XG_HIP(hipStreamSynchronize(g_dev.stream));
   }
-  XG_HIP(hipStreamBeginCapture(g_dev.stream, hipStreamCaptureModeThreadLocal));
-  int rc = issue(b, dev);
+  int rc = XG_OK;
   hipGraph_t graph = nullptr;
-  hipError_t e = hipStreamEndCapture(g_dev.stream, &graph);
+  hipError_t e = hipSuccess;
+  {
+    std::lock_guard<std::recursive_mutex> lock(g_recording);
+    XG_HIP(hipStreamBeginCapture(g_dev.stream, hipStreamCaptureModeThreadLocal));
+    rc = issue(b, dev);
+    e = hipStreamEndCapture(g_dev.stream, &graph);
+  }
   reset_table(b);
   if (rc || e != hipSuccess) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -776,6 +781,7 @@ int xg_batch_create(void* packed_entry, int32_t tick, xg_batch** out) {
 
 int xg_batch_destroy(xg_batch* b) {
   if (!b) return XG_OK;
+  std::lock_guard<std::recursive_mutex> lock(g_recording);
   if (g_dev.ready) (void)hipStreamSynchronize(g_dev.stream);
   for (auto& g : b->cache) destroy_graph(g);
   if (b->d_table) (void)hipFree(b->d_table);

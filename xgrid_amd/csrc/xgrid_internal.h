@@ -7,6 +7,7 @@
 
 #include <climits>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -42,6 +43,12 @@ struct Device {
   int64_t fuse_max_cells = 0;   // a chained statement walks at most this many cells
 };
 extern Device g_dev;
+
+// Held by the thread that has the kernel stream record a graph, from its begin to its end, and by
+// whatever a garbage collector may run meanwhile on another thread: freeing grids, destroying
+// kernels and batches.  These enqueue on that stream or wait for it, and waiting for a stream that
+// records ends the recording with an error.
+extern std::recursive_mutex g_recording;
 
 inline int check_ready() {
   if (!g_dev.ready) return fail(XG_ERR_STATE, "xg_init has not been called");

@@ -125,6 +125,7 @@ struct xg_kernel {
   uint64_t tick = 0;
   int64_t n_launch = 0, n_fused = 0, n_replay = 0, n_capture = 0;
   int64_t capture_mark = 0;         // n_launch when the current capture began
+  std::unique_lock<std::recursive_mutex> recording;   // held (g_recording) while this kernel's call is captured
   int32_t timed_sid = -1;
   std::vector<xgi::EventPair> events;
   std::vector<xgi::LoopPlan> loops;

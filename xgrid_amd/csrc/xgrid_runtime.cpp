@@ -29,6 +29,7 @@ namespace xgi {
 
 thread_local std::string t_err;
 Device g_dev;
+std::recursive_mutex g_recording;
 
 /* A serving loop admits and retires grids while other requests' kernels run:
  * hipFree waits for the whole device, and so did the stream synchronisations
@@ -56,13 +57,12 @@ int dev_alloc(size_t bytes, bool zero, void** out) {
   return XG_OK;
 }
 
-/* While the kernel stream records a graph (another thread inside a call), a free
- * enqueued there would become part of the graph: such frees wait in a list until
- * the next release made outside a capture. */
+/* While the kernel stream records a graph, a free enqueued there would become part of the
+ * graph: a free by another thread waits for the end, one by the recording thread itself
+ * waits in a list until the next release made outside a capture. */
 void dev_free(void* p) {
-  static std::mutex mu;
   static std::vector<void*> held;
-  std::lock_guard<std::mutex> lock(mu);
+  std::lock_guard<std::recursive_mutex> lock(g_recording);
   if (p) held.push_back(p);
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(g_dev.stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return;
@@ -855,6 +855,7 @@ void fill_tb_hdr(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int iters, int32_t* f
 // arguments are not freed under a launch in flight.
 void destroy_entry(GraphEntry& e) {
   if (e.exec) {
+    std::lock_guard<std::recursive_mutex> lock(g_recording);
     if (g_dev.ready) (void)hipStreamSynchronize(g_dev.stream);
     (void)hipGraphExecDestroy(e.exec);
   }
@@ -922,8 +923,10 @@ int api_begin(xg_kernel* k, xg_grid* const* grids, int32_t ngrids, const void* k
       }
       k->mode = kCapture;
       k->capture_mark = k->n_launch;
+      k->recording = std::unique_lock<std::recursive_mutex>(g_recording);
       hipError_t err = hipStreamBeginCapture(g_dev.stream, hipStreamCaptureModeThreadLocal);
       if (err != hipSuccess) {
+        k->recording.unlock();
         k->mode = kDirect;
         k->cur = nullptr;
         return set_status(k, fail(XG_ERR_HIP, std::string("hipStreamBeginCapture: ") + hipGetErrorString(err)));
@@ -1010,6 +1013,7 @@ int api_end(xg_kernel* k) {
   if (k->mode == kCapture) {
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(g_dev.stream, &graph);
+    k->recording.unlock();
     GraphEntry* ent = k->cur;
     if (e != hipSuccess || k->status != XG_OK) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -1348,6 +1352,7 @@ int xg_module_function(xg_module* m, const char* name, void** out_fn) {
 
 int xg_module_unload(xg_module* m) {
   if (!m) return XG_OK;
+  std::lock_guard<std::recursive_mutex> lock(g_recording);
   if (g_dev.ready) XG_HIP(hipStreamSynchronize(g_dev.stream));  // its kernels may still run
   XG_HIP(hipModuleUnload(m->mod));
   delete m;
@@ -1376,6 +1381,7 @@ int xg_grid_create(int32_t dims, const int32_t* shape, int32_t elem_bytes, xg_gr
 
 int xg_grid_destroy(xg_grid* g) {
   if (!g) return XG_OK;
+  std::lock_guard<std::recursive_mutex> lock(g_recording);
   // the memory is released behind the kernels queued on the kernel stream; work that
   // a caller queued elsewhere on a handed-out level pointer is waited for first
   if (g->exported && g_dev.ready) (void)hipDeviceSynchronize();
