@@ -284,8 +284,8 @@ int xg_grid_norm_diff(xg_grid* a, int32_t level_a, int32_t type_a, xg_grid* b, i
  * call.  Its partials live in a static device array of 512 partials (8,192
  * bytes per GPU, held until the process ends; its address is looked up by
  * xg_init) and its result in pinned host memory that xg_init allocates.  Any
- * class size fits: at most 512 workgroups each reduce a strided slice.  Every call on a GPU shares that GPU's array, so
- * calls that overlap on one GPU (several host threads at once) race.
+ * class size fits: at most 512 workgroups each reduce a strided slice.  Every call on a GPU shares that GPU's array:
+ * calls of several host threads take turns, here and in the other norms.
  * Synchronises the backend stream. */
 int xg_grid_norm_diff_noalloc(xg_grid* a, int32_t level_a, int32_t type_a, xg_grid* b, int32_t level_b,
                               int32_t type_b, int32_t klass, double* l2, double* linf, int64_t* cells);

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 
 #include "xgrid_internal.h"
@@ -273,16 +274,22 @@ int64_t class_domain(const xg_grid* G, int32_t klass, xg_dom& dom, int32_t* shap
   return ceil_div(rows, (int64_t)64 >> lg);
 }
 
-// Where one reduction's partials, count and result go: scratch 0 or 1.
+// Where one reduction's partials, count and result go: scratch 0 or 1.  Held from the launch until
+// the result is read: calls of several threads take turns.
+std::mutex g_space[2];
 struct RedSpace {
   Partial* part;
   uint32_t* done;
   Partial* out;
+  std::unique_lock<std::mutex> held;
 };
 
 int red_space(int which, RedSpace& r) {
   if (g_dev.id < 0 || g_dev.id >= kMaxDevices || !g_done[g_dev.id] || !g_result)
     return fail(XG_ERR_STATE, "the device's scratch address was not looked up (xg_init)");
+  r.held = std::unique_lock<std::mutex>(g_space[which]);
+  if (!which)
+    if (int rc = ensure_partials()) return rc;
   r.part = which ? g_scratch[g_dev.id] : g_part;
   r.done = g_done[g_dev.id] + which * kDoneLines * kDoneLine;
   r.out = g_result + which;
@@ -359,7 +366,6 @@ extern "C" {
 int xg_grid_norm_diff(xg_grid* a, int32_t level_a, int32_t type_a, xg_grid* b, int32_t level_b, int32_t type_b,
                       int32_t klass, double* l2, double* linf, int64_t* cells) {
   if (int rc = check_ready()) return rc;
-  if (int rc = ensure_partials()) return rc;
   RedSpace sp;
   if (int rc = red_space(0, sp)) return rc;
   return norm_diff(a, level_a, type_a, b, level_b, type_b, klass, l2, linf, cells, sp);
@@ -390,7 +396,6 @@ int xg_grid_poisson_residual(xg_grid* p, int32_t level_p, int32_t type_p, xg_gri
     for (int a = 0; a < p->dims; ++a)
       if (cp.lo[a] < 1 || cp.hi[a] > p->shape[a] - 1)
         return fail(XG_ERR_ARG, "the class reaches the edge of the grid: the residual's stencil would leave it");
-  if (int rc = ensure_partials()) return rc;
   RedSpace sp;
   if (int rc = red_space(0, sp)) return rc;
   xg_dom dom;
