@@ -104,7 +104,9 @@ class HipKernel:
         self.op = op
         self.lib = _lib.ensure_device(cfg.device)
         low, info, self.code_object = compile_kernel(op, block_shape)
-        self.block_shape = tuple(block_shape) if block_shape is not None else low.block_shape
+        # the tile shape asked for, or the one the default build's loops have (None: wave tiles)
+        self.block_shape = tuple(block_shape) if block_shape is not None else \
+            None if any(L.waves for L in low.loops) else low.block_shape
         self.lowered = low
         self.info = info
         self.depth = info.depth

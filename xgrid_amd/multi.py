@@ -68,8 +68,8 @@ class MultiSolver:
         return b
 
     def autotune(self, specs: list, limit: int = 48, use_cache: bool = True) -> dict:
-        """Pick the blocked-loop tile shape of each batch (kernel and size class) on
-        fresh copies of a sample of its `specs`, before any instance is added."""
+        """Pick the blocked-loop build of each batch (kernel and size class: the default one, None,
+        or a tile shape) on fresh copies of a sample of its `specs`, before any instance is added."""
         from . import autotune
         if self.members:
             raise RuntimeError("autotune before adding instances")
