@@ -504,8 +504,8 @@ int run_loop(xg_batch* b, int32_t lid, int64_t trip, const std::vector<int>& idx
     for (int t : blocked) {
       xg_kernel* k = b->inst[(size_t)idx[(size_t)t]].k;
       LoopPlan& L = k->loops[(size_t)lid];
-      if (wave_outrun(L, trip)) {
-        L.state = -1;
+      L.outrun = wave_outrun(L, trip);
+      if (L.outrun) {
         plain.push_back(t);
         continue;
       }

@@ -83,6 +83,7 @@ struct LoopPlan : LoopProof {
   xg_loop_desc d;
   std::vector<LoopProof> others;   // other masks' proofs, most recent first
   WaveCut cut;                     // wave tiles: the cut of the launches being made
+  bool outrun = false;             // wave tiles: the last call's iterations needed too wide a halo (wave_outrun)
   // wave tiles: the cut last chosen for one grid, and what it was chosen for (choosing takes the
   // host 13 us, as long as two launches)
   WaveCut chosen;
@@ -174,8 +175,8 @@ WaveCut wave_cut_for(const xg_loop_desc& d, WaveCut c, const WaveShape& s);
 // Header of a mask's checking launch, and what its answer (XG_WAVE_MAX_ITERS numbers) says.
 void fill_wave_check(xg_kernel* k, LoopPlan& L, xg_tb_hdr& TH, int32_t* answer);
 void wave_answer(LoopPlan& L, const int32_t* answer);
-// Is the loop to be left to plain launches: a launch of trip iterations (at most tmax) would need
-// too wide a halo?
+// Is a call to be left to plain launches: a launch of its trip iterations (at most tmax) would need
+// too wide a halo?  Fewer iterations may still run blocked, so the proof keeps what each count needs.
 bool wave_outrun(const LoopPlan& L, int64_t trip);
 constexpr size_t kCheckBytes = XG_WAVE_MAX_ITERS * sizeof(int32_t);   // answer of a checking launch
 constexpr int kWaveCheckThreads = 1024;

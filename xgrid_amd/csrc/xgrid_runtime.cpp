@@ -1160,6 +1160,8 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
   xg_grid* G = k->grids[(size_t)L.d.grid_arg];
   if (!loop_blockable(k, L)) return 0;
   if (L.state < 0) return 0;
+  L.outrun = L.d.nwave && L.state == 1 && wave_outrun(L, trip);
+  if (L.outrun) return 0;
   // A check proves launches of up to the iterations it ran: the set of exact region
   // cells only shrinks from one iteration to the next, so a proof at T covers fewer
   // iterations, but a launch of more iterations than any check ran needs its own.
@@ -1193,10 +1195,8 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
     }
   }
   if (L.d.nwave) {
-    if (wave_outrun(L, trip)) {
-      L.state = -1;
-      return 0;
-    }
+    L.outrun = wave_outrun(L, trip);
+    if (L.outrun) return 0;
     wave_cut_plain(L, G, trip);
     if (L.cut.waves == 0) return 0;
   }
@@ -1685,7 +1685,7 @@ int xg_kernel_loop_info(xg_kernel* k, int32_t lid, int64_t* launches, int64_t* i
   const LoopPlan& L = k->loops[(size_t)lid];
   if (launches) *launches = L.launches;
   if (iterations) *iterations = L.iterations;
-  if (state) *state = L.state;
+  if (state) *state = L.outrun ? -1 : L.state;
   return XG_OK;
 }
 
@@ -1697,13 +1697,16 @@ int xg_kernel_time_loop(xg_kernel* k, int32_t lid, int32_t trip, int32_t reps, d
     return fail(XG_ERR_STATE, "the loop has not run blocked yet");
   if (k->mode != kDirect) return fail(XG_ERR_STATE, "a call is in progress");
   xg_grid* G = k->grids[(size_t)L.d.grid_arg];
+  if (!loop_blockable(k, L) || L.state != 1) return fail(XG_ERR_STATE, "the loop has not run blocked on this mask");
+  if (L.d.nwave) {
+    if (wave_outrun(L, trip)) return fail(XG_ERR_STATE, "that many iterations do not run blocked on this mask");
+    wave_cut_plain(L, G, trip);
+    if (L.cut.waves == 0) return fail(XG_ERR_STATE, "no tile holds the loop");
+  }
   std::vector<const void*> ps;
   for (auto& p : L.last_params) ps.push_back(p.data());
   // one trip = the launches a call makes for `trip` iterations
-  auto run_trip = [&]() -> int {
-    if (L.d.nwave) wave_cut_plain(L, G, trip);
-    return run_blocked(k, L, G, ps.data(), trip);
-  };
+  auto run_trip = [&]() -> int { return run_blocked(k, L, G, ps.data(), trip); };
   hipEvent_t e0, e1;
   XG_HIP(hipEventCreate(&e0));
   XG_HIP(hipEventCreate(&e1));
