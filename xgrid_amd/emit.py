@@ -1902,39 +1902,6 @@ class Emitter:
         for j, sid in quots:
             o(f"  const xg_s{sid}::Divs dq{j} = xg_s{sid}::divisors(R{j}, P{j});")
 
-        def sample():
-            """Corrected quotients of a column in one row of each wave, before the iterations: numbers below
-            the bound, as where a field spreads from rest, come in bands, and a workgroup that meets
-            them divides at once instead of running all its iterations twice.  (Looked at during the
-            iterations, the kernel spills.)  The waves' answers go through the half of the exchange
-            that is used second.  FP64 cavities from rest, 1000^2 (steps 10 to 40) 212 -> 173 us a step, 2000^2
-            (10 to 110) 458 -> 379, with divisions throughout 180 and 402; developed flow 1000^2 137.5 -> 139,
-            2049^2 the same, FP32 300^2 177 -> 173, 2049^2 220 -> 214 (scheduled differently)."""
-            o("  if constexpr (QT) {")
-            o("    constexpr int q = BR / 2;")
-            o("    uint64_t doubt = 0;")
-            for j, s in enumerate(L.stmts):
-                if s.stmt.klass != 0 or s.stmt.sid not in self._quot:
-                    continue
-                o("    {")
-                o(f"      xg_s{s.stmt.sid}::Quot qt(dq{j});")
-                o("      T prev[K], cur[K], next[K];")
-                o("#pragma unroll")
-                o("      for (int k = 0; k < K; ++k) { cur[k] = V[q][k]; "
-                  "prev[k] = q > 0 ? V[q > 0 ? q - 1 : 0][k] : U[k]; next[k] = q + 1 < BR ? V[q + 1 < BR ? q + 1 : q][k] : D[k]; }")
-                o("      (void)prev; (void)next;")
-                o("      constexpr int k = 0;")
-                gather(self._tb_reads[s.stmt.sid], True, "      ")
-                o(f"      (void)xg_s{s.stmt.sid}_t<false>::value_rgq(s, R{j}, P{j}, pre{j}[q][k], qt);")
-                o("      doubt |= qt.doubt;")
-                o("    }")
-            o("    uint32_t* const said = (uint32_t*)(ex + WV);")
-            o("    if (lane == 0) said[w] = doubt != 0 ? 1u : 0u;")
-            o("    __syncthreads();")
-            o("    if (__ballot(lane < WV && said[lane < WV ? lane : 0] != 0u)) return false;")
-            o("    __builtin_amdgcn_sched_barrier(0);")
-            o("  }")
-
         def run(body):
             o("  auto run = [&](auto mode) -> bool {")
             o("  /* the form of uniform divisions: 0 divide, 1 reciprocal, 2 corrected quotient */")
@@ -1943,8 +1910,6 @@ class Emitter:
             prefetch()
             for j, sid in quots:
                 o(f"  xg_s{sid}::Quot qt{j}(dq{j});")
-            if any(s.stmt.klass == 0 and s.stmt.sid in self._quot for s in L.stmts):
-                sample()
             iterations(body)
             o(f"  return {' && '.join(f'qt{j}.doubt == 0' for j, _ in quots) or 'true'};")
             o("  };")
