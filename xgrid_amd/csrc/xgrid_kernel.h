@@ -16,10 +16,10 @@ namespace xgi {
 constexpr int kThreads = 256;
 constexpr int kGroupThreads = 1024;
 constexpr int64_t kFuseMaxCells = 4096;  // default of g_dev.fuse_max_cells (XGRID_FUSE_MAX_CELLS)
-// A call with fewer launches runs them directly: replaying a graph of one kernel takes 21.8 us
-// of host time against 6.3.  A small cavity is three launches and over 60 us of device time,
-// which hides either.
-constexpr int64_t kGraphMinLaunches = 3;
+// A call with fewer launches runs them directly: replaying a graph takes 21 to 33 us of host time, three
+// launches 12 (45^2 to 400^2, three statements, us a call: 21 and 12), and a small cavity, which is
+// three launches and 50 us of device time, 60 against 57.5.
+constexpr int64_t kGraphMinLaunches = 4;
 // Store grids of which two levels do not fit the 256 MB last-level cache (Infinity Cache) take
 // non-temporal stores in 3-D box tiles: by the time the next update reads a cell it has left the
 // cache anyway, and the write stream drains faster.  The line lies where both ways meet (heat
