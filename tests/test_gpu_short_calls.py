@@ -1,4 +1,5 @@
-"""Calls of a few launches: three are made directly (replaying a graph costs more)."""
+"""Calls of a few launches: three are made directly (replaying a graph costs more), and a pair of interiors
+inside a chain does not cut it in two."""
 import numpy as np
 import pytest
 
@@ -21,9 +22,10 @@ def _kernel():
     return steps
 
 
-@pytest.mark.parametrize("n, launches", [(200, 3)])
+@pytest.mark.parametrize("n, launches", [(45, 1), (200, 3)])
 def test_launches(double, n, launches):
-    """u, the pair of v and w, the wall; no graph, however often the call repeats."""
+    """45^2: one chain (v and w are a pair, with u before and the wall after them).  200^2: u, the pair, the
+    wall; no graph, however often the call repeats."""
     k = _kernel()
     rng = np.random.default_rng(1)
     mask = np.full((n, n), 9, np.int32)

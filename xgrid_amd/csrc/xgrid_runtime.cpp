@@ -618,11 +618,14 @@ int flush(xg_kernel* k) {
   }
   // a pair of interiors that the chain's one workgroup would walk in several turns is better as a
   // launch of its own (b and the first sweep of a 65^2 FP64 cavity call, 3969 cells each: chained with
-  // the walls 14.8 us, 3.3 us and 3.9 us for the walls so; the call 103 -> 96 us)
+  // the walls 14.8 us, 3.3 us and 3.9 us for the walls so; the call 103 -> 96 us), if it is the first or
+  // the last of its chain: one out of the middle leaves two chains, and three launches cost a short
+  // call more than one (three statements and a wall, 45^2 FP64 7.7 us, 12 so)
   for (size_t i = 0; i + 1 < run.size(); ++i) {
     const xg_stmt_desc& d = k->stmts[(size_t)run[i].sid].d;
     const ClassPlan& p = k->grids[(size_t)d.store_arg]->plan(d.klass);
-    if (ok[i] && ok[i + 1] && p.kind == XG_DOM_BOX && p.count > kGroupThreads && pairable(k, run[i].sid, run[i + 1].sid))
+    const bool ends = i == 0 || !ok[i - 1] || i + 2 == run.size() || !ok[i + 2];
+    if (ends && ok[i] && ok[i + 1] && p.kind == XG_DOM_BOX && p.count > kGroupThreads && pairable(k, run[i].sid, run[i + 1].sid))
       ok[i] = ok[i + 1] = 0, ++i;
   }
   thread_local std::vector<int> segs;
