@@ -17,9 +17,10 @@ constexpr int kThreads = 256;
 constexpr int kGroupThreads = 1024;
 constexpr int64_t kFuseMaxCells = 4096;  // default of g_dev.fuse_max_cells (XGRID_FUSE_MAX_CELLS)
 // A call with fewer launches runs them directly: replaying a graph takes 21 to 33 us of host time, three
-// launches 12 (45^2 to 400^2, three statements, us a call: 21 and 12), and a small cavity, which is
-// three launches and 50 us of device time, 60 against 57.5.
-constexpr int64_t kGraphMinLaunches = 4;
+// launches 12 (45^2 to 400^2, three statements, us a call: 21 and 12).  With a blocked loop among them the
+// device time hides either way, and such calls stay graphs from three launches on (9^2 to 33^2
+// cavities, all of whose calls are: 60 us a call, 57.5 made directly).
+constexpr int64_t kGraphMinLaunches = 4, kGraphMinLaunchesLoop = 3;
 // Store grids of which two levels do not fit the 256 MB last-level cache (Infinity Cache) take
 // non-temporal stores in 3-D box tiles: by the time the next update reads a cell it has left the
 // cache anyway, and the write stream drains faster.  The line lies where both ways meet (heat
@@ -126,6 +127,7 @@ struct xg_kernel {
   uint64_t tick = 0;
   int64_t n_launch = 0, n_fused = 0, n_replay = 0, n_capture = 0;
   int64_t capture_mark = 0;         // n_launch when the current capture began
+  bool capture_loop = false;        // a blocked loop is in the current capture
   std::unique_lock<std::recursive_mutex> recording;   // held (g_recording) while this kernel's call is captured
   int32_t timed_sid = -1;
   std::vector<xgi::EventPair> events;

@@ -926,6 +926,7 @@ int api_begin(xg_kernel* k, xg_grid* const* grids, int32_t ngrids, const void* k
       }
       k->mode = kCapture;
       k->capture_mark = k->n_launch;
+      k->capture_loop = false;
       k->recording = std::unique_lock<std::recursive_mutex>(g_recording);
       hipError_t err = hipStreamBeginCapture(g_dev.stream, hipStreamCaptureModeThreadLocal);
       if (err != hipSuccess) {
@@ -1042,7 +1043,7 @@ int api_end(xg_kernel* k) {
     e = hipGraphLaunch(exec, g_dev.stream);
     k->mode = kDirect;
     if (e != hipSuccess) return set_status(k, fail(XG_ERR_HIP, std::string("hipGraphLaunch: ") + hipGetErrorString(e)));
-    if (k->n_launch - k->capture_mark < kGraphMinLaunches) {
+    if (k->n_launch - k->capture_mark < (k->capture_loop ? kGraphMinLaunchesLoop : kGraphMinLaunches)) {
       // launching this graph costs more host time than launching its few kernels
       (void)hipStreamSynchronize(g_dev.stream);
       (void)hipGraphExecDestroy(exec);
@@ -1208,6 +1209,7 @@ int api_loop(xg_kernel* k, int32_t lid, int64_t trip, const void* const* params,
     return 1;
   }
   L.iterations += trip - done;
+  k->capture_loop = true;
   account();
   return 1;
 }
