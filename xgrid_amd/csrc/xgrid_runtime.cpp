@@ -607,7 +607,7 @@ int flush(xg_kernel* k) {
     k->arena.clear();
     return rc;
   }
-  // eligibility: in place, small, no hazard
+  // eligibility: in place, small, no hazard (2: of a chain that stays whole)
   thread_local std::vector<char> ok;
   ok.assign(run.size(), 0);
   for (size_t i = 0; i < run.size(); ++i) {
@@ -621,17 +621,51 @@ int flush(xg_kernel* k) {
   // the walls 14.8 us, 3.3 us and 3.9 us for the walls so; the call 103 -> 96 us), if it is the first or
   // the last of its chain: one out of the middle leaves two chains, and three launches cost a short
   // call more than one (three statements and a wall, 45^2 FP64 7.7 us, 12 so)
-  for (size_t i = 0; i + 1 < run.size(); ++i) {
-    const xg_stmt_desc& d = k->stmts[(size_t)run[i].sid].d;
-    const ClassPlan& p = k->grids[(size_t)d.store_arg]->plan(d.klass);
-    const bool ends = i == 0 || !ok[i - 1] || i + 2 == run.size() || !ok[i + 2];
-    if (ends && ok[i] && ok[i + 1] && p.kind == XG_DOM_BOX && p.count > kGroupThreads && pairable(k, run[i].sid, run[i + 1].sid))
-      ok[i] = ok[i + 1] = 0, ++i;
-  }
   thread_local std::vector<int> segs;
+  auto cells = [&](size_t t) {
+    const xg_stmt_desc& d = k->stmts[(size_t)run[t].sid].d;
+    return k->grids[(size_t)d.store_arg]->plan(d.klass).count;
+  };
+  for (size_t i = 0, j; i < run.size(); i = j) {
+    j = i + 1;
+    if (!ok[i]) continue;
+    int64_t turns = ceil_div(cells(i), kGroupThreads);
+    for (; j < run.size() && ok[j]; ++j) turns += ceil_div(cells(j), kGroupThreads);
+    if (j - i < 2) continue;
+    thread_local std::vector<char> out;   // the first of a pair that leaves the chain [i, j)
+    out.assign(j - i, 0);
+    for (size_t t = i; t + 1 < j; ++t) {
+      const xg_stmt_desc& d = k->stmts[(size_t)run[t].sid].d;
+      const ClassPlan& p = k->grids[(size_t)d.store_arg]->plan(d.klass);
+      const bool ends = t == i || (t >= i + 2 && out[t - 2 - i]) || t + 2 == j;
+      if (ends && p.kind == XG_DOM_BOX && p.count > kGroupThreads && pairable(k, run[t].sid, run[t + 1].sid))
+        out[t - i] = 1, ++t;
+    }
+    // The chain stays whole where the launches of its pairs and fans take longer: about 2.4 + 2.9 us a
+    // launch, of host time, against 3.7 + 0.6 us per turn of the chain's workgroup, and 6.8 at
+    // least (a call, us, whole and split: two fields where one reads the other, 45^2, 5 turns,
+    // 7.0 and 8.2, 64^2, 9 turns, 8.5 and 8.1; three fields 45^2, 9 turns, three launches, 8.9
+    // and 11.5, 64^2, 15 turns, 12.4 and 11.2).
+    int64_t launches = 0;
+    for (size_t t = i; t < j; ++launches) {
+      if (const size_t n = fan_run(k, run, t, segs)) {
+        t += n;
+      } else if (out[t - i]) {
+        t += 2;
+      } else {
+        do ++t;
+        while (t < j && !out[t - i]);
+      }
+    }
+    const bool whole = launches > 1 && turns < 5 * launches - 2;
+    for (size_t t = i; t < j; ++t) {
+      if (whole) ok[t] = 2;
+      else if (out[t - i]) ok[t] = ok[t + 1] = 0, ++t;
+    }
+  }
   size_t i = 0;
   while (i < run.size() && rc == XG_OK) {
-    if (const size_t n = fan_run(k, run, i, segs)) {
+    if (const size_t n = ok[i] == 2 ? 0 : fan_run(k, run, i, segs)) {
       rc = exec_fan(k, run, i, n, segs);
       i += n;
       continue;
