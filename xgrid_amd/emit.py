@@ -1678,12 +1678,17 @@ class Emitter:
         crosses into the next wave's rows; one column away, from the lane's other
         columns or, over a DPP lane shift, its neighbour's.
 
-        What bounds it: vector issue.  A cavity sweep is 8 FP64 operations per cell (4
-        cycles per wave each) and here little else: inside the box of class 0 a cell is 10
-        instructions (7 FP64 where the divisor is a power of two, one product moved out of
+        What bounds it: vector issue, and waves that have ended.  A cavity sweep is 8 FP64
+        operations per cell (4 cycles per wave each) and here little else: inside the box of
+        class 0 a cell is 10 instructions (7 FP64 where the divisor is a power of two, one product moved out of
         the iterations, and 2 lane moves), with no test, select, index or LDS read per cell; the
         LDS layout spends about 40, and its region fills the LDS where this one
-        fills registers.  50 cavity sweeps (1 launch = T iterations) with the LDS layout
+        fills registers.  Counters of one 2049^2 FP64 launch (10 iterations, 42 us, 490 workgroups of 16
+        waves, one per unit): halo cells and edge tiles included 14.2 million vector instructions,
+        23 us of every SIMD's issue; a wave issues one in 20 % of its cycles, so four of them keep a SIMD
+        0.82 busy; but a SIMD holds 2.7 waves on average, as 490 workgroups are 1.9 rounds of
+        256 and edge tiles take longer.  LDS waits are 1.5 % of wave cycles.  50 cavity
+        sweeps (1 launch = T iterations) with the LDS layout
         and with this one: 2049^2 FP64 580 -> 242 us, FP32 459 -> 189 us, 1000^2 FP64
         251 -> 135 us, 300^2 FP32 120 -> 81 us, 65^2 FP64 116 -> 81 us.
 
@@ -2427,15 +2432,17 @@ class Emitter:
 
     PREFETCH_MAX = 4   # most other-grid loads of a blocked statement kept in registers per cell
 
-    # 1024 work-items; the region (core + halo 12 on each side) takes as many rows as
-    # leave LDS for two workgroups per CU (32 waves): 72 x 64 with 8-byte cells (80.6
+    # Tiles of the LDS layout, which loops run that wave tiles do not fit (below) and whose shapes name
+    # every loop's plans.  1024 work-items; the region (core + halo 12 on each side) takes as many
+    # rows as leave LDS for two workgroups per CU (32 waves): 72 x 64 with 8-byte cells (80.6
     # KB each), 96 x 64 with 4-byte cells
     DEFAULT_BLOCK_SHAPE = (48, 64, 1024, 10, "lds")
     DEFAULT_BLOCK_SHAPE_4B = (72, 64, 1024, 10, "lds")
-    # Plain calls on smaller grids take a second tile: 1024 work-items on a 64 x 64
-    # region (two workgroups per CU in either precision), whose launches are shorter.
-    # Measured per cavity step: it wins up to 724^2 (FP32) and 1024^2 (FP64) cells and
-    # loses from 1024^2 (FP32) and 1448^2 (FP64) up.
+    # Plain calls on smaller grids take a second plan.  In the LDS layout that is a second tile: 1024
+    # work-items on a 64 x 64 region (two workgroups per CU in either precision), whose launches
+    # are shorter (cavity steps in LDS: it won up to 724^2 (FP32) and 1024^2 (FP64) cells and lost from
+    # 1024^2 (FP32) and 1448^2 (FP64) up).  On wave tiles both plans run the same kernels, cut for the
+    # grid, and differ in their proofs and counters only.
     SMALL_GRID_SHAPE = (40, 64, 1024, 10, "lds")
     SMALL_GRID_MAX_CELLS = {4: 800 * 800, 8: 1300 * 1300}
 
