@@ -41,6 +41,16 @@
 
 namespace xg {
 
+/* A compile-time value carried as a value (selects a template instantiation). */
+template <bool B>
+struct bconst {
+  static constexpr bool value = B;
+};
+template <int I>
+struct iconst {
+  static constexpr int value = I;
+};
+
 /* Workgroup tile: 256 work-items, NC cells each per chunk, CH chunks in turn.
  *   1-D: 1024 consecutive cells (work-item t: t, t+256, t+512, t+768)
  *   2-D: 4 rows x 64 columns (one cell per work-item), or x 64 times the columns that 16 bytes
@@ -330,7 +340,14 @@ struct TileCells {
     }
   }
 
-  /* The same for a 2-D tile at least CPL columns wide, a work-item's cells kept adjacent (one
+  /* Is this 2-D tile no wider than a wave: one cell per work-item, at (row(), col()), fills as many
+   * lanes as it has columns, CPL of them a CPL-th (100000 x 20, five-point, FP32 20 us a call, 25 with four;
+   * 100000 x 9 20 and 39)? */
+  __device__ __forceinline__ bool narrow() const { return thi[1] - tlo[1] <= 64; }
+  __device__ __forceinline__ int row() const { return tlo[0] + ((int)threadIdx.x >> 6); }
+  __device__ __forceinline__ int col() const { return tlo[1] + ((int)threadIdx.x & 63); }
+
+  /* The same as clamp_to_tile for a 2-D tile at least CPL columns wide, a work-item's cells kept adjacent (one
    * address, and vector loads): a lane that ends past the tile moves back as a whole, and
    * the cells it passes on the way are another lane's. */
   __device__ __forceinline__ void slide_to_tile() {
@@ -406,10 +423,18 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
      * in flight together: a cell past the tile's edge is evaluated at the
      * nearest cell inside the tile (a valid address) and not stored. */
     constexpr bool WIDE = D == 2 && S::CPL > 1;
-    const bool wide = WIDE && tc.thi[1] - tc.tlo[1] >= S::CPL;   /* the lane's cells are adjacent */
     if constexpr (WIDE) {
-      if (wide) tc.slide_to_tile();
-      else tc.clamp_to_tile();
+      if (tc.narrow()) {
+        const int i = min(tc.row(), tc.thi[0] - 1), j = min(tc.col(), tc.thi[1] - 1);
+        bool in = tc.row() < tc.thi[0] && tc.col() < tc.thi[1];
+        if (MASKED) in = in && gp<const int32_t>(H.dom.mask)[lin<D>(H.out.shape, i, j, 0)] == H.dom.klass;
+        T x;
+        if (tile_safe<S>(H, tc.tlo, tc.thi)) x = S::template value<true>(R, P, H.out.shape, i, j, 0);
+        else x = S::template value<false>(R, P, H.out.shape, i, j, 0);
+        if (in) store<S, OV>(H, i, j, 0, x);
+        continue;
+      }
+      tc.slide_to_tile();
     } else {
       tc.clamp_to_tile();
     }
@@ -422,7 +447,7 @@ __device__ __forceinline__ void box_cells(const xg_launch_hdr& H, const typename
     bool pairs = false;   /* store a lane's CPL columns with one 16-byte store */
     bool safe = tile_safe<S>(H, tc.tlo, tc.thi);
     if constexpr (D == 3 && S::ST3) safe = safe && H.out.shape[2] >= S::CPL;
-    if (safe && (!WIDE || wide)) {
+    if (safe) {
       if constexpr (D == 3 && S::ST3) {
         /* Staged 3-D tile: each array's columns of the tile's planes are read
          * once into registers; column neighbours come over DPP lane shifts and
@@ -649,17 +674,34 @@ __device__ void run_pair(const xg_launch_hdr& HA, const typename SA::Refs& RA, c
     if (tc.tlo[0] >= HA.dom.hi[0]) break;
     constexpr int NC = TC::NC;
     constexpr bool WIDE = D == 2 && SA::CPL > 1;
-    const bool wide = WIDE && tc.thi[1] - tc.tlo[1] >= SA::CPL;
+    const bool safe = tile_safe<SA>(HA, tc.tlo, tc.thi) && tile_safe<SB>(HB, tc.tlo, tc.thi);
     /* evaluate every cell without branching (see box_cells) */
     if constexpr (WIDE) {
-      if (wide) tc.slide_to_tile();
-      else tc.clamp_to_tile();
+      if (tc.narrow()) {
+        const int i = min(tc.row(), tc.thi[0] - 1), j = min(tc.col(), tc.thi[1] - 1);
+        const bool in = tc.row() < tc.thi[0] && tc.col() < tc.thi[1];
+        auto cell = [&](auto inside) {
+          constexpr bool SAFE = decltype(inside)::value;
+          const typename SA::T a = SA::template value<SAFE>(RA, PA, HA.out.shape, i, j, 0);
+          typename SB::T b;
+          if constexpr (FWD) b = SB::template value_fwd<SAFE>(RB, PB, HB.out.shape, i, j, 0, a);
+          else b = SB::template value<SAFE>(RB, PB, HB.out.shape, i, j, 0);
+          if (in) {
+            store<SA, OV>(HA, i, j, 0, a);
+            store<SB, OV>(HB, i, j, 0, b);
+          }
+        };
+        if (safe) cell(bconst<true>());
+        else cell(bconst<false>());
+        continue;
+      }
+      tc.slide_to_tile();
     } else {
       tc.clamp_to_tile();
     }
     typename SA::T va[NC];
     typename SB::T vb[NC];
-    if (tile_safe<SA>(HA, tc.tlo, tc.thi) && tile_safe<SB>(HB, tc.tlo, tc.thi) && (!WIDE || wide)) {
+    if (safe) {
       if constexpr (WIDE) {
         SA::value_row(va, RA, PA, HA.out.shape, tc.c[0][0], tc.c[0][1]);
         if constexpr (FWD) SB::value_row_fwd(vb, RB, PB, HB.out.shape, tc.c[0][0], tc.c[0][1], va);
@@ -951,16 +993,6 @@ struct Quot {
       return q;
     } else return a / b;
   }
-};
-
-/* A compile-time value carried as a value (selects a template instantiation). */
-template <bool B>
-struct bconst {
-  static constexpr bool value = B;
-};
-template <int I>
-struct iconst {
-  static constexpr int value = I;
 };
 
 /* ---- temporally blocked loops (2-D), LDS regions --------------------------
