@@ -41,7 +41,8 @@ def lower_kernel(op, block_shape: tuple | None = None, fits: dict | None = None)
 def compile_kernel(op, block_shape: tuple | None = None) -> tuple:
     """Lower a kernel and compile its device code, with blocked loops on wave tiles only where
     the code object says that they fit (Emitter.FIT_FULL): each loop whose 4-row tile spills registers is
-    built anew the next way.  A loop that fits, such as the cavity's, takes one compile.
+    built anew the next way, and so are staged 3-D statements that spill (Emitter.ST3_SCRATCH).  Where all
+    fits, as in the cavity and the heat equation, that takes one compile.
     Returns (lowered kernel, analysis, code object path)."""
     cfg = get_config()
     fits: dict = {}
@@ -50,12 +51,16 @@ def compile_kernel(op, block_shape: tuple | None = None) -> tuple:
         low, info = lower_kernel(op, block_shape, fits)
         path = compile_device(low.device_src, cfg.cacheroot, cfg.fp_contract)
         loops = [] if given else [L for L in low.loops if L.waves]
-        scratch = kernel_scratch(path) if loops else {}
+        staged = [m.stmt.sid for m in low.stmts if m.stmt.dimension == 3 and m.tile3_cols != 64]
+        scratch = kernel_scratch(path) if loops or staged else {}
         again = [L for L in loops if scratch[L.waves[-1].kernel] > 0]
-        if not again:
+        tight = [n for n in staged if ("st3", n) not in fits and scratch[f"xg_k{n}"] > Emitter.ST3_SCRATCH]
+        if not again and not tight:
             break
         for L in again:
             fits[L.lid] = fits.get(L.lid, Emitter.FIT_FULL) + 1
+        for n in tight:
+            fits["st3", n] = True
     for L in loops:
         if fits.get(L.lid) == Emitter.FIT_ROOM and scratch[L.waves[0].kernel] > Emitter.ROOM_8_ROWS_SCRATCH:
             del L.waves[0]           # (the list is the small-grid plan's too)

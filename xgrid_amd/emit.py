@@ -756,7 +756,9 @@ class Emitter:
                  entry: str = "xg_entry", macro: list | None = None, block_shape: tuple | None = None,
                  fits: dict | None = None):
         self.info = info
-        self.fits = fits or {}         # loop -> how its wave tiles are built (FIT_*; default: FIT_FULL)
+        # loop -> how its wave tiles are built (FIT_*; default: FIT_FULL); ("st3", statement): its staged
+        # tiles are built for ST3_ROOM_WAVES
+        self.fits = fits or {}
         self.shape = tuple(block_shape) if block_shape is not None else None   # None: by element size
         self.used_shape = None         # the shape the blockable loops were built with
         self.macro = list(macro or [])
@@ -1203,7 +1205,8 @@ class Emitter:
         wv = wvb = ""
         if expr_st3 is not None:
             w = max(1, min(8, 163840 // max(1, plan3.lds_bytes())))
-            wv = f" __attribute__((amdgpu_waves_per_eu({w})))"
+            asked = min(w, self.ST3_ROOM_WAVES) if ("st3", sid) in self.fits else w
+            wv = f" __attribute__((amdgpu_waves_per_eu({asked})))"
             self._st3_waves[sid] = wv
             wvb = f" __attribute__((amdgpu_waves_per_eu({max(1, w - 2)})))"
         out.append(f'extern "C" __global__ void __launch_bounds__(256){wv} xg_k{sid}({args}) '
@@ -2467,6 +2470,13 @@ class Emitter:
     # Most values, walls and all, for which FIT_ROOM keeps the 8-row tile, and the scratch bytes it may take
     # then: 2049^2 FP64 with and without it, two values 289 and 370 us, three 846 and 358.
     ROOM_8_ROWS_VALUES, ROOM_8_ROWS_SCRATCH = 2, 512
+
+    # Staged 3-D kernels whose registers spill more scratch than this at the waves that their LDS leaves room for
+    # (six: 80 registers) are built for five (96).  A body whose reads reach two cells (124 bytes of scratch
+    # FP64, 292 FP32), us, on six and five waves: 256^3 FP64 138 and 62,
+    # 250x333x301 FP64 345 and 274, 130^3 FP32 63 and 40; on four 60, 305 and 40.  Little
+    # scratch is no loss (28 bytes, 512^3 FP32: 204 us on six, 209 on five).
+    ST3_ROOM_WAVES, ST3_SCRATCH = 5, 64
 
     @classmethod
     def block_shape(cls, spec: str | None = None, elem: int = 8) -> tuple:
