@@ -363,7 +363,8 @@ struct TileCells {
 };
 
 /* Store a lane's 2-D cells, computed for adjacent columns (slide_to_tile): where all are its own
- * and the statement stores them where they are, as one vector. */
+ * and the statement stores them where they are (a two-phase statement's first phase does), as one
+ * vector. */
 template <class S, int OV, class TC>
 __device__ __forceinline__ void store_row(const xg_launch_hdr& H, const TC& tc, const typename S::T* v) {
   typedef typename S::T T;
@@ -371,11 +372,12 @@ __device__ __forceinline__ void store_row(const xg_launch_hdr& H, const TC& tc, 
   bool all = tc.in[0];
 #pragma unroll
   for (int n = 1; n < K; ++n) all = all && tc.in[n];
-  if (S::SO0 == 0 && S::SO1 == 0 && all && !(H.dom.flags & XG_F_TO_TMP)) {
+  const bool to_tmp = H.dom.flags & XG_F_TO_TMP;
+  if (((S::SO0 == 0 && S::SO1 == 0) || to_tmp) && all) {
     vecn<T, K> w;
 #pragma unroll
     for (int n = 0; n < K; ++n) w[n] = v[n];
-    put_u<T, K>(gp<T>(H.out.ptr) + lin<2>(H.out.shape, tc.c[0][0], tc.c[0][1], 0), w);
+    put_u<T, K>(gp<T>(to_tmp ? H.src.ptr : H.out.ptr) + lin<2>(H.out.shape, tc.c[0][0], tc.c[0][1], 0), w);
   } else {
 #pragma unroll
     for (int n = 0; n < K; ++n)
