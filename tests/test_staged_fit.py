@@ -3,10 +3,13 @@ import numpy as np
 import pytest
 
 import xgrid_amd as xgrid
-from xgrid_amd.backend import compile_kernel
+from xgrid_amd.backend import compile_batch, compile_kernel
+from xgrid_amd.batch import Batch
 from xgrid_amd.compilers import kernel_scratch
+from xgrid_amd.config import get_config
 
 from helpers import assert_bitexact, grid_pair, run_pair
+from oracle.cpu_path import CpuKernel
 
 f3 = xgrid.grid[float, 3]
 
@@ -38,6 +41,7 @@ def test_waves(prec, tmp_path):
         head = next(l for l in low.device_src.split("\n") if 'extern "C"' in l and " xg_k0(" in l)
         assert f"amdgpu_waves_per_eu({asked})" in head
         assert kernel_scratch(path)["xg_k0"] <= 64
+        assert kernel_scratch(compile_batch(low, get_config()))["xg_k0_b"] <= 64
 
 
 @pytest.mark.gpu
@@ -51,3 +55,25 @@ def test_reach_two(prec, shape, request):
     d, h = grid_pair(xg, shape, float, mask, rng.random(shape))
     run_pair(_far(), (d, 0.05), (h, 0.05), steps=4)
     assert_bitexact(d, h)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["double", "single"])
+def test_reach_two_batched(prec, request):
+    xg = request.getfixturevalue(prec)
+    k = _far()
+    b = Batch(k)
+    rng = np.random.default_rng(6)
+    pairs = []
+    for shape in ((9, 10, 11), (20, 18, 133), (37, 21, 260)):
+        mask = np.ones(shape, np.int32)
+        mask[2:-2, 2:-2, 2:-2] = 0
+        pairs.append(grid_pair(xg, shape, float, mask, rng.random(shape)))
+        b.add(pairs[-1][0], 0.05)
+    b.step(4)
+    ck = CpuKernel(k)
+    for d, h in pairs:
+        for _ in range(4):
+            ck(h, 0.05)
+        assert_bitexact(d, h)
+    b.close()

@@ -19,7 +19,7 @@ from . import _lib
 from .analysis import analyze
 from .compilers import compile_device, compile_host, kernel_scratch, load_host
 from .config import get_config
-from .emit import Emitter, Lowered, read_reach
+from .emit import Emitter, Lowered, ask_fewer_waves, read_reach
 from .grid import Grid
 from .types import Boolean, Floating, GridType, Integer, Pointer, Structure, Void, element_nbytes
 
@@ -51,7 +51,7 @@ def compile_kernel(op, block_shape: tuple | None = None) -> tuple:
         low, info = lower_kernel(op, block_shape, fits)
         path = compile_device(low.device_src, cfg.cacheroot, cfg.fp_contract)
         loops = [] if given else [L for L in low.loops if L.waves]
-        staged = [m.stmt.sid for m in low.stmts if m.stmt.dimension == 3 and m.tile3_cols != 64]
+        staged = staged_statements(low)
         scratch = kernel_scratch(path) if loops or staged else {}
         again = [L for L in loops if scratch[L.waves[-1].kernel] > 0]
         tight = [n for n in staged if ("st3", n) not in fits and scratch[f"xg_k{n}"] > Emitter.ST3_SCRATCH]
@@ -65,6 +65,27 @@ def compile_kernel(op, block_shape: tuple | None = None) -> tuple:
         if fits.get(L.lid) == Emitter.FIT_ROOM and scratch[L.waves[0].kernel] > Emitter.ROOM_8_ROWS_SCRATCH:
             del L.waves[0]           # (the list is the small-grid plan's too)
     return low, info, path
+
+
+def staged_statements(low: Lowered) -> list:
+    return [m.stmt.sid for m in low.stmts if m.stmt.dimension == 3 and m.tile3_cols != 64]
+
+
+def compile_batch(low: Lowered, cfg) -> str:
+    """Compile a kernel's batched variants.  Staged 3-D ones that spill (Emitter.ST3_SCRATCH) at the four waves
+    per SIMD they ask for are built for fewer, down to two: a body whose reads reach two cells, four 130^3
+    instances, us, on four / three / two waves: FP64 322 / 224 / 288 (scratch 236 / 60 / 0 bytes), FP32
+    240 / 240 / 210 (392 / 240 / 0); one of diagonal reads 198 / 92 / 89 and 165 / 129 / 80."""
+    src = low.batch_src
+    staged = staged_statements(low)
+    for waves in (4, 3, 2):
+        path = compile_device(src, cfg.cacheroot, cfg.fp_contract)
+        scratch = kernel_scratch(path) if staged else {}
+        tight = [n for n in staged if scratch[f"xg_k{n}_b"] > Emitter.ST3_SCRATCH]
+        if not tight or waves == 2:
+            return path
+        for n in tight:
+            src = ask_fewer_waves(src, f"xg_k{n}_b")
 
 
 def _ctype_of(t):
@@ -256,7 +277,7 @@ class HipKernel:
         if self.module_b is not None:
             return
         cfg = self.cfg
-        path = compile_device(self.lowered.batch_src, cfg.cacheroot, cfg.fp_contract)
+        path = compile_batch(self.lowered, cfg)
         mod = c_void_p()
         _lib.check(self.lib.xg_module_load(path.encode(), ctypes.byref(mod)), "xg_module_load")
         self.module_b = mod.value

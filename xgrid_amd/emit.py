@@ -171,6 +171,12 @@ class LoopMeta:
         return f"xg_tb{self.lid}_chk"
 
 
+def ask_fewer_waves(src: str, kernel: str) -> str:
+    """The source with `kernel`'s launch attribute asking for one wave per SIMD less."""
+    return re.sub(r"amdgpu_waves_per_eu\((\d+)\)(\)+ " + kernel + r"\()",
+                  lambda m: f"amdgpu_waves_per_eu({max(1, int(m[1]) - 1)}){m[2]}", src)
+
+
 @dataclass
 class Lowered:
     device_src: str               # the kernels plain calls launch
